@@ -83,7 +83,7 @@ def build_oracle(with_ref: bool = True) -> None:
     compiled reference driver (test infrastructure, never shipped)."""
     odir = os.path.join(ROOT, "oracle")
     subprocess.run(["make", "-s", "-C", odir], check=True)
-    if with_ref and os.path.isdir("/root/reference"):
+    if with_ref and os.path.isfile("/root/reference/mgsolver.for"):
         subprocess.run(["make", "-s", "-C", odir, "ref"], check=True)
 
 
