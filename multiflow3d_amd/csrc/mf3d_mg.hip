@@ -133,6 +133,8 @@ struct mf3d_mg {
     // coarse tail: levels lt..L-1 run in LDS, one workgroup per block
     int lt = 0;
     BlockLevel *d_tail = nullptr;
+    TLv *d_tlv = nullptr;          // its levels (as d_tail) and their cell and ghost lists
+    unsigned *d_ttab = nullptr;
     size_t tail_lds = 0;
     // outer step tiles (finest level)
     Tile *t_out = nullptr;
@@ -900,7 +902,7 @@ void tail(mf3d_mg *mg, bool from_zero, const int *done) {
         co.cz[l - lt] = (const T *)mg->lv[l].cz;
     }
     hipLaunchKernelGGL((k_tail<T, VAR>), dim3(mg->cfg.nblocks), dim3(TAIL_NT), mg->tail_lds, mg->stream, mg->d_tail,
-                       mg->cfg.nblocks, L - lt, (const T *)V.rhs, from_zero ? nullptr : (const T *)V.phi[V.cur],
+                       (const TLv *)mg->d_tlv, (const unsigned *)mg->d_ttab, mg->cfg.nblocks, L - lt, (const T *)V.rhs, from_zero ? nullptr : (const T *)V.phi[V.cur],
                        (T *)V.phi[1 - V.cur], co, mg->cfg.nu_pre, mg->cfg.nu_post,
                        mg->cdirect ? (const double *)mg->d_cinv : nullptr, mg->nc,
                        TailC64<T>{mg->c64 ? 1 : 0, mg->lv[L - 1].dcx, mg->lv[L - 1].dcy, mg->lv[L - 1].dcz}, done);
@@ -1296,9 +1298,27 @@ int choose_tail(mf3d_mg *mg) {
         return MF3D_EDEVICE;
     }
     std::vector<BlockLevel> tl;
+    std::vector<TLv> lv;
+    std::vector<unsigned> tab;
+    std::vector<int> off(nb, 0);  // LDS entries: every level's potential, then every level's RHS
     for (int l = mg->lt; l < L; ++l)
-        for (int b = 0; b < nb; ++b) tl.push_back(mg->lv[l].hb[b]);
-    return upload(mg, &mg->d_tail, tl);
+        for (int b = 0; b < nb; ++b) {
+            const BlockLevel &g = mg->lv[l].hb[b];
+            tl.push_back(g);
+            TLv v = tlv_of(g.n0, g.n1, g.n2, g.neu);
+            v.po = off[b];
+            off[b] += v.sz * (v.n2 + 2);
+            tail_tables(v, tab);
+            lv.push_back(v);
+        }
+    for (int l = mg->lt, q = 0; l < L; ++l)
+        for (int b = 0; b < nb; ++b, ++q) {
+            lv[q].ro = off[b];
+            off[b] += lv[q].sz * (lv[q].n2 + 2);
+        }
+    int rc;
+    if ((rc = upload(mg, &mg->d_tail, tl)) || (rc = upload(mg, &mg->d_tlv, lv))) return rc;
+    return upload(mg, &mg->d_ttab, tab);
 }
 
 template <typename T, bool VAR>
