@@ -70,6 +70,10 @@ struct Level {
     bool adi_rhs = false;
     int adi_cells = 0, adi_sstride = 0;
     void *adi_apr[3] = {}, *adi_a[3] = {};  // the LDS kernel's Thomas coefficients per line axis
+    // constant coefficients and extents of at most ADC_LINE: k_adi_cls with
+    // this many cells a thread (0: not), its dynamic LDS and class tables
+    int adi_k = 0;
+    void *adi_tab = nullptr;
     int sw_ty = 4;  // sweep tile rows of the march; 0: 3-D tiles (k_rb3d)
     // the zero-start march (k_rbz) on its own chunks: the default depth
     // (the deepest that still gives ~1024 workgroups), which suits its
@@ -766,6 +770,16 @@ void sweep_inplace(mf3d_mg *mg, Level &L, const int *done) {
         return;
     }
     const unsigned nt = adi_threads(L);
+    if (L.adi_k) {
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(nb), dim3(ADC_NT), L.adi_lds, mg->stream, p, rhs, (const T *)L.adi_tab,
+                               L.adi_sstride, L.db, done);
+        };
+        if (L.adi_k == 1) go(k_adi_cls<T, 1>);
+        else if (L.adi_k == 2) go(k_adi_cls<T, 2>);
+        else go(k_adi_cls<T, 5>);
+        return;
+    }
     if (L.adi_lds) {  // a 256-thread workgroup per block
         const AdiCoef<T> ac{{(const T *)L.adi_apr[0], (const T *)L.adi_apr[1], (const T *)L.adi_apr[2]},
                             {(const T *)L.adi_a[0], (const T *)L.adi_a[1], (const T *)L.adi_a[2]}};
@@ -1574,8 +1588,11 @@ int coarse_factor(mf3d_mg *mg) {
     return 0;
 }
 
-// ADI smoother set-up: per level, the whole-sweep LDS kernel where the
-// level's largest block (its ghosted potential and the per-diagonal
+// ADI smoother set-up: per level, with constant coefficients the class-table
+// kernel (k_adi_cls: the shipped deck's sweep 413 -> 173 us in FP64) where
+// every extent is at most ADC_LINE (its lines live in registers) and the
+// largest block's ghosted potential and the tables fit in kAdiLdsMax bytes;
+// else the whole-sweep LDS kernel where the level's largest block (its ghosted potential and the per-diagonal
 // scratch, with the RHS if that fits too) fits in kAdiLdsMax bytes.
 constexpr size_t kAdiLdsMax = 150 * 1024;
 
@@ -1586,17 +1603,28 @@ int adi_setup(mf3d_mg *mg) {
     size_t most = 0;
     for (Level &V : mg->lv) {
         size_t cells = 0, diag = 1;  // the largest ghosted box; the most cells one diagonal holds
+        int line = 0, plane = 0, tt = 0;  // k_adi_cls: the longest line, the largest plane of lane axis x line,
+                                          // the entries of a pass's lines
         for (const BlockLevel &g : V.hb) {
             cells = std::max(cells, (size_t)(g.sz * (g.n2 + 2)));
             const size_t n0 = g.n0, n1 = g.n1, n2 = g.n2;
             diag = std::max({diag, std::min(n0, n2) * n1, std::min(n1, n2) * n0, std::min(n0, n1) * n2});
+            line = std::max({line, g.n0, g.n1, g.n2});
+            plane = std::max({plane, g.n2 * g.n1, g.n1 * g.n0});
+            tt = std::max({tt, g.n2 * adc_stride(g.n1), g.n1 * adc_stride(g.n0), g.n1 * adc_stride(g.n2)});
         }
         V.adi_cells = (int)cells;
         V.adi_sstride = (int)diag;
         V.adi_lds = 0;
         V.adi_rhs = false;
+        const size_t cls_lds = (cells + 2 * (size_t)tt + 2 * ADC_CLS * ADC_LINE) * w;
         const bool fits = allow && diag <= 1024;  // the next diagonal's prefetch: 4 entries per thread
-        if (fits && (2 * cells + 5 * diag) * w <= kAdiLdsMax) {
+        V.adi_k = 0;
+        if (allow && !mg->cfg.variable_coef && line <= ADC_LINE && cls_lds <= kAdiLdsMax) {
+            V.adi_k = plane <= ADC_NT ? 1 : (plane <= 2 * ADC_NT ? 2 : 5);  // ADC_LINE^2 <= 5 * ADC_NT
+            V.adi_lds = cls_lds;
+            V.adi_sstride = tt;
+        } else if (fits && (2 * cells + 5 * diag) * w <= kAdiLdsMax) {
             V.adi_lds = (2 * cells + 5 * diag) * w;
             V.adi_rhs = true;
         } else if (fits && (cells + 5 * diag) * w <= kAdiLdsMax) {
@@ -1607,7 +1635,10 @@ int adi_setup(mf3d_mg *mg) {
     if (most > 64 * 1024) {
         const hipFuncAttribute attr = hipFuncAttributeMaxDynamicSharedMemorySize;
         const int bytes = (int)most;
-        const void *fns[8] = {(const void *)k_adi_lds<double, false, false>, (const void *)k_adi_lds<double, false, true>,
+        const void *fns[14] = {(const void *)k_adi_cls<double, 1>, (const void *)k_adi_cls<double, 2>,
+                              (const void *)k_adi_cls<double, 5>, (const void *)k_adi_cls<float, 1>,
+                              (const void *)k_adi_cls<float, 2>, (const void *)k_adi_cls<float, 5>,
+                              (const void *)k_adi_lds<double, false, false>, (const void *)k_adi_lds<double, false, true>,
                               (const void *)k_adi_lds<double, true, false>,  (const void *)k_adi_lds<double, true, true>,
                               (const void *)k_adi_lds<float, false, false>,  (const void *)k_adi_lds<float, false, true>,
                               (const void *)k_adi_lds<float, true, false>,   (const void *)k_adi_lds<float, true, true>};
@@ -1626,6 +1657,11 @@ template <typename T, bool VAR>
 int adi_coef_build(mf3d_mg *mg) {
     for (Level &V : mg->lv) {
         if (!V.adi_lds) continue;
+        if (V.adi_k) {
+            hipLaunchKernelGGL(k_adi_classes<T>, dim3((unsigned)mg->cfg.nblocks), dim3(64), 0, mg->stream,
+                               (T *)V.adi_tab, V.db);
+            continue;
+        }
         int most = 1;
         for (const BlockLevel &g : V.hb) most = std::max({most, g.n0 * g.n2, g.n1 * g.n2, g.n0 * g.n1});
         const dim3 grid((unsigned)((most + 255) / 256), (unsigned)mg->cfg.nblocks);
@@ -1853,7 +1889,9 @@ int build(mf3d_mg *mg) {
         bool global = false;  // a level runs the per-pass kernels: their a(m) scratch
         for (Level &V : mg->lv) {
             global = global || !V.adi_lds;
-            if (V.adi_lds)
+            if (V.adi_k) {
+                if ((rc = dev_alloc(mg, &V.adi_tab, (size_t)nb * 6 * ADC_CLS * ADC_LINE * w))) return rc;
+            } else if (V.adi_lds)
                 for (int a = 0; a < 3; ++a)
                     if ((rc = dev_alloc(mg, &V.adi_apr[a], V.cells_gh * w)) ||
                         (rc = dev_alloc(mg, &V.adi_a[a], V.cells_gh * w)))

@@ -420,4 +420,262 @@ __global__ __launch_bounds__(256) void k_adi_lds(T *__restrict__ p, const T *__r
     for (int c = (int)threadIdx.x; c < cells; c += (int)blockDim.x) p[g.off + c] = P[c];
 }
 
+// ---------------------------------------------------------------------------
+// Constant coefficients: the same sweep with little but the recurrences left
+// between two diagonals.
+//
+// What bounds it: the chain of line recurrences, 3 dependent operations a
+// cell forward and 2 back on one lane a line (22 and 15 clocks in FP64),
+// diagonal after diagonal, and the LDS accesses of the one wave that runs
+// it: a wave issues one about every 10 to 20 clocks, however few lanes it
+// has.  HBM, LDS bandwidth and the other waves are idle beside it.  So
+//   - the lines of a diagonal pass through LDS with a line's cells side by
+//     side, two (FP64) or four (FP32) a 16-byte access, and c(m) stays in
+//     registers: 2 accesses for 2 cells and direction where k_adi_lds has 6;
+//   - the Thomas sequences depend on the line only through the walls it
+//     touches: at most 16 classes a pass (low / high end of each cross axis),
+//     a table in LDS (k_adi_classes builds it once), not a stream per cell;
+//   - every thread keeps its cells' (lane coordinate, place on the line) for
+//     the whole pass and moves to the next diagonal by adding one stride; it
+//     stores the finished diagonal's phi and forms the next one's cross terms
+//     in one phase;
+//   - the loop over the diagonals stays rolled, so that its code fits in the
+//     instruction cache.
+// The reference's 80 blocks of 40 x 10 x 25: 413 -> 173 us a sweep in FP64,
+// 370 -> 147 us in FP32.
+//
+// Lanes run along k in the j pass (whose lines are the shortest) and along j
+// in the others; diagonals and every operand are those of the sweep above.
+constexpr int ADC_NT = 512, ADC_LINE = 48, ADC_CLS = 16;
+static_assert(3 * ADC_CLS <= 64 && ADC_LINE * ADC_LINE <= 5 * ADC_NT, "a wave builds a block's classes; 5 cells a thread reach");
+
+// Entries between two lines of a diagonal in LDS: whole groups of 8 cells, as
+// adc_line reads them, and 4 more to spread the banks.
+__host__ __device__ inline int adc_stride(int nm) { return (nm + 7) / 8 * 8 + 4; }
+
+// apr(m) and a(m) of every class of lines: tab[block][axis][apr, a][class][m],
+// ADC_LINE entries a line.  Class bits: 1 low / 2 high end of the lane axis, 4
+// low / 8 high end of the other (adc_axes).  One thread a class and axis.
+template <typename T>
+__global__ __launch_bounds__(64) void k_adi_classes(T *__restrict__ tab, const BlockLevel *__restrict__ bls) {
+    const BlockLevel g = bls[blockIdx.x];
+    const int ax = (int)threadIdx.x / ADC_CLS, cls = (int)threadIdx.x % ADC_CLS;
+    if (ax >= 3) return;
+    const int n[3] = {g.n0, g.n1, g.n2};
+    const int ua = ax == 1 ? 2 : 1, va = ax == 2 ? 0 : (ax == 1 ? 0 : 2);  // lane axis, other axis
+    T lo[3], hi[3];  // the coefficient below and above along each axis
+    for (int d = 0; d < 3; ++d) lo[d] = hi[d] = cconst<T>(g, d);
+    if ((cls & 1) && (g.neu & (1 << (2 * ua)))) lo[ua] = T(0);
+    if ((cls & 2) && (g.neu & (2 << (2 * ua)))) hi[ua] = T(0);
+    if ((cls & 4) && (g.neu & (1 << (2 * va)))) lo[va] = T(0);
+    if ((cls & 8) && (g.neu & (2 << (2 * va)))) hi[va] = T(0);
+    T *apr_out = tab + ((long long)blockIdx.x * 3 + ax) * 2 * ADC_CLS * ADC_LINE + cls * ADC_LINE;
+    T *a_out = apr_out + ADC_CLS * ADC_LINE;
+    T a_prev = T(0);
+    for (int m = 1; m <= n[ax]; ++m) {
+        T l[3] = {lo[0], lo[1], lo[2]}, h[3] = {hi[0], hi[1], hi[2]};
+        if (m == 1 && (g.neu & (1 << (2 * ax)))) l[ax] = T(0);
+        if (m == n[ax] && (g.neu & (2 << (2 * ax)))) h[ax] = T(0);
+        T s = l[0] + h[0];
+        s = s + l[1];
+        s = s + h[1];
+        s = s + l[2];
+        s = s + h[2];
+        const T ap = -s;
+        const T apr = T(1) / (ap - l[ax] * a_prev);
+        a_prev = h[ax] * apr;
+        apr_out[m - 1] = apr;
+        a_out[m - 1] = a_prev;
+    }
+}
+
+// One line's recurrences on one lane, at most 8 * NCH cells: t(m) from tl, apr
+// and a from ta and tb, phi(m) to tl (each 16-byte aligned, 8 * NCH entries;
+// past the line's end they are read and written but feed nothing).  cur, nxt:
+// the ghosts before and after the line; lo1, lo: the coefficient towards the
+// previous cell of the first cell and of the others.
+template <typename T, int NCH>
+__device__ __forceinline__ void adc_line(T *tl, int nm, const T *ta, const T *tb, T cur, T nxt, T lo1, T lo) {
+    constexpr int V = 16 / (int)sizeof(T), N = 8 * NCH, G = 4;  // G cells' operands are read together
+    constexpr int NG = N / G;                                    // the last group may lie past the end: left out
+    using TV = T __attribute__((ext_vector_type(16 / sizeof(T))));
+    const TV *t4 = reinterpret_cast<const TV *>(tl), *p4 = reinterpret_cast<const TV *>(ta),
+             *a4 = reinterpret_cast<const TV *>(tb);
+    T c[N];
+    TV t[3][G / V], x[3][G / V];
+    auto ld = [&](const TV *q, int g, TV *r) {
+#pragma unroll
+        for (int e = 0; e < G / V; ++e) r[e] = q[g * (G / V) + e];
+    };
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        ld(t4, g, t[g]);
+        ld(p4, g, x[g]);
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (g + 2 < NG) {
+            ld(t4, g + 2, t[(g + 2) % 3]);
+            ld(p4, g + 2, x[(g + 2) % 3]);
+        }
+        if (g == NG - 1 && g * G >= nm) continue;
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+            cur = (t[g % 3][e / V][e % V] - (g == 0 && e == 0 ? lo1 : lo) * cur) * x[g % 3][e / V][e % V];
+            c[g * G + e] = cur;
+        }
+    }
+    ld(a4, NG - 1, x[(NG - 1) % 3]);
+    ld(a4, NG - 2, x[(NG - 2) % 3]);
+#pragma unroll
+    for (int g = NG - 1; g >= 0; --g) {
+        if (g > 1) ld(a4, g - 2, x[(g - 2) % 3]);
+        if (g == NG - 1 && g * G >= nm) continue;
+        TV o[G / V];
+#pragma unroll
+        for (int e = G - 1; e >= 0; --e) {
+            const T f = c[g * G + e] - x[g % 3][e / V][e % V] * nxt;
+            nxt = g < NG - 2 || g * G + e < nm ? f : nxt;  // only cells of the last two groups may lie past the end
+            o[e / V][e % V] = nxt;
+        }
+#pragma unroll
+        for (int e = 0; e < G / V; ++e) reinterpret_cast<TV *>(tl)[g * (G / V) + e] = o[e];
+    }
+}
+
+// One pass (lines along AX) of a block in LDS, K cells a thread.  L: the
+// dynamic LDS; at tt the lines of the current diagonal and those of the one
+// before, ttn entries each and in turn, S entries a line, lane coordinate u =
+// 1 .. at u - 1: t before the recurrences, phi after them; at po the block.
+template <typename T, int AX, int K>
+__device__ __forceinline__ void adc_pass(const BlockLevel &g, T *L, int tt, int ttn, int po,
+                                         const T *__restrict__ rhs, const T *__restrict__ tab) {
+    constexpr int NT = ADC_NT;
+    const int sy = (int)g.sy, sz = (int)g.sz, tid = (int)threadIdx.x;
+    const int nm = AX == 0 ? g.n0 : (AX == 1 ? g.n1 : g.n2), st = AX == 0 ? 1 : (AX == 1 ? sy : sz);
+    // the cross terms' first and second axis, in the reference's order
+    // (j pass: E, W, T, B; i pass: N, S, T, B; k pass: N, S, E, W)
+    const int np = AX == 1 ? g.n0 : g.n1, nq = AX == 2 ? g.n0 : g.n2;
+    const int sp = AX == 1 ? 1 : sy, sq = AX == 2 ? 1 : sz;
+    const T cp = cconst<T>(g, AX == 1 ? 0 : 1), cq = cconst<T>(g, AX == 2 ? 0 : 2);
+    const bool plo = g.neu & (AX == 1 ? kNeuW : kNeuS), phi = g.neu & (AX == 1 ? kNeuE : kNeuN);
+    const bool qlo = g.neu & (AX == 2 ? kNeuW : kNeuB), qhi = g.neu & (AX == 2 ? kNeuE : kNeuT);
+    // lanes along u, the other cross axis v = d - u
+    constexpr bool SEC = AX == 1;
+    const int nu = SEC ? nq : np, nv = SEC ? np : nq, su = SEC ? sq : sp, sv = SEC ? sp : sq, dmax = nu + nv;
+    const int S = adc_stride(nm);
+    T *TA = L, *TB = L + ADC_CLS * ADC_LINE;
+    for (int e = tid; e < ADC_CLS * ADC_LINE; e += NT) {
+        TA[e] = tab[e];
+        TB[e] = tab[ADC_CLS * ADC_LINE + e];
+    }
+    int uu[K], base[K], tix[K];
+    T ulo[K], uhi[K];  // the coefficients below and above along the lane axis
+    const T cu = SEC ? cq : cp, cv = SEC ? cp : cq;
+    const bool uwl = SEC ? qlo : plo, uwh = SEC ? qhi : phi, vwl = SEC ? plo : qlo, vwh = SEC ? phi : qhi;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int c = tid + k * NT, m = c / nu, u = c - m * nu + 1;
+        uu[k] = c < nu * nm ? u : 1 << 20;  // no cell: never on a diagonal
+        base[k] = po + u * (su - sv) + (m + 1) * st;
+        tix[k] = tt + (u - 1) * S + m;
+        ulo[k] = uwl && u == 1 ? T(0) : cu;
+        uhi[k] = uwh && u == nu ? T(0) : cu;
+    }
+    T r[K];
+    auto load = [&](int d) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int v = d - uu[k];
+            r[k] = v >= 1 && v <= nv ? rhs[base[k] - po + d * sv] : T(0);
+        }
+    };
+    load(2);
+    const int lane = tid & 63;
+    const T lo = cconst<T>(g, AX), lo1 = (g.neu & (1 << (2 * AX))) ? T(0) : lo;
+    __syncthreads();  // the class table, and the pass before
+#pragma unroll 1
+    for (int d = 2; d <= dmax + 1; ++d) {
+        // phi of diagonal d - 1 into the block, the cross terms of diagonal d.
+        // All four reads are made together, at entry 0 where there is none.
+        const int now = d & 1 ? ttn : 0, then = ttn - now;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int u = uu[k], v = d - u, at = base[k] + d * sv;
+            const bool on = v >= 1 && v <= nv, was = v >= 2 && v <= nv + 1;
+            const T before = L[was ? tix[k] + then : (on ? at - sv : 0)];  // (u, v-1): just solved, or the ghost
+            const T below = L[on ? (u == 1 ? at - su : tix[k] + then - S) : 0];  // (u-1, v)
+            const T above = L[on ? at + su : 0], next = L[on ? at + sv : 0];
+            const T vlo = vwl && v == 1 ? T(0) : cv, vhi = vwh && v == nv ? T(0) : cv;
+            T s;
+            if (SEC) {
+                s = r[k] - vhi * next;
+                s = s - vlo * before;
+                s = s - uhi[k] * above;
+                s = s - ulo[k] * below;
+            } else {
+                s = r[k] - uhi[k] * above;
+                s = s - ulo[k] * below;
+                s = s - vhi * next;
+                s = s - vlo * before;
+            }
+            if (on) L[tix[k] + now] = s;
+            if (was) L[at - sv] = before;
+        }
+        if (d > dmax) break;  // uniform: the last diagonal is stored
+        load(d + 1);
+        const int u = lane + 1, v = d - u;
+        const bool solve = tid < 64 && u <= nu && v >= 1 && v <= nv;
+        const int q0 = po + (solve ? u * su + v * sv : 0);
+        const T g0 = L[q0], g1 = L[q0 + st * (nm + 1)];  // the line's ghosts, which no pass changes
+        __syncthreads();
+        if (solve) {
+            const int cls = (u == 1 ? 1 : 0) | (u == nu ? 2 : 0) | (v == 1 ? 4 : 0) | (v == nv ? 8 : 0);
+            const T *ta = TA + cls * ADC_LINE, *tb = TB + cls * ADC_LINE;
+            T *tl = L + tt + now + lane * S;
+            switch ((nm + 7) / 8) {
+                case 1: adc_line<T, 1>(tl, nm, ta, tb, g0, g1, lo1, lo); break;
+                case 2: adc_line<T, 2>(tl, nm, ta, tb, g0, g1, lo1, lo); break;
+                case 3: adc_line<T, 3>(tl, nm, ta, tb, g0, g1, lo1, lo); break;
+                case 4: adc_line<T, 4>(tl, nm, ta, tb, g0, g1, lo1, lo); break;
+                case 5: adc_line<T, 5>(tl, nm, ta, tb, g0, g1, lo1, lo); break;
+                default: adc_line<T, 6>(tl, nm, ta, tb, g0, g1, lo1, lo); break;
+            }
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+}
+
+// A whole ADI sweep (j, i, then k lines) of one block per workgroup, constant
+// coefficients, every extent at most ADC_LINE and K * ADC_NT cells at most on
+// each plane of lane axis x line.  Dynamic LDS: the class tables (2 * ADC_CLS *
+// ADC_LINE entries), two diagonals' lines (tt entries each), the block's ghosted potential.
+template <typename T, int K>
+__global__ __launch_bounds__(ADC_NT) void k_adi_cls(T *__restrict__ p, const T *__restrict__ rhs,
+                                                    const T *__restrict__ tab, int tt,
+                                                    const BlockLevel *__restrict__ bls,
+                                                    const int *__restrict__ done) {
+    if (done && *done) return;
+    extern __shared__ __align__(16) unsigned char adc_smem[];
+    constexpr int t0 = 2 * ADC_CLS * ADC_LINE;
+    T *L = reinterpret_cast<T *>(adc_smem), *P = L + t0 + 2 * tt;
+    const BlockLevel g = bls[blockIdx.x];
+    const int cells = (int)(g.sz * (g.n2 + 2));
+    T *pg = p + g.off;
+    constexpr int U = 8;
+    for (int c0 = (int)threadIdx.x; c0 < cells; c0 += U * ADC_NT) {
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = pg[min(c0 + u * ADC_NT, cells - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) P[min(c0 + u * ADC_NT, cells - 1)] = v[u];
+    }
+    const T *tb = tab + (long long)blockIdx.x * 3 * 2 * ADC_CLS * ADC_LINE;
+    adc_pass<T, 1, K>(g, L, t0, tt, t0 + 2 * tt, rhs + g.off, tb + 2 * ADC_CLS * ADC_LINE);
+    adc_pass<T, 0, K>(g, L, t0, tt, t0 + 2 * tt, rhs + g.off, tb);
+    adc_pass<T, 2, K>(g, L, t0, tt, t0 + 2 * tt, rhs + g.off, tb + 4 * ADC_CLS * ADC_LINE);
+    for (int c = (int)threadIdx.x; c < cells; c += ADC_NT) pg[c] = P[c];
+}
+
 }  // namespace mf3d
