@@ -50,7 +50,16 @@ def sweep_bytes_per_launch(w, c=0):
     return (3 * (3 + c) + (2 + c)) / 4.0 * w
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_rbs_256cubed_L7_traffic.md")
+def leg_bytes_per_launch(w):
+    """Finest-level launches of a lone block's V(2,2) cycle with constant
+    coefficients: the down leg (two sweeps from zero and the restricted
+    residual: RHS read, potential and coarse RHS written) and the up leg
+    (prolongation and two sweeps: RHS, potential and coarse potential read,
+    potential written), 21/8 w per cell on average."""
+    return (2.125 + 3.125) / 2.0 * w
+
+
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_leg_256cubed_L7_traffic.md")
 VEL_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_velmas_256cubed_L7.md")
 
 
@@ -69,8 +78,8 @@ def cpu_model():
 def measured_traffic(form, path=TRAFFIC_FILE, key="traffic_bytes_per_launch:"):
     """HBM bytes per launch of the 256^3, 7-level workload from a committed
     rocprofv3 PMC summary: FETCH_SIZE x 2 + WRITE_SIZE, the factors fixed by
-    a 1 GiB copy in the same runs.  For k_rbs (default) the finest-level
-    launch mix (3 full sweeps + 1 zero-start sweep); for k_velmas the key
+    a 1 GiB copy in the same runs.  For k_leg (default) the finest-level
+    launch mix (a down and an up leg); for k_velmas the key
     velocity_traffic_bytes_per_launch of its summary.  None when absent."""
     try:
         with open(path) as fh:
@@ -151,18 +160,20 @@ def rel_l2_mean_removed(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
-def sweep_roofline(r, w, n0, c=0, traffic=None, traffic_source=None, kernel="k_rbs"):
-    """Roofline of the finest-level sweep from the hook's launch times:
-    sweep_bytes_per_launch(w, c) x n0 interior cells per launch."""
+def sweep_roofline(r, w, n0, c=0, traffic=None, traffic_source=None, legs=False):
+    """Roofline of the finest-level sweep (legs: of the cycle's two legs) from
+    the hook's launch times: sweep_bytes_per_launch(w, c) or
+    leg_bytes_per_launch(w) x n0 interior cells per launch."""
     if not r["launches"]:
         return None
     avg_s = r["kernel_ms"] / r["launches"] * 1e-3
-    per_launch = sweep_bytes_per_launch(w, c) * n0
+    per_launch = (leg_bytes_per_launch(w) if legs else sweep_bytes_per_launch(w, c)) * n0
     achieved = per_launch / avg_s / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBPS, 4),
             "traffic": traffic, "traffic_source": traffic_source if traffic else None,
-            "kernel": f"{kernel} (fused red-black sweep, finest level)", "avg_us": round(avg_s * 1e6, 2),
+            "kernel": "k_leg (one leg of the V-cycle, two red-black sweeps and the transfer, finest level)"
+            if legs else "k_rbs (fused red-black sweep, finest level)", "avg_us": round(avg_s * 1e6, 2),
             "launches_timed": r["launches"], "bytes_per_launch": int(per_launch),
             "timed_with": "HIP events on the solver's stream around each launch, inside the timed "
                           "region (graph replay)" if r["hook_replay"] else
@@ -539,15 +550,17 @@ def main():
         print(f"# calibration copy: {nbytes} bytes read, {nbytes} bytes written", file=sys.stderr, flush=True)
         del a, b
 
-    # Dominant kernel: k_rbs, one fused red-black sweep (both colours) of the
-    # finest level; sweep_bytes_per_launch gives its algorithmic bytes.
+    # Dominant kernel: k_leg, one leg of the V-cycle on the finest level;
+    # leg_bytes_per_launch gives its algorithmic bytes.  MF3D_LEGS=0 runs sweeps
+    # apart (k_rbs).
+    legs = os.environ.get("MF3D_LEGS", "1") != "0"
     N0 = levels_cells[0]
-    src = ("profiles/k_rbs_256cubed_L7_traffic.md (rocprofv3 FETCH_SIZE x2 + WRITE_SIZE per launch, "
+    src = ("profiles/k_leg_256cubed_L7_traffic.md (rocprofv3 FETCH_SIZE x2 + WRITE_SIZE per launch, "
            "calibrated on a 1 GiB copy)")
 
     def roofline(r, w):
-        traffic = measured_traffic("fp64" if w == 8 else "mixed") if (n, L) == (256, 7) else None
-        return sweep_roofline(r, w, N0, 0, traffic, src)
+        traffic = measured_traffic("fp64" if w == 8 else "mixed") if legs and (n, L) == (256, 7) else None
+        return sweep_roofline(r, w, N0, 0, traffic, src, legs)
 
     cpu = None
     if not args.no_cpu_baseline:

@@ -35,6 +35,7 @@
 #include "mg_coarse.hpp"
 #include "mg_common.hpp"
 #include "mg_ghostmap.hpp"
+#include "mg_leg.hpp"
 #include "mg_refine.hpp"
 #include "mg_outer.hpp"
 #include "mg_setup.hpp"
@@ -82,6 +83,10 @@ struct Level {
     // its steps heavier) the full sweep's tuned tiles
     Tile *t_swz = nullptr;
     int n_swz = 0, swz_ty = 4;
+    // the level's legs as one launch each (k_leg): tiles, and which legs
+    Tile *t_leg = nullptr;
+    int n_leg = 0, leg_ny = 0;
+    bool leg_down = false, leg_up = false;
     Region *r_full = nullptr;
     int n_full = 0, max_full = 0;
     // refined block grids: the level's ghosts as expressions (no regions)
@@ -218,6 +223,9 @@ struct mf3d_mg {
     // levels on 3-D tiles fuse the prolongation into their first post-sweep
     // (k_rb3d<..., PRO>); MF3D_FUSE_PROLONG=0 keeps them apart, bitwise the same
     bool fuse_pro = true;
+    // a lone block's levels run each leg of the cycle in one launch (k_leg);
+    // MF3D_LEGS=0 keeps sweeps, restriction and prolongation apart, bitwise the same
+    bool legs = true;
     // the velocity form's fields on the caller's ghost shell: G layers
     // (every block's `ghost`), per-block shell geometry, total length
     int G = 1;
@@ -948,6 +956,28 @@ void prolong_sweep(mf3d_mg *mg, int l, const int *done) {
     gather<T>(mg, l, done);
 }
 
+// The down leg of level l (two sweeps from zero, the residual into level l+1's
+// RHS) or its up leg (prolongation from level l+1, two sweeps).
+template <typename T>
+void leg(mf3d_mg *mg, int l, bool up, const int *done) {
+    Level &F = mg->lv[l], &C = mg->lv[l + 1];
+    const bool tk = tk_on(mg, MF3D_K_SMOOTH, l);
+    const bool yper = !(F.hb[0].neu & (kNeuS | kNeuN));
+    const uint32_t bytes = (uint32_t)(F.cells_gh * (long long)sizeof(T));
+    const uint32_t cbytes = (uint32_t)(C.cells_gh * (long long)sizeof(T));
+    if (tk) tk_mark(mg);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(F.n_leg), dim3(32 * F.leg_ny), leg_lds<T>(up, yper, F.leg_ny), mg->stream, (const T *)F.phi[F.cur],
+                           (T *)F.phi[1 - F.cur], (const T *)F.rhs, bytes, F.db, F.t_leg, done,
+                           (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db);
+    };
+    constexpr int NY = leg_ny<T>();
+    if (F.leg_ny == NY) up ? go(k_leg<T, true, NY>) : go(k_leg<T, false, NY>);
+    else up ? go(k_leg<T, true, LEG_NY_SMALL>) : go(k_leg<T, false, LEG_NY_SMALL>);
+    if (tk) tk_mark(mg);
+    F.cur = 1 - F.cur;
+}
+
 template <typename T, bool VAR>
 void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
     const int L = mg->cfg.levels, lt = mg->lt;
@@ -955,25 +985,40 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
         tail<T, VAR>(mg, zero_start, done);
         return;
     }
-    relax<T, VAR>(mg, 0, mg->cfg.nu_pre, zero_start, done);
+    // the down leg of level l; true: it restricted into level l+1 too
+    auto down = [&](int l, bool zero) {
+        if (zero && mg->lv[l].leg_down) {
+            leg<T>(mg, l, false, done);
+            return true;
+        }
+        relax<T, VAR>(mg, l, mg->cfg.nu_pre, zero, done);
+        return false;
+    };
+    bool restricted = L > 1 ? down(0, zero_start) : false;
     int post0 = mg->cfg.nu_post;  // level 0's post-sweeps left after a fused prolongation
+    if (L == 1) relax<T, VAR>(mg, 0, mg->cfg.nu_pre, zero_start, done);
     if (L > 1) {
         const int ldown = std::min(lt, L);
         for (int l = 1; l < ldown; ++l) {
-            restrict_to<T, VAR>(mg, l, done);
+            if (!restricted) restrict_to<T, VAR>(mg, l, done);
+            restricted = false;
             if (l == L - 1 && mg->cdirect) coarse_direct<T>(mg, done);
             else if (l == L - 1 && mg->c64 && sizeof(T) == 4)
                 coarse_smooth64<VAR>(mg, mg->cfg.nu_pre + mg->cfg.nu_post, done);
-            else relax<T, VAR>(mg, l, mg->cfg.nu_pre + (l == L - 1 ? mg->cfg.nu_post : 0), true, done);
+            else if (l == L - 1) relax<T, VAR>(mg, l, mg->cfg.nu_pre + mg->cfg.nu_post, true, done);
+            else restricted = down(l, true);
         }
         if (lt < L) {
-            restrict_to<T, VAR>(mg, lt, done);
+            if (!restricted) restrict_to<T, VAR>(mg, lt, done);
             tail<T, VAR>(mg, true, done);
         }
         for (int l = ldown - 1; l >= 0; --l) {
             if (l == L - 1) continue;
             int post = mg->cfg.nu_post;
-            if (fused_prolong(mg, l)) {
+            if (mg->lv[l].leg_up) {
+                leg<T>(mg, l, true, done);
+                post = 0;
+            } else if (fused_prolong(mg, l)) {
                 prolong_sweep<T, VAR>(mg, l, done);
                 --post;
             } else {
@@ -1678,8 +1723,109 @@ int adi_coef_build(mf3d_mg *mg) {
     return 0;
 }
 
+// Leg tiles (k_leg) of a level: LEG_TX x ty columns and chunks of tz planes
+// (even).  Every workgroup takes a compute unit's registers, so a launch
+// runs in rounds of `slots`, and a chunk costs its planes and the 7 to 8 steps
+// of its ring: the depth with the least rounds x (depth + 8), which is also
+// returned (*steps).
+std::vector<Tile> leg_tiles(const std::vector<BlockLevel> &hb, int ty, int slots, long long *steps) {
+    auto count = [&](int tz) {
+        long long n = 0;
+        for (const BlockLevel &g : hb)
+            n += (long long)((g.n0 + LEG_TX - 1) / LEG_TX) * ((g.n1 + ty - 1) / ty) * ((g.n2 + tz - 1) / tz);
+        return n;
+    };
+    int nzmax = 2, best = 2;
+    for (const BlockLevel &g : hb) nzmax = std::max(nzmax, g.n2);
+    long long cost = -1;
+    for (int tz = 2; tz <= nzmax; tz += 2) {
+        const long long c = (count(tz) + slots - 1) / slots * (tz + 8);
+        if (cost < 0 || c <= cost) {
+            cost = c;
+            best = tz;
+        }
+    }
+    *steps = cost;
+    std::vector<Tile> t;
+    for (int b = 0; b < (int)hb.size(); ++b) {
+        const BlockLevel &g = hb[b];
+        for (int z = 1; z <= g.n2; z += best)
+            for (int y = 1; y <= g.n1; y += ty)
+                for (int x = 1; x <= g.n0; x += LEG_TX) t.push_back(Tile{b, x, y, z, std::min(g.n2, z + best - 1)});
+    }
+    return t;
+}
+
+// Which levels run their legs as one launch each: red-black sweeps of lone
+// blocks with constant coefficients, two a leg, every extent even and at
+// least 8 (the ring of a tile then crosses one periodic face at most once a
+// side), above the LDS tail and the coarsest level.
+int leg_setup(mf3d_mg *mg) {
+    const mf3d_mg_cfg &c = mg->cfg;
+    const int L = c.levels;
+    const bool mixed = c.precision == MF3D_MIXED;
+    const bool any_up = c.nu_post == 2, any_down = any_up && c.nu_pre == 2;  // the down leg writes no ghosts: the up leg needs none
+    if (!mg->legs || c.smoother != 3 || c.variable_coef || mg->refined || !any_up) return 0;
+    const hipFuncAttribute attr = hipFuncAttributeMaxDynamicSharedMemorySize;
+    int cus = 0;
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
+    constexpr int SM = LEG_NY_SMALL, N4 = leg_ny<float>(), N8 = leg_ny<double>();
+    struct {
+        const void *fn;
+        int lds;
+    } ks[] = {{(const void *)k_leg<float, true, N4>, leg_lds<float>(true, true, N4)},
+              {(const void *)k_leg<float, false, N4>, leg_lds<float>(false, true, N4)},
+              {(const void *)k_leg<float, true, SM>, leg_lds<float>(true, true, SM)},
+              {(const void *)k_leg<float, false, SM>, leg_lds<float>(false, true, SM)},
+              {(const void *)k_leg<double, true, N8>, leg_lds<double>(true, true, N8)},
+              {(const void *)k_leg<double, false, N8>, leg_lds<double>(false, true, N8)},
+              {(const void *)k_leg<double, true, SM>, leg_lds<double>(true, true, SM)},
+              {(const void *)k_leg<double, false, SM>, leg_lds<double>(false, true, SM)}};
+    for (const auto &k : ks)
+        if (hipFuncSetAttribute(k.fn, attr, k.lds) != hipSuccess) {
+            mg->err = "hipFuncSetAttribute (leg LDS) failed";
+            return MF3D_EDEVICE;
+        }
+    for (int l = 0; l < std::min(mg->lt, L - 1); ++l) {
+        Level &V = mg->lv[l];
+        bool ok = V.own_ghosts;
+        int yper = 0;
+        for (const BlockLevel &g : V.hb) {
+            ok = ok && g.n0 >= 8 && g.n1 >= 8 && g.n2 >= 8 && !((g.n0 | g.n1 | g.n2) & 1);
+            yper |= !(g.neu & (kNeuS | kNeuN)) ? 2 : 1;
+        }
+        if (!ok || yper == 3) continue;  // the LDS layout is one for the launch
+        // The rows of a workgroup: a step takes 1.2 us with many rows and 0.95 with
+        // few, of which half belong to the ring.  Few on levels that leave compute
+        // units idle (64^3: 13.0 us against 14.7 a leg in FP32, 17.4 against 18.4 in
+        // FP64), many from where all are busy (128^3: 34 against 25).
+        long long many, few;
+        auto t = leg_tiles(V.hb, (mixed ? N4 : N8) - 8, std::max(1, cus), &many);
+        auto ts = leg_tiles(V.hb, SM - 8, std::max(1, cus), &few);
+        V.leg_ny = mixed ? N4 : N8;
+        if (few * 4 < many * 5) {
+            V.leg_ny = SM;
+            t = std::move(ts);
+        }
+        t = xcd_order(t);
+        V.n_leg = (int)t.size();
+        if (int rc = upload(mg, &V.t_leg, t)) return rc;
+        V.leg_down = any_down;
+        V.leg_up = any_up;
+    }
+    return 0;
+}
+
 int build(mf3d_mg *mg) {
     const mf3d_mg_cfg &c = mg->cfg;
+    {
+        const char *e = std::getenv("MF3D_LEGS");
+        if (e && std::strcmp(e, "0") != 0 && std::strcmp(e, "1") != 0) {
+            mg->err = "MF3D_LEGS must be 0 or 1";
+            return MF3D_EINVAL;
+        }
+        mg->legs = !(e && e[0] == '0');
+    }
     {
         const char *e = std::getenv("MF3D_FUSE_PROLONG");
         if (e && std::strcmp(e, "0") != 0 && std::strcmp(e, "1") != 0) {
@@ -1831,7 +1977,7 @@ int build(mf3d_mg *mg) {
         mg->n_out = (int)tout.size();
         if ((rc = upload(mg, &mg->t_out, tout))) return rc;
     }
-    if ((rc = decide_coarse(mg)) || (rc = choose_tail(mg))) return rc;
+    if ((rc = decide_coarse(mg)) || (rc = choose_tail(mg)) || (rc = leg_setup(mg))) return rc;
     if (mg->cdirect && (rc = coarse_setup(mg))) return rc;
     if (mg->c64) {
         const long long ghc = mg->lv[L - 1].cells_gh;

@@ -1,0 +1,518 @@
+// mg_leg.hpp -- one leg of the V-cycle on a level of a lone block in one
+// pass over memory: down (two red-black sweeps from zero, the residual and its
+// restriction) and up (prolongation and two red-black sweeps).
+//
+// What the sweeps, restriction and prolongation of a leg cost apart is their
+// passes over memory (5 and 6 fields in, 3 out and a quarter of one more) and,
+// on small levels, their launches.  Here a leg reads the RHS (and the
+// potential and the coarse potential) once and writes the potential (and
+// the coarse RHS) once.
+//
+// A workgroup owns a tile of columns and marches over planes.  A thread owns
+// two neighbouring columns of one row, the cells (i, i+1) with i odd, and
+// keeps their potential and RHS of the last planes in registers.  At step c
+// it updates, of the column whose turn it is, red plane c of the first
+// sweep, black plane c-1, red plane c-2 of the second sweep and black plane
+// c-3: four updates of one column, because the colour of a column's cells
+// alternates with the plane.  Labelling the columns by their parity instead
+// of their place -- A: i + j even, B: i + j odd -- makes that column the same
+// label in every thread, A on odd planes c and B on even ones, so with the
+// march unrolled nothing selects at run time.  An update's z neighbours and one
+// x neighbour are the thread's own registers, the other x neighbour is a
+// neighbouring lane's (a DPP move), the two y neighbours come through LDS, where
+// each update leaves its value.  An update reads there only what the step
+// before wrote, so every buffer has two halves used in turn and a step
+// has one barrier.
+//
+// Tiles overlap: cells in a ring around the stored ones are computed by the
+// neighbouring workgroups too, from the same inputs, one cell less on
+// every half sweep.  Beyond a periodic face the ring holds the cells it wraps
+// to.  The reference refreshes a block's ghosts only after a whole
+// sweep (mgsolver.for:610-611), so across such a face a black update reads
+// the red value from before the sweep: updates keep the value they replace
+// (o1, o2), and a neighbour across the face takes that one.  Beyond a wall
+// the coefficient is zero and the ring's values, finite, do not matter.
+// Same operands, same order as k_rbs, k_restrict and k_prolong: bitwise
+// their results.
+//
+// Measured on the level of 256^3 cells, sweeps and transfers apart against the
+// leg: FP32 down 125 us (47 + 50 + 28) against 71, up 127 (27 + 2 x 50) against 90;
+// FP64 down 264 against 140, up 310 against 190.  HBM traffic is 1.12 to 1.30
+// times what a leg has to move and takes half the time; the bound is a step's
+// serial chain, 2700 clocks in FP32 for about 120 vector and 80 scalar
+// instructions a wavefront between two barriers, the four updates
+// depending on each other.  Small levels: a fixed 3 us and 1 us a step, and the
+// instruction cache, cold in every launch, so rare cases (the planes
+// beside the z faces) take a divisor from LDS instead of code of their own: 64^3
+// FP32 13.0 a leg against 16.3 in two or three launches.
+#pragma once
+#include "mg_common.hpp"
+#include "mg_sweep.hpp"
+
+namespace mf3d {
+
+// Rows and pairs of columns (32) of a workgroup; the ring is 4 rows, and 6
+// columns: the outermost pair has no lane beside it to take coarse values from.
+// FP64 has 24 rows, 168 registers a thread; at 32 rows, 128, it spills.  Levels
+// too small to fill the card take LEG_NY_SMALL rows.
+constexpr int LEG_TX = 52, LEG_NY_SMALL = 16;
+template <typename T>
+constexpr int leg_ny() { return sizeof(T) == 4 ? 32 : 24; }
+
+template <int CTRL>
+__device__ __forceinline__ int dpp_i(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+// The value of lane - 1 (from_left) and lane + 1 (from_right); 0 past the wavefront's ends.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) { return __builtin_bit_cast(float, dpp_i<CTRL>(__builtin_bit_cast(int, v))); }
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+    const uint2 b = __builtin_bit_cast(uint2, v);
+    return __builtin_bit_cast(double, uint2{(unsigned)dpp_i<CTRL>((int)b.x), (unsigned)dpp_i<CTRL>((int)b.y)});
+}
+template <typename T> __device__ __forceinline__ T from_left(T v) { return dpp<0x138>(v); }
+template <typename T> __device__ __forceinline__ T from_right(T v) { return dpp<0x130>(v); }
+
+// Planes in flight: what the registers leave room for.
+template <typename T, bool UP>
+constexpr int leg_depth() { return sizeof(T) == 8 && UP ? 1 : 3; }
+
+// Two neighbouring entries of a field, at a byte offset of any alignment of
+// one entry.
+template <typename T> struct Pair { T l, r; };
+template <typename T> __device__ __forceinline__ Pair<T> bload2(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff);
+template <> __device__ __forceinline__ Pair<float> bload2<float>(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(Pair<float>, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+}
+template <> __device__ __forceinline__ Pair<double> bload2<double>(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(Pair<double>, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
+template <typename T> __device__ __forceinline__ void bstore2(__amdgpu_buffer_rsrc_t r, Pair<T> v, uint32_t voff, uint32_t soff);
+template <> __device__ __forceinline__ void bstore2<float>(__amdgpu_buffer_rsrc_t r, Pair<float> v, uint32_t voff, uint32_t soff) {
+    using V = decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V, v), r, voff, soff, 0);
+}
+template <> __device__ __forceinline__ void bstore2<double>(__amdgpu_buffer_rsrc_t r, Pair<double> v, uint32_t voff, uint32_t soff) {
+    using V = decltype(__builtin_amdgcn_raw_buffer_load_b128(r, 0, 0, 0));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(V, v), r, voff, soff, 0);
+}
+
+// The cell 1..n that coordinate v stands for: around a periodic axis, or
+// the nearest one beyond walls.
+__device__ __forceinline__ int leg_map(int v, int n, bool per) {
+    if (!per) return v < 1 ? 1 : (v > n ? n : v);
+    while (v < 1) v += n;
+    while (v > n) v -= n;
+    return v;
+}
+
+// LDS: a thread's divisors on the planes beside the z faces (four), then
+// halves of 32 * (rows + 2) entries: up: the old black, red 1, black 1, red 2
+// planes (two each) and, where y is periodic, the reds they replace; down: red
+// 1, black 1 (two each), red 2 (three), black 2 (two), then the replaced reds.
+template <typename T>
+constexpr int leg_lds(bool up, bool yper, int ny) {
+    return 32 * (int)sizeof(T) * (4 * ny + (ny + 2) * (up ? 8 + (yper ? 4 : 0) : 9 + (yper ? 2 : 0)));
+}
+
+template <typename T, bool UP, int NY>
+__global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *__restrict__ pout,
+                                                const T *__restrict__ rhs, uint32_t bytes,
+                                                const BlockLevel *__restrict__ bls, const Tile *__restrict__ tiles,
+                                                const int *__restrict__ done, const T *__restrict__ phic,
+                                                T *__restrict__ rhsc, uint32_t cbytes,
+                                                const BlockLevel *__restrict__ blc) {
+    if (done && *done) return;
+    extern __shared__ __align__(16) unsigned char leg_smem[];
+    T *face = reinterpret_cast<T *>(leg_smem), *sm = face + 4 * 32 * NY;
+    constexpr uint32_t W = sizeof(T);
+    constexpr int LEG_NT = 32 * NY, LEG_TY = NY - 8, LEG_ROW = 32 * (NY + 2);
+    constexpr int NS = 6;  // planes in the registers' rings, the unroll
+    const Tile t = tiles[blockIdx.x];
+    const BlockLevel g = bls[t.b], gc = blc[t.b];
+    const auto rs_in = make_rsrc(pin, bytes), rs_f = make_rsrc(rhs, bytes), rs_out = make_rsrc(pout, bytes);
+    const auto rs_c = make_rsrc(UP ? phic : rhsc, cbytes);
+    // A wavefront takes two rows: down, whose restriction adds them, an odd row
+    // and the even one after it; up two rows of one parity, whose prolongation
+    // weights are then scalars.
+    const int tid = (int)threadIdx.x;
+    const int row = UP ? (tid >> 7) * 4 + ((tid >> 6) & 1) + ((tid >> 5) & 1) * 2 : tid >> 5;
+    const int pair = (row & 1) ? 31 - (tid & 31) : (tid & 31);
+    const int i = t.x0 - 6 + 2 * pair, j = t.y0 - 4 + row;  // i odd: the pair (i, i+1)
+    const bool px = !(g.neu & (kNeuW | kNeuE)), py = !(g.neu & (kNeuS | kNeuN)), pz = !(g.neu & (kNeuB | kNeuT));
+    const int im = leg_map(i, g.n0, px) | 1, jm = leg_map(j, g.n1, py);  // | 1: beyond a wall, the last pair's left
+    const int ip = im > g.n0 ? g.n0 - 1 : im;
+    const uint32_t pb = (uint32_t)g.sz * W, cpb = (uint32_t)gc.sz * W, csy = (uint32_t)gc.sy * W;
+    const uint32_t vo = ((uint32_t)g.off + (uint32_t)(ip + (int)g.sy * jm)) * W;
+    const uint32_t vc = ((uint32_t)gc.off + (uint32_t)(((ip + 1) >> 1) + (int)gc.sy * (jm >> 1))) * W;
+    // Column A (i + j even) is the left one of an odd row's pairs and the right
+    // one of an even row's.  Even rows run from right to left, so that A's outer
+    // x neighbour is the lane before in both, and B's the one after.
+    const bool la = UP ? (__builtin_amdgcn_readfirstlane(j) & 1) != 0 : (j & 1) != 0;
+    // coefficients: towards the pair's other column always c0; towards the
+    // outer side zero at a wall (FP64 keeps c0 and takes a zero neighbour);
+    // S and N are c1, a wall row's neighbour read as zero from a pad row
+    const T c0 = cconst<T>(g, 0), c1 = cconst<T>(g, 1), c2 = cconst<T>(g, 2);
+    const bool wL = i == 1 && (g.neu & kNeuW), wR = i + 1 == g.n0 && (g.neu & kNeuE);
+    const T oL = wL ? T(0) : c0, oR = wR ? T(0) : c0;
+    const T oA = la ? oL : oR, oB = la ? oR : oL;
+    const T wA = la ? oL : c0, eAc = la ? c0 : oR, wB = la ? c0 : oL, eBc = la ? oR : c0;  // aw and ae
+    const bool wS = j == 1 && (g.neu & kNeuS), wN = j == g.n1 && (g.neu & kNeuN);
+    constexpr bool RCP = sizeof(T) == 4;  // the FP32 inner cycle multiplies by 1/ap
+    auto part = [&](T o) {  // a column's diagonal without the z faces
+        T s = o + c0;  // aw + ae: one of them is c0, the sum does not depend on the order
+        s = s + (wS ? T(0) : c1);
+        return s + (wN ? T(0) : c1);
+    };
+    auto diag = [](T s, T ab, T at) { return -((s + ab) + at); };
+    auto divisor = [&](T s, T ab, T at) { return RCP ? T(1) / diag(s, ab, at) : diag(s, ab, at); };
+    const T sA = part(oA), sB = part(oB);
+    const T dA = divisor(sA, c2, c2), dB = divisor(sB, c2, c2);
+    // divisors of planes 1 and n2 of the two columns
+    auto at_face = [&](int m, bool isA) -> T & { return face[((m == 1 ? 0 : 2) + (isA ? 0 : 1)) * LEG_NT + tid]; };
+    const T wallB = g.neu & kNeuB ? T(0) : c2, wallT = g.neu & kNeuT ? T(0) : c2;
+    at_face(1, true) = divisor(sA, wallB, c2);
+    at_face(1, false) = divisor(sB, wallB, c2);
+    at_face(g.n2, true) = divisor(sA, c2, wallT);
+    at_face(g.n2, false) = divisor(sB, c2, wallT);
+    // the red value of this column that goes to the lane across a periodic
+    // face is the one from before the sweep
+    const bool eL = px && ip == 1, eR = px && ip + 1 == g.n0;
+    const bool eA = la ? eL : eR, eB = la ? eR : eL;
+    // this thread's entry of an LDS half (after a pad row), its y neighbours'
+    // (a pad row's zero beyond a wall), and whether one lies across a periodic face
+    const int at0 = 32 * (row + 1) + pair, atS = wS ? pair : at0 - 32, atN = wN ? pair : at0 + 32;
+    const bool ySo = py && jm == 1, yNo = py && jm == g.n1;
+
+    auto buf = [&](int b, int slot) { return sm + (2 * b + slot) * LEG_ROW; };
+    // buffers: up 0 old black, 1 red 1, 2 black 1, 3 red 2, 4 / 5 the reds that
+    // sweep 1 / 2 replaced; down 1 -> 0 red 1, 2 -> 1 black 1, 2 black 2, (red 2:
+    // three planes after those), 4 the reds that sweep 2 replaced
+    constexpr int R1 = UP ? 1 : 0, B1 = UP ? 2 : 1, B2 = 2, O1 = 4, O2 = UP ? 5 : 4;
+    auto red2 = [&](int slot2, int slot3) { return UP ? buf(3, slot2) : sm + (6 + slot3) * LEG_ROW; };
+    auto old2 = [&](int slot2) { return UP ? buf(O2, slot2) : sm + (9 + slot2) * LEG_ROW; };
+    for (int e = tid; e < LEG_ROW * (UP ? 8 + (py ? 4 : 0) : 9 + (py ? 2 : 0)); e += LEG_NT)
+        sm[e] = T(0);  // the pad rows stay zero; the first steps read the rest before it is written
+    __syncthreads();
+
+    T A[NS], B[NS], fA[NS], fB[NS], o1[NS], o2[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) A[s] = B[s] = fA[s] = fB[s] = o1[s] = o2[s] = T(0);
+
+    // Loads run D planes ahead, so a step's wait finds them done.  Planes 2m and
+    // 2m + 1 take the coarse planes m and m + 1 (rows jm/2 and jm/2 + 1 of each,
+    // e0 and e1; around a periodic axis a ghost plane holds the same values as
+    // the plane it wraps to); en: plane m + 2, on its way.
+    constexpr int D = leg_depth<T, UP>();
+    struct In {
+        Pair<T> f, p;
+    } L[D];
+    T e0[2], e1[2], en[2];
+    auto load = [&](In &q, int k) {  // plane k (mapped)
+        q.f = bload2<T>(rs_f, vo, (uint32_t)k * pb);
+        if constexpr (UP) q.p = bload2<T>(rs_in, vo, (uint32_t)k * pb);
+    };
+    auto load_c = [&](T *e, int m) {  // coarse plane m of the unwrapped planes 2m - 2 .. 2m + 1
+        const int nc = g.n2 >> 1, k = pz ? (m < 1 ? m + nc : (m > nc ? m - nc : m)) : (m < 0 ? 0 : (m > nc + 1 ? nc + 1 : m));
+        e[0] = bload<T>(rs_c, vc, (uint32_t)k * cpb);
+        e[1] = bload<T>(rs_c, vc + csy, (uint32_t)k * cpb);
+    };
+    // a plane's values, the potential corrected as k_prolong does it
+    auto take = [&](const In &q, bool odd, T &a, T &b, T &ra, T &rb) {
+        ra = la ? q.f.l : q.f.r;
+        rb = la ? q.f.r : q.f.l;
+        if constexpr (UP) {
+            const T m[4] = {e0[0], e0[1], e1[0], e1[1]};
+            // weights of the coarse rows and planes, literals: every call has
+            // its plane's parity and its branch the row's
+            auto weight = [&](int n, bool odd_row) {
+                return T((((n & 1) != 0) == odd_row ? 3 : 1) * (((n & 2) != 0) == odd ? 3 : 1));
+            };
+            // the pair's own coarse column (weight 3) and the outer one (weight
+            // 1): the left column's terms begin with the outer one's
+            auto outer_first = [&](auto shift, bool odd_row) {
+                T v = weight(0, odd_row) * shift(m[0]);
+#pragma unroll
+                for (int n = 1; n < 4; ++n) v = v + weight(n, odd_row) * shift(m[n]);
+#pragma unroll
+                for (int n = 0; n < 4; ++n) v = v + (T(3) * weight(n, odd_row)) * m[n];
+                return v;
+            };
+            auto own_first = [&](auto shift, bool odd_row) {
+                T v = (T(3) * weight(0, odd_row)) * m[0];
+#pragma unroll
+                for (int n = 1; n < 4; ++n) v = v + (T(3) * weight(n, odd_row)) * m[n];
+#pragma unroll
+                for (int n = 0; n < 4; ++n) v = v + weight(n, odd_row) * shift(m[n]);
+                return v;
+            };
+            auto before = [](T v) { return from_left(v); };
+            auto after = [](T v) { return from_right(v); };
+            if (la) {  // uniform: an odd row
+                a = q.p.l + outer_first(before, true) / T(64);
+                b = q.p.r + own_first(after, true) / T(64);
+            } else {
+                a = q.p.r + own_first(before, false) / T(64);
+                b = q.p.l + outer_first(after, false) / T(64);
+            }
+        }
+    };
+    auto next = [&](int z, int before) {  // the plane that plane z maps to, after `before`'s
+        return pz ? (before == g.n2 ? 1 : before + 1) : (z < 1 ? 1 : (z > g.n2 ? g.n2 : z));
+    };
+    // One update of column A (X_A) or B on a plane mapped to m.  The outer x
+    // neighbour and the own one are ordered W, E in FP32, whose sum contracts;
+    // in FP64 the two products are rounded before they are added and the
+    // order is free.  zB, zT: the neighbours below and above; qB, qT: those a
+    // black update takes across a periodic face.
+    auto sum = [&](bool isA, T outer, T own, T yS, T yN, T ab, T zB, T at, T zT) -> T {
+        T s;
+        if constexpr (RCP) {
+            const bool left = isA ? la : !la;
+            s = (isA ? wA : wB) * (left ? outer : own);
+            s = madd(s, isA ? eAc : eBc, left ? own : outer);
+        } else {
+            s = c0 * outer;
+            s = s + c0 * own;
+        }
+        s = madd(s, c1, yS);
+        s = madd(s, c1, yN);
+        s = madd(s, ab, zB);
+        s = madd(s, at, zT);
+        return s;
+    };
+    auto relax = [&](bool isA, T r, T outer, T own, T yS, T yN, int m, T zB, T zT, T qB, T qT) -> T {
+        T d = isA ? dA : dB, ab = c2, at = c2;
+        if (m == 1 || m == g.n2) {  // uniform, rare
+            d = at_face(m, isA);
+            if (m == 1) {
+                ab = wallB;
+                if (pz) zB = qB;
+            } else {
+                at = wallT;
+                if (pz) zT = qT;
+            }
+        }
+        const T s = sum(isA, outer, own, yS, yN, ab, zB, at, zT);
+        return RCP ? (r - s) * d : (r - s) / d;
+    };
+    const bool xw = sizeof(T) == 8 && !px, xA = xw && (la ? wL : wR), xB = xw && (la ? wR : wL);  // A, B beside a wall
+    auto outer_of = [&](bool isA, T v) {
+        T o = isA ? from_left(v) : from_right(v);
+        if (xw) o = (isA ? xA : xB) ? T(0) : o;  // uniform
+        return o;
+    };
+
+    const int cm = UP ? t.z0 - 3 : t.z0 - 4, ce = UP ? t.z1 + 3 : t.z1 + 4;  // first and last step
+    constexpr int P0 = UP ? 0 : 1;                                           // parity of cm (z0 is odd)
+    // plane cm + d sits in slot d mod NS; mz: the plane each slot's maps to
+    int mz[NS];
+#pragma unroll
+    for (int d = -4; d < 2; ++d) mz[(d + NS) % NS] = leg_map(cm + d, g.n2, pz);
+    int kl = mz[1];  // the last plane asked for
+    {
+        In q[3];
+        if constexpr (UP) {  // planes cm - 1 (odd), cm, cm + 1
+            load(q[0], mz[NS - 1]);
+            load_c(e0, (cm - 2) / 2);
+            load_c(e1, cm / 2);
+            load_c(en, cm / 2 + 1);
+        }
+        load(q[1], mz[0]);
+        load(q[2], mz[1]);
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            kl = next(cm + 2 + d, kl);
+            load(L[d], kl);
+        }
+        if constexpr (UP) {
+            take(q[0], true, A[NS - 1], B[NS - 1], fA[NS - 1], fB[NS - 1]);
+            e0[0] = e1[0];
+            e0[1] = e1[1];
+            e1[0] = en[0];
+            e1[1] = en[1];
+            load_c(en, cm / 2 + 2);
+        }
+        take(q[1], P0, A[0], B[0], fA[0], fB[0]);
+        take(q[2], !P0, A[1], B[1], fA[1], fB[1]);
+        if constexpr (UP) buf(0, P0)[at0] = P0 ? B[0] : A[0];  // black: A on even planes
+    }
+    __syncthreads();
+
+    const bool stored = pair >= 3 && pair < 3 + LEG_TX / 2 && i <= g.n0 && row >= 4 && row < 4 + LEG_TY && j <= g.n1;
+    const bool img = __any(stored && (ghost_image(i, g.n0, g.neu & kNeuW, g.neu & kNeuE) >= 0 ||
+                                      ghost_image(i + 1, g.n0, g.neu & kNeuW, g.neu & kNeuE) >= 0 ||
+                                      ghost_image(j, g.n1, g.neu & kNeuS, g.neu & kNeuN) >= 0));  // in the wavefront
+    const int sy = (int)g.sy;
+    const uint32_t ob = (uint32_t)g.off * W;
+    auto roff = [&](int x, int y) { return ob + (uint32_t)(x + sy * y) * W; };
+    const uint32_t vs = roff(i, j);
+    auto store = [&](int z, T a, T b) {  // plane z of this thread's stored cells and their ghost images
+        if (z < t.z0 || z > t.z1) return;  // uniform
+        if (!stored) return;
+        const Pair<T> v{la ? a : b, la ? b : a};
+        bstore2<T>(rs_out, v, vs, (uint32_t)z * pb);
+        if (!UP || !(img || z == 1 || z == g.n2)) return;  // uniform; the up leg reads no ghosts of its level
+        const int iz = ghost_image(z, g.n2, g.neu & kNeuB, g.neu & kNeuT);
+        int x = i, y = j;  // opaque, or the addresses of every image stay in registers
+        asm volatile("" : "+v"(x), "+v"(y));
+        const int xl = ghost_image(x, g.n0, g.neu & kNeuW, g.neu & kNeuE);
+        const int xr = ghost_image(x + 1, g.n0, g.neu & kNeuW, g.neu & kNeuE);
+        const int yg = ghost_image(y, g.n1, g.neu & kNeuS, g.neu & kNeuN);
+        auto plane = [&](int zz) {
+            const uint32_t s = (uint32_t)zz * pb;
+            if (zz != z) bstore2<T>(rs_out, v, roff(x, y), s);
+            if (yg >= 0) bstore2<T>(rs_out, v, roff(x, yg), s);
+            if (xl >= 0) {
+                bstore<T>(rs_out, v.l, roff(xl, y), s);
+                if (yg >= 0) bstore<T>(rs_out, v.l, roff(xl, yg), s);
+            }
+            if (xr >= 0) {
+                bstore<T>(rs_out, v.r, roff(xr, y), s);
+                if (yg >= 0) bstore<T>(rs_out, v.r, roff(xr, yg), s);
+            }
+        };
+        plane(z);
+        if (iz >= 0) plane(iz);
+    };
+
+    const uint32_t vcs = ((uint32_t)gc.off + (uint32_t)(((i + 1) >> 1) + (int)gc.sy * ((j + 1) >> 1))) * W;
+    T acc = T(0);  // down: the restricted residual's sum so far
+    // Step J of a turn, plane c = cm + NS m + J: X is the column updated in
+    // it (red on planes c and c-2, black on c-1 and c-3), Y the other.
+    auto step = [&](int c, auto jc) {
+        constexpr int J = decltype(jc)::value, PC = (J + P0) & 1, J3 = J % 3;
+        constexpr auto sl = [](int d) { return ((J + d) % NS + NS) % NS; };
+        constexpr bool XA = PC != 0;  // X is column A
+        T *X = XA ? A : B, *Y = XA ? B : A;
+        const T *fX = XA ? fA : fB, *fY = XA ? fB : fA;
+        const bool edge = XA ? eB : eA;  // of the sending column, Y
+        mz[sl(2)] = next(c + 2, mz[sl(1)]);
+        // the y neighbours of the four updates, written in the step before
+        T y1S = T(0), y1N = T(0);
+        if constexpr (UP) {
+            const T *b0 = buf(0, PC);
+            y1S = b0[atS];
+            y1N = b0[atN];
+        }
+        const T *b1 = buf(R1, 1 - PC), *b2 = buf(B1, PC), *b3 = red2(1 - PC, (J3 + 1) % 3);
+        T y2S = b1[atS], y2N = b1[atN];
+        const T y3S = b2[atS], y3N = b2[atN];
+        T y4S = b3[atS], y4N = b3[atN];
+        if (py) {  // uniform
+            if constexpr (UP) {
+                const T *q = buf(O1, 1 - PC);
+                const T a = q[atS], b = q[atN];
+                y2S = ySo ? a : y2S;
+                y2N = yNo ? b : y2N;
+            } else {
+                y2S = ySo ? T(0) : y2S;
+                y2N = yNo ? T(0) : y2N;
+            }
+            const T *q = old2(1 - PC);
+            const T a = q[atS], b = q[atN];
+            y4S = ySo ? a : y4S;
+            y4N = yNo ? b : y4N;
+        }
+        if constexpr (UP) buf(0, 1 - PC)[at0] = X[sl(1)];  // plane c+1: its black column is X
+
+        // red, sweep 1, plane c
+        if constexpr (UP) {
+            const T v = X[sl(0)];
+            o1[sl(0)] = v;
+            if (py) buf(O1, PC)[at0] = v;
+            X[sl(0)] = relax(XA, fX[sl(0)], outer_of(XA, Y[sl(0)]), Y[sl(0)], y1S, y1N, mz[sl(0)], X[sl(-1)], X[sl(1)],
+                             X[sl(-1)], X[sl(1)]);
+        } else {
+            const int m = mz[sl(0)];
+            T d = XA ? dA : dB;
+            if (m == 1 || m == g.n2) d = at_face(m, XA);
+            X[sl(0)] = RCP ? (fX[sl(0)] - T(0)) * d : (fX[sl(0)] - T(0)) / d;
+        }
+        buf(R1, PC)[at0] = X[sl(0)];
+
+        // black, sweep 1, plane c-1; across a periodic face the old reds
+        {
+            const T yv = edge ? o1[sl(-1)] : Y[sl(-1)];
+            X[sl(-1)] = relax(XA, fX[sl(-1)], outer_of(XA, yv), Y[sl(-1)], y2S, y2N, mz[sl(-1)], X[sl(-2)], X[sl(0)],
+                              o1[sl(-2)], o1[sl(0)]);
+            buf(B1, 1 - PC)[at0] = X[sl(-1)];
+        }
+        // red, sweep 2, plane c-2
+        {
+            const T v = X[sl(-2)];
+            o2[sl(-2)] = v;
+            if (py) old2(PC)[at0] = v;
+            X[sl(-2)] = relax(XA, fX[sl(-2)], outer_of(XA, Y[sl(-2)]), Y[sl(-2)], y3S, y3N, mz[sl(-2)], X[sl(-3)],
+                              X[sl(-1)], X[sl(-3)], X[sl(-1)]);
+            red2(PC, (J3 + 2) % 3)[at0] = X[sl(-2)];
+        }
+        // black, sweep 2, plane c-3
+        {
+            const T yv = edge ? o2[sl(-3)] : Y[sl(-3)];
+            X[sl(-3)] = relax(XA, fX[sl(-3)], outer_of(XA, yv), Y[sl(-3)], y4S, y4N, mz[sl(-3)], X[sl(-4)], X[sl(-2)],
+                              o2[sl(-4)], o2[sl(-2)]);
+            if constexpr (!UP) buf(B2, 1 - PC)[at0] = X[sl(-3)];
+        }
+        store(c - 3, A[sl(-3)], B[sl(-3)]);
+
+        if constexpr (!UP) {  // the residual of plane c-4, its ghosts refreshed, into the coarse RHS
+            const int z = c - 4;  // only planes of the chunk matter, which map to themselves
+            const T ab = z == 1 ? wallB : c2, at = z == g.n2 ? wallT : c2;
+            const T *bb = buf(B2, PC), *br = red2(0, J3);
+            auto res = [&](bool isA, T o, T f, T own, T outer, T yS, T yN, T zB, T zT, T self) {
+                // without contraction, as k_restrict: aw*W + ae*E is free of order
+                T s = (RCP ? o : c0) * outer;
+                s = s + c0 * own;
+                s = s + c1 * yS;
+                s = s + c1 * yN;
+                s = s + ab * zB;
+                s = s + at * zT;
+                s = s + diag(isA ? sA : sB, ab, at) * self;
+                return f - s;
+            };
+            // X on plane c-4 is red (its y neighbours black 2), Y black (red 2)
+            const T rx = res(XA, XA ? oA : oB, fX[sl(-4)], Y[sl(-4)], outer_of(XA, Y[sl(-4)]), bb[atS], bb[atN],
+                             X[sl(-5)], X[sl(-3)], X[sl(-4)]);
+            const T ry = res(!XA, XA ? oB : oA, fY[sl(-4)], X[sl(-4)], outer_of(!XA, X[sl(-4)]), br[atS], br[atN],
+                             Y[sl(-5)], Y[sl(-3)], Y[sl(-4)]);
+            const T ra = XA ? rx : ry, rb = XA ? ry : rx;
+            // the even row's (A is its right column): the same pair, in the
+            // wavefront's upper half from the other end
+            const T ul = __shfl_xor(rb, 63, 64), ur = __shfl_xor(ra, 63, 64);
+            // children in the order (0,0,0) (1,0,0) (0,1,0) (1,1,0) (0,0,1) (1,0,1) (0,1,1) (1,1,1)
+            acc = PC ? ra : acc + ra;  // plane c-4 odd: the lower one
+            acc = acc + rb;
+            acc = acc + ul;
+            acc = acc + ur;
+            if (!PC && z >= t.z0 && z <= t.z1 && stored && !(row & 1)) bstore<T>(rs_c, T(0.125) * acc, vcs, (uint32_t)(z >> 1) * cpb);
+        }
+        if constexpr (UP && PC == 0) {  // plane c+2 is even: the next two coarse planes
+            e0[0] = e1[0];
+            e0[1] = e1[1];
+            e1[0] = en[0];
+            e1[1] = en[1];
+            load_c(en, (c + 2) / 2 + 2);
+        }
+        take(L[J % D], PC != 0, A[sl(2)], B[sl(2)], fA[sl(2)], fB[sl(2)]);
+        kl = next(c + 2 + D, kl);
+        load(L[J % D], kl);
+        __syncthreads();
+    };
+    for (int c = cm; c <= ce; c += NS) {
+        step(c, Step<0>{});
+        if (c + 1 > ce) break;
+        step(c + 1, Step<1>{});
+        if (c + 2 > ce) break;
+        step(c + 2, Step<2>{});
+        if (c + 3 > ce) break;
+        step(c + 3, Step<3>{});
+        if (c + 4 > ce) break;
+        step(c + 4, Step<4>{});
+        if (c + 5 > ce) break;
+        step(c + 5, Step<5>{});
+    }
+}
+
+}  // namespace mf3d
