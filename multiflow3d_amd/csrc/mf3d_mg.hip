@@ -223,6 +223,9 @@ struct mf3d_mg {
     // levels on 3-D tiles fuse the prolongation into their first post-sweep
     // (k_rb3d<..., PRO>); MF3D_FUSE_PROLONG=0 keeps them apart, bitwise the same
     bool fuse_pro = true;
+    // the outer passes form level 0's coefficients from the density instead of
+    // reading the face arrays, bitwise the same (MF3D_OUTER_DENSITY=1 / 0: always / never)
+    bool dens_outer = false;
     // a lone block's levels run each leg of the cycle in one launch (k_leg);
     // MF3D_LEGS=0 keeps sweeps, restriction and prolongation apart, bitwise the same
     bool legs = true;
@@ -1035,21 +1038,21 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
 // initial residual, first = true).  Defect correction: p += e, r = f - A p.
 // GCR(1): beta from (A z, w_prev), d = z - beta d_prev, w = A d, alpha,
 // p += alpha d, r = f - A p.
-template <typename T, bool VAR>
-void outer_step(mf3d_mg *mg, int from, const int *done, bool first = false) {
+template <typename T, int COEF>
+void outer_step_c(mf3d_mg *mg, int from, const int *done, bool first) {
     Level &L0 = mg->lv[0];
-    const double *cx = VAR ? L0.dcx : nullptr, *cy = VAR ? L0.dcy : nullptr, *cz = VAR ? L0.dcz : nullptr;
+    const OuterCoef cf{L0.dcx, L0.dcy, L0.dcz, L0.dens};
     const bool tk = tk_on(mg, MF3D_K_OUTER, 0);
     if (mg->cfg.krylov == MF3D_OUTER_GCR) {
         const T *z = (const T *)L0.phi[L0.cur];
         if (!first) {
-            hipLaunchKernelGGL((k_krylov_lds<2, T, T, VAR, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, z,
-                               nullptr, nullptr, nullptr, mg->kw, nullptr, nullptr, cx, cy, cz, mg->st, L0.db,
+            hipLaunchKernelGGL((k_krylov_lds<2, T, T, COEF, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, z,
+                               nullptr, nullptr, nullptr, mg->kw, nullptr, nullptr, cf, mg->st, L0.db,
                                mg->t_out, mg->partials, done);
             hipLaunchKernelGGL(k_gcr_scalar<true>, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts,
                                mg->st);
-            hipLaunchKernelGGL((k_krylov_lds<1, T, T, VAR, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, z,
-                               mg->kd[from], mg->kd[1 - from], nullptr, mg->kr, mg->kw, nullptr, cx, cy, cz, mg->st,
+            hipLaunchKernelGGL((k_krylov_lds<1, T, T, COEF, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, z,
+                               mg->kd[from], mg->kd[1 - from], nullptr, mg->kr, mg->kw, nullptr, cf, mg->st,
                                L0.db, mg->t_out, mg->partials, done);
             hipLaunchKernelGGL(k_gcr_scalar<false>, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts,
                                mg->st);
@@ -1060,15 +1063,15 @@ void outer_step(mf3d_mg *mg, int from, const int *done, bool first = false) {
                                mg->kd[1 - from], mg->st, L0.cells_gh, done);
             fill_ghosts<double>(mg, L0, mg->pbuf[1 - from], done);
             if (tk) tk_mark(mg);
-            hipLaunchKernelGGL((k_krylov_lds<3, double, T, VAR, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0,
+            hipLaunchKernelGGL((k_krylov_lds<3, double, T, COEF, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0,
                                mg->stream, mg->pbuf[1 - from], nullptr, nullptr, mg->f_g, nullptr, mg->kr,
-                               (T *)L0.rhs, cx, cy, cz, mg->st, L0.db, mg->t_out, mg->partials, done);
+                               (T *)L0.rhs, cf, mg->st, L0.db, mg->t_out, mg->partials, done);
             if (tk) tk_mark(mg);
         } else {
             if (tk) tk_mark(mg);
-            hipLaunchKernelGGL((k_krylov_lds<0, double, T, VAR, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0,
+            hipLaunchKernelGGL((k_krylov_lds<0, double, T, COEF, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0,
                                mg->stream, mg->pbuf[from], mg->kd[1 - from], mg->pbuf[1 - from], mg->f_g, nullptr,
-                               mg->kr, (T *)L0.rhs, cx, cy, cz, mg->st, L0.db, mg->t_out, mg->partials, done);
+                               mg->kr, (T *)L0.rhs, cf, mg->st, L0.db, mg->t_out, mg->partials, done);
             if (tk) tk_mark(mg);
         }
         hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts, mg->st,
@@ -1081,8 +1084,8 @@ void outer_step(mf3d_mg *mg, int from, const int *done, bool first = false) {
                            (const T *)L0.phi[L0.cur], L0.cells_gh, done);
         fill_ghosts<double>(mg, L0, mg->pbuf[1 - from], done);
         if (tk) tk_mark(mg);
-        hipLaunchKernelGGL((k_outer_lds<T, VAR, 8, false>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream,
-                           mg->pbuf[1 - from], nullptr, (const T *)nullptr, mg->f_g, (T *)L0.rhs, cx, cy, cz, L0.db,
+        hipLaunchKernelGGL((k_outer_lds<T, COEF, 8, false>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream,
+                           mg->pbuf[1 - from], nullptr, (const T *)nullptr, mg->f_g, (T *)L0.rhs, cf, L0.db,
                            mg->t_out, mg->partials, done);
         if (tk) tk_mark(mg);
         hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts, mg->st,
@@ -1090,12 +1093,20 @@ void outer_step(mf3d_mg *mg, int from, const int *done, bool first = false) {
         return;
     }
     if (tk) tk_mark(mg);
-    hipLaunchKernelGGL((k_outer_lds<T, VAR, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, mg->pbuf[from],
-                       mg->pbuf[1 - from], (const T *)L0.phi[L0.cur], mg->f_g, (T *)L0.rhs, cx, cy, cz, L0.db,
+    hipLaunchKernelGGL((k_outer_lds<T, COEF, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, mg->pbuf[from],
+                       mg->pbuf[1 - from], (const T *)L0.phi[L0.cur], mg->f_g, (T *)L0.rhs, cf, L0.db,
                        mg->t_out, mg->partials, done);
     if (tk) tk_mark(mg);
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts, mg->st,
                        mg->d_hist, mg->d_rmax, mg->cfg.min_cycles);
+}
+
+template <typename T, bool VAR>
+void outer_step(mf3d_mg *mg, int from, const int *done, bool first = false) {
+    if constexpr (VAR)
+        mg->dens_outer ? outer_step_c<T, kCoefDensity>(mg, from, done, first)
+                       : outer_step_c<T, kCoefArrays>(mg, from, done, first);
+    else outer_step_c<T, kCoefConst>(mg, from, done, first);
 }
 
 // Record one cycle reading pbuf[g] into a graph.
@@ -1973,6 +1984,17 @@ int build(mf3d_mg *mg) {
     }
     Level &L0 = mg->lv[0];
     {
+        const char *e = std::getenv("MF3D_OUTER_DENSITY");
+        if (e && std::strcmp(e, "0") != 0 && std::strcmp(e, "1") != 0) {
+            mg->err = "MF3D_OUTER_DENSITY must be 0 or 1";
+            return MF3D_EINVAL;
+        }
+        const int dens = e ? e[0] - '0' : 2;  // 2: by size
+        // From 2^22 cells the coefficients come from the density: below, the face
+        // arrays fit in the caches and the divisions cost more than their bytes
+        // (us for the three passes of a GCR step, arrays / density: 96^3 43 / 52,
+        // 160^3 164 / 159, 192^3 261 / 237, 256^3 580 / 496, 384^3 2127 / 1599).
+        mg->dens_outer = c.variable_coef && (dens == 2 ? L0.cells_gh > (1LL << 22) : dens == 1);
         auto tout = xcd_order(sweep_tiles(L0.hb, 8));
         mg->n_out = (int)tout.size();
         if ((rc = upload(mg, &mg->t_out, tout))) return rc;

@@ -6,6 +6,118 @@
 
 namespace mf3d {
 
+// Where the passes below take level 0's coefficients from: constants, the face
+// arrays, or the density.
+enum { kCoefConst, kCoefArrays, kCoefDensity };
+struct OuterCoef {
+    const double *__restrict__ x, *__restrict__ y, *__restrict__ z, *__restrict__ dens;
+};
+
+// Level-0 face coefficients from the density, as k_lsm_coef writes them, for the
+// z-marching passes below: a face takes the mean of its two cells, at the
+// block's edge the cell inside, 0 on a Neumann face.  Those passes are bound by
+// memory, and the density is 8 bytes a cell where the three coefficient
+// arrays are 24.  A division takes a SIMD 62 clocks, so each face of a tile is
+// formed once: a thread forms the west and south faces of its cell and, as
+// the planes go by, the top one (the next plane's bottom one); two of the
+// wavefronts also those east and north of the tile.  x and y faces
+// pass through LDS (two planes, used in turn).  At 384^3 the GCR passes (MODE 0, 1,
+// 2 below) took 928, 770 and 429 us with the arrays, 729, 597 and 273 with
+// the density (4.0 to 4.2 TB/s).
+template <int COEF, int TY>
+struct DensFaces {
+    static constexpr bool DENS = COEF == kCoefDensity;
+    static constexpr int NX = (SW_TX + 1) * TY, NY = SW_TX * (TY + 1), LDS = DENS ? 2 * (NX + NY) : 1;
+    const OuterCoef cf;
+    double *lds;
+    const BlockLevel &g;
+    long long q, qa, qb;  // the own column; the outer face's two cells
+    int i, j, z1, tx, ty, face;
+    bool extra, ex;       // this thread forms an outer face; an east one
+    int ei, ej;
+    double c, t, w, s, a, b, below;
+
+    __device__ __forceinline__ static double form(double h, double own, double before, bool first, bool last, bool wall0,
+                                                  bool wall1) {
+        const double m = last ? before : (first ? own : 0.5 * (own + before));
+        return last ? (wall1 ? 0.0 : h / m) : (first && wall0 ? 0.0 : h / m);
+    }
+    __device__ __forceinline__ DensFaces(const OuterCoef &o, double *l, const BlockLevel &bl, const Tile &tl)
+        : cf(o), lds(l), g(bl), z1(tl.z1), tx(threadIdx.x), ty(threadIdx.y) {
+        if constexpr (DENS) {
+            auto cx = [&](int x) { return x < g.n0 + 1 ? x : g.n0 + 1; };
+            auto cy = [&](int y) { return y < g.n1 + 1 ? y : g.n1 + 1; };
+            i = cx(tl.x0 + tx);
+            j = cy(tl.y0 + ty);
+            q = gidx(g, i, j, 0);
+            ex = ty == 0;
+            extra = ex ? tx < TY : ty == TY - 1;
+            ei = ex ? cx(tl.x0 + SW_TX) : i;
+            ej = ex ? cy(tl.y0 + (tx < TY ? tx : 0)) : cy(tl.y0 + TY);
+            face = ex ? SW_TX + (SW_TX + 1) * (tx < TY ? tx : 0) : NX + SW_TX * TY + tx;
+            qa = gidx(g, ei, ej, 0);
+            qb = qa - (ex ? 1 : g.sy);
+            c = cf.dens[q + g.sz * tl.z0];
+            below = form(g.gz, c, cf.dens[q + g.sz * (tl.z0 - 1)], tl.z0 == 1, false, g.neu & kNeuB, false);
+            load(tl.z0);
+        }
+    }
+    // the densities that plane k's faces take, k = z1 at most
+    __device__ __forceinline__ void load(int k) {
+        if constexpr (DENS) {
+            const long long zo = g.sz * (k < z1 ? k : z1);
+            t = cf.dens[q + zo + g.sz];
+            w = cf.dens[q + zo - 1];
+            s = cf.dens[q + zo - g.sy];
+            if (extra) {
+                a = cf.dens[qa + zo];
+                b = cf.dens[qb + zo];
+            }
+        }
+    }
+    // plane k's x and y faces to LDS
+    __device__ __forceinline__ void store(int k) {
+        if constexpr (DENS) {
+            double *F = lds + (k & 1) * (NX + NY);
+            F[(SW_TX + 1) * ty + tx] = form(g.gx, c, w, i == 1, i == g.n0 + 1, g.neu & kNeuW, g.neu & kNeuE);
+            F[NX + SW_TX * ty + tx] = form(g.gy, c, s, j == 1, j == g.n1 + 1, g.neu & kNeuS, g.neu & kNeuN);
+            if (extra)
+                F[face] = ex ? form(g.gx, a, b, false, ei == g.n0 + 1, false, g.neu & kNeuE)
+                             : form(g.gy, a, b, false, ej == g.n1 + 1, false, g.neu & kNeuN);
+        }
+    }
+    // the top face of plane k, before load() replaces the next plane's density
+    __device__ __forceinline__ double top(int k) {
+        if constexpr (DENS) {
+            const double v = form(g.gz, t, c, false, k == g.n2, false, g.neu & kNeuT);
+            c = t;
+            return v;
+        }
+        return 0.0;
+    }
+    // the coefficients of this thread's cell on plane k, after the barrier
+    __device__ __forceinline__ void get(int x, int y, int k, double at_k, double &aw, double &ae, double &as, double &an,
+                                        double &ab, double &at, double &ap) {
+        if constexpr (DENS) {
+            const double *F = lds + (k & 1) * (NX + NY);
+            aw = F[(SW_TX + 1) * ty + tx];
+            ae = F[(SW_TX + 1) * ty + tx + 1];
+            as = F[NX + SW_TX * ty + tx];
+            an = F[NX + SW_TX * (ty + 1) + tx];
+            ab = below;
+            at = below = at_k;
+            double sum = aw + ae;
+            sum = sum + as;
+            sum = sum + an;
+            sum = sum + ab;
+            sum = sum + at;
+            ap = -sum;
+        } else {
+            coefs<double, COEF == kCoefArrays>(g, cf.x, cf.y, cf.z, gidx(g, x, y, k), x, y, k, aw, ae, as, an, ab, at, ap);
+        }
+    }
+};
+
 // FP64 outer step (newsolv_mg.for:38-54 in Poisson form):
 // p_new = p_old + e over every ghosted cell (both operands carry mapped
 // ghosts, so p_new does too), and on interior cells r = f - A p_new.  r
@@ -21,11 +133,10 @@ namespace mf3d {
 // ADD = false (refined block grids, whose 2:1 ghosts are not the sum of the
 // ghosts of p_old and e): pold already holds p_new with its ghosts; only r
 // and the partials are formed (e and pnew unused).
-template <typename TE, bool VAR, int TY, bool ADD = true>
+template <typename TE, int COEF, int TY, bool ADD = true>
 __global__ __launch_bounds__(SW_TX *TY) void k_outer_lds(
     const double *__restrict__ pold, double *__restrict__ pnew, const TE *__restrict__ e,
-    const double *__restrict__ f, TE *__restrict__ rhs0, const double *__restrict__ cx,
-    const double *__restrict__ cy, const double *__restrict__ cz,
+    const double *__restrict__ f, TE *__restrict__ rhs0, OuterCoef cf,
     const BlockLevel *__restrict__ bls, const Tile *__restrict__ tiles,
     double *__restrict__ partials, const int *__restrict__ done) {
     if (done && *done) return;
@@ -96,6 +207,8 @@ __global__ __launch_bounds__(SW_TX *TY) void k_outer_lds(
         }
     };
     double r2 = 0.0, ra = 0.0;
+    __shared__ double sf[DensFaces<COEF, TY>::LDS];
+    DensFaces<COEF, TY> faces(cf, sf, g, t);
     {
         Regs R;
         load_regs(R, t.z0 - 2);
@@ -106,6 +219,9 @@ __global__ __launch_bounds__(SW_TX *TY) void k_outer_lds(
     auto step = [&](int c, Regs &R) {
         store_plane(c + 1, R.pp, R.pe);
         const double f_cur = R.ff;
+        faces.store(c);
+        const double at_c = faces.top(c);
+        faces.load(c + 1);
         load_regs(R, c + 3);
         __syncthreads();
         if (has_col) {
@@ -115,7 +231,7 @@ __global__ __launch_bounds__(SW_TX *TY) void k_outer_lds(
             const int l = (bx - xb) + LX * (by - yb);
             const long long q = gidx(g, bx, by, c);
             double aw, ae, as, an, ab, at, ap;
-            coefs<double, VAR>(g, cx, cy, cz, q, bx, by, c, aw, ae, as, an, ab, at, ap);
+            faces.get(bx, by, c, at_c, aw, ae, as, an, ab, at, ap);
             double s = aw * P[l - 1];
             s = s + ae * P[l + 1];
             s = s + as * P[l - LX];
@@ -177,12 +293,11 @@ __global__ __launch_bounds__(256) void k_padd(double *__restrict__ pnew, const d
 //   MODE 2:  v = z; partials (A v . w_prev, 0)
 //   MODE 3:  v = p_new as given (a refined grid's, its 2:1 ghosts from the
 //            exchange after k_paxpy); r = f - A v and partials as MODE 0
-template <int MODE, typename TA, typename TR, bool VAR, int TY>
+template <int MODE, typename TA, typename TR, int COEF, int TY>
 __global__ __launch_bounds__(SW_TX *TY) void k_krylov_lds(
     const TA *__restrict__ fa, const double *__restrict__ fb, double *__restrict__ vout,
     const double *__restrict__ f, const double *__restrict__ r64in, double *__restrict__ out64,
-    TR *__restrict__ rhs0, const double *__restrict__ cx, const double *__restrict__ cy,
-    const double *__restrict__ cz, const SolveState *__restrict__ st,
+    TR *__restrict__ rhs0, OuterCoef cf, const SolveState *__restrict__ st,
     const BlockLevel *__restrict__ bls, const Tile *__restrict__ tiles,
     double *__restrict__ partials, const int *__restrict__ done) {
     if (done && *done) return;
@@ -213,30 +328,62 @@ __global__ __launch_bounds__(SW_TX *TY) void k_krylov_lds(
     }
     const int bx = t.x0 + threadIdx.x, by = t.y0 + threadIdx.y;
     const bool has_col = bx <= g.n0 && by <= g.n1;
-    auto plane = [&](int c) {  // form plane c of v in LDS, write owned cells
+    // What the next step consumes is loaded a step ahead: plane c+1 of v's
+    // operands, and plane c of the interior operand and the densities.  The ring has four planes, so a step writing one needs no second
+    // barrier: the slowest wave reads the three before.
+    struct Regs {
+        TA a[KL];
+        double b[KL], x;
+    };
+    constexpr bool SUM = MODE == 0 || MODE == 1;  // v is a sum, written too
+    auto load_v = [&](Regs &R, int c) {
+        const long long zo = g.sz * (long long)(c < t.z1 + 1 ? c : t.z1 + 1);
+#pragma unroll
+        for (int k = 0; k < KL; ++k) {
+            R.a[k] = fa[lsrc[k] + zo];
+            if constexpr (SUM) R.b[k] = fb[lsrc[k] + zo];
+        }
+    };
+    const int cbx = has_col ? bx : 1, cby = has_col ? by : 1;
+    auto load_c = [&](Regs &R, int c) {
+        const long long q = gidx(g, cbx, cby, c < t.z1 ? c : t.z1);
+        R.x = MODE == 1 || MODE == 2 ? r64in[q] : f[q];
+    };
+    auto plane = [&](const Regs &R, int c) {  // form plane c of v in LDS, write owned cells
         double *P = sp[(c + NS) % NS];
         const bool zown = c >= wz0 && c <= wz1;
         const long long zo = g.sz * (long long)c;
 #pragma unroll
         for (int k = 0; k < KL; ++k) {
             if (tid + k * NT >= LXY) continue;
-            double v;
-            if (MODE == 2 || MODE == 3) {
-                const double a = (double)fa[lsrc[k] + zo];
-                v = lok[k] ? a : 0.0;
-            } else {
-                const double a = (double)fa[lsrc[k] + zo], b = fb[lsrc[k] + zo];
-                v = lok[k] ? a + sc * b : 0.0;
-                if (zown && lown[k]) vout[lofs[k] + zo] = v;
-            }
+            const double a = (double)R.a[k];
+            double v = a;
+            if constexpr (SUM) v = a + sc * R.b[k];
+            if (!lok[k]) v = 0.0;
+            if (SUM && zown && lown[k]) vout[lofs[k] + zo] = v;
             P[tid + k * NT] = v;
         }
     };
     double s1 = 0.0, s2 = 0.0;
-    plane(t.z0 - 1);
-    plane(t.z0);
+    __shared__ double sf[DensFaces<COEF, TY>::LDS];
+    Regs R, P0, P1;
+    load_v(P0, t.z0 - 1);
+    load_v(P1, t.z0);
+    load_v(R, t.z0 + 1);
+    load_c(R, t.z0);
+    DensFaces<COEF, TY> faces(cf, sf, g, t);
+    {
+        plane(P0, t.z0 - 1);
+        plane(P1, t.z0);
+    }
     for (int c = t.z0; c <= t.z1; ++c) {
-        plane(c + 1);
+        plane(R, c + 1);
+        const double x = R.x;
+        faces.store(c);
+        const double at_c = faces.top(c);
+        faces.load(c + 1);
+        load_v(R, c + 2);
+        load_c(R, c + 1);
         __syncthreads();
         if (has_col) {
             const double *P = sp[c % NS];
@@ -245,7 +392,7 @@ __global__ __launch_bounds__(SW_TX *TY) void k_krylov_lds(
             const int l = (bx - xb) + LX * (by - yb);
             const long long q = gidx(g, bx, by, c);
             double aw, ae, as, an, ab, at, ap;
-            coefs<double, VAR>(g, cx, cy, cz, q, bx, by, c, aw, ae, as, an, ab, at, ap);
+            faces.get(bx, by, c, at_c, aw, ae, as, an, ab, at, ap);
             double s = aw * P[l - 1];
             s = s + ae * P[l + 1];
             s = s + as * P[l - LX];
@@ -256,18 +403,17 @@ __global__ __launch_bounds__(SW_TX *TY) void k_krylov_lds(
             if (MODE == 1) {
                 out64[q] = s;  // w = A d
                 s1 = s1 + s * s;
-                s2 = s2 + r64in[q] * s;
+                s2 = s2 + x * s;
             } else if (MODE == 2) {
-                s1 = s1 + s * r64in[q];
+                s1 = s1 + s * x;
             } else {
-                const double r = f[q] - s;
+                const double r = x - s;
                 out64[q] = r;
                 rhs0[q] = (TR)r;
                 s1 = s1 + r * r;
                 s2 = fmax(s2, g.lsm ? fabs(r) : fabs(r * g.h0 * g.h1 * g.h2));
             }
         }
-        __syncthreads();
     }
     if (MODE == 0 || MODE == 3)
         block_sum_max<SW_TX * TY>(s1, s2, partials + 2 * (long long)blockIdx.x);
