@@ -23,6 +23,7 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBPS = 8000.0
 W_SEED = 20261202  # the workloads' base seed
+LEGS = os.environ.get("MF3D_LEGS", "1") != "0"  # a lone block's legs as one launch each
 METRIC = "MG solves/s to 1e-8 resid (mixed vs FP64), HBM GB/s % peak, p50/p99 ms"
 
 
@@ -50,13 +51,13 @@ def sweep_bytes_per_launch(w, c=0):
     return (3 * (3 + c) + (2 + c)) / 4.0 * w
 
 
-def leg_bytes_per_launch(w):
-    """Finest-level launches of a lone block's V(2,2) cycle with constant
-    coefficients: the down leg (two sweeps from zero and the restricted
-    residual: RHS read, potential and coarse RHS written) and the up leg
-    (prolongation and two sweeps: RHS, potential and coarse potential read,
-    potential written), 21/8 w per cell on average."""
-    return (2.125 + 3.125) / 2.0 * w
+def leg_bytes_per_launch(w, c=0):
+    """Finest-level launches of a lone block's V(2,2) cycle: the down leg
+    (two sweeps from zero and the restricted residual: RHS read, potential
+    and coarse RHS written) and the up leg (prolongation and two sweeps: RHS,
+    potential and coarse potential read, potential written), each with c
+    coefficient arrays read, (21/8 + c) w per cell on average."""
+    return ((2.125 + 3.125) / 2.0 + c) * w
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_leg_256cubed_L7_traffic.md")
@@ -163,11 +164,11 @@ def rel_l2_mean_removed(a, b):
 def sweep_roofline(r, w, n0, c=0, traffic=None, traffic_source=None, legs=False):
     """Roofline of the finest-level sweep (legs: of the cycle's two legs) from
     the hook's launch times: sweep_bytes_per_launch(w, c) or
-    leg_bytes_per_launch(w) x n0 interior cells per launch."""
+    leg_bytes_per_launch(w, c) x n0 interior cells per launch."""
     if not r["launches"]:
         return None
     avg_s = r["kernel_ms"] / r["launches"] * 1e-3
-    per_launch = (leg_bytes_per_launch(w) if legs else sweep_bytes_per_launch(w, c)) * n0
+    per_launch = (leg_bytes_per_launch(w, c) if legs else sweep_bytes_per_launch(w, c)) * n0
     achieved = per_launch / avg_s / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBPS, 4),
@@ -284,7 +285,7 @@ def run_two_phase(steps, warmup, tol, maxcy, n=384):
                         f"V(2,2) RBGS, {L} levels, to {tol:g} relative residual",
             "cells": n0, "levels": L,
             "fp64": solve_leg(r64, 8, cells, 3, True, sweep_roofline(r64, 8, n0, 3)),
-            "mixed": solve_leg(rmx, 4, cells, 3, True, sweep_roofline(rmx, 4, n0, 3)),
+            "mixed": solve_leg(rmx, 4, cells, 3, True, sweep_roofline(rmx, 4, n0, 3, legs=LEGS)),
             "mixed_rel_l2_vs_fp64": rel_l2_mean_removed(rmx["p"], r64["p"]),
             "speedup_mixed_vs_fp64": round(r64["ms"] / rmx["ms"], 3),
             "coarsest_cells": cells[-1], "direct_coarse": direct, "accuracy": acc,
@@ -553,14 +554,13 @@ def main():
     # Dominant kernel: k_leg, one leg of the V-cycle on the finest level;
     # leg_bytes_per_launch gives its algorithmic bytes.  MF3D_LEGS=0 runs sweeps
     # apart (k_rbs).
-    legs = os.environ.get("MF3D_LEGS", "1") != "0"
     N0 = levels_cells[0]
     src = ("profiles/k_leg_256cubed_L7_traffic.md (rocprofv3 FETCH_SIZE x2 + WRITE_SIZE per launch, "
            "calibrated on a 1 GiB copy)")
 
     def roofline(r, w):
-        traffic = measured_traffic("fp64" if w == 8 else "mixed") if legs and (n, L) == (256, 7) else None
-        return sweep_roofline(r, w, N0, 0, traffic, src, legs)
+        traffic = measured_traffic("fp64" if w == 8 else "mixed") if LEGS and (n, L) == (256, 7) else None
+        return sweep_roofline(r, w, N0, 0, traffic, src, LEGS)
 
     cpu = None
     if not args.no_cpu_baseline:

@@ -84,9 +84,10 @@ struct Level {
     Tile *t_swz = nullptr;
     int n_swz = 0, swz_ty = 4;
     // the level's legs as one launch each (k_leg): tiles, and which legs
-    Tile *t_leg = nullptr;
-    int n_leg = 0, leg_ny = 0;
-    bool leg_down = false, leg_up = false;
+    struct Leg {
+        Tile *t = nullptr;
+        int n = 0, ny = 0;  // workgroups (0: the leg runs as separate kernels), rows of one
+    } legs[2];              // down, up
     Region *r_full = nullptr;
     int n_full = 0, max_full = 0;
     // refined block grids: the level's ghosts as expressions (no regions)
@@ -961,22 +962,24 @@ void prolong_sweep(mf3d_mg *mg, int l, const int *done) {
 
 // The down leg of level l (two sweeps from zero, the residual into level l+1's
 // RHS) or its up leg (prolongation from level l+1, two sweeps).
-template <typename T>
-void leg(mf3d_mg *mg, int l, bool up, const int *done) {
+template <typename T, bool VAR, bool UP>
+void leg(mf3d_mg *mg, int l, const int *done) {
     Level &F = mg->lv[l], &C = mg->lv[l + 1];
+    const Level::Leg &g = F.legs[UP];
     const bool tk = tk_on(mg, MF3D_K_SMOOTH, l);
     const bool yper = !(F.hb[0].neu & (kNeuS | kNeuN));
     const uint32_t bytes = (uint32_t)(F.cells_gh * (long long)sizeof(T));
     const uint32_t cbytes = (uint32_t)(C.cells_gh * (long long)sizeof(T));
+    const LegFaces<T> faces{(const T *)F.cx, (const T *)F.cy, (const T *)F.cz};
     if (tk) tk_mark(mg);
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(F.n_leg), dim3(32 * F.leg_ny), leg_lds<T>(up, yper, F.leg_ny), mg->stream, (const T *)F.phi[F.cur],
-                           (T *)F.phi[1 - F.cur], (const T *)F.rhs, bytes, F.db, F.t_leg, done,
-                           (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db);
+        hipLaunchKernelGGL(kern, dim3(g.n), dim3(32 * g.ny), leg_lds<T>(UP, yper, g.ny, VAR), mg->stream,
+                           (const T *)F.phi[F.cur], (T *)F.phi[1 - F.cur], (const T *)F.rhs, faces, bytes, F.db, g.t,
+                           done, (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db);
     };
-    constexpr int NY = leg_ny<T>();
-    if (F.leg_ny == NY) up ? go(k_leg<T, true, NY>) : go(k_leg<T, false, NY>);
-    else up ? go(k_leg<T, true, LEG_NY_SMALL>) : go(k_leg<T, false, LEG_NY_SMALL>);
+    constexpr int NY = leg_ny<T>(VAR);
+    if (g.ny == NY) go(k_leg<T, UP, NY, VAR>);
+    else go(k_leg<T, UP, LEG_NY_SMALL, VAR>);
     if (tk) tk_mark(mg);
     F.cur = 1 - F.cur;
 }
@@ -990,9 +993,11 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
     }
     // the down leg of level l; true: it restricted into level l+1 too
     auto down = [&](int l, bool zero) {
-        if (zero && mg->lv[l].leg_down) {
-            leg<T>(mg, l, false, done);
-            return true;
+        if constexpr (leg_type<T, VAR>()) {
+            if (zero && mg->lv[l].legs[0].n) {
+                leg<T, VAR, false>(mg, l, done);
+                return true;
+            }
         }
         relax<T, VAR>(mg, l, mg->cfg.nu_pre, zero, done);
         return false;
@@ -1018,8 +1023,12 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
         for (int l = ldown - 1; l >= 0; --l) {
             if (l == L - 1) continue;
             int post = mg->cfg.nu_post;
-            if (mg->lv[l].leg_up) {
-                leg<T>(mg, l, true, done);
+            bool whole = false;
+            if constexpr (leg_type<T, VAR>()) {
+                whole = mg->lv[l].legs[1].n != 0;
+                if (whole) leg<T, VAR, true>(mg, l, done);
+            }
+            if (whole) {
                 post = 0;
             } else if (fused_prolong(mg, l)) {
                 prolong_sweep<T, VAR>(mg, l, done);
@@ -1767,37 +1776,36 @@ std::vector<Tile> leg_tiles(const std::vector<BlockLevel> &hb, int ty, int slots
     return t;
 }
 
-// Which levels run their legs as one launch each: red-black sweeps of lone
-// blocks with constant coefficients, two a leg, every extent even and at
-// least 8 (the ring of a tile then crosses one periodic face at most once a
-// side), above the LDS tail and the coarsest level.
-int leg_setup(mf3d_mg *mg) {
-    const mf3d_mg_cfg &c = mg->cfg;
-    const int L = c.levels;
-    const bool mixed = c.precision == MF3D_MIXED;
-    const bool any_up = c.nu_post == 2, any_down = any_up && c.nu_pre == 2;  // the down leg writes no ghosts: the up leg needs none
-    if (!mg->legs || c.smoother != 3 || c.variable_coef || mg->refined || !any_up) return 0;
+// One leg's kernels may use the LDS they need, and its tiles on level V.
+template <typename T, bool VAR, bool UP>
+int leg_level(mf3d_mg *mg, Level &V, int cus) {
+    constexpr int SM = LEG_NY_SMALL, NY = leg_ny<T>(VAR);
     const hipFuncAttribute attr = hipFuncAttributeMaxDynamicSharedMemorySize;
+    if (hipFuncSetAttribute((const void *)k_leg<T, UP, NY, VAR>, attr, leg_lds<T>(UP, true, NY, VAR)) != hipSuccess ||
+        hipFuncSetAttribute((const void *)k_leg<T, UP, SM, VAR>, attr, leg_lds<T>(UP, true, SM, VAR)) != hipSuccess) {
+        mg->err = "hipFuncSetAttribute (leg LDS) failed";
+        return MF3D_EDEVICE;
+    }
+    // The rows of a workgroup: a step takes 1.2 us with many rows and 0.95 with
+    // few, of which half belong to the ring.  Few on levels that leave compute
+    // units idle (64^3: 13.0 us against 14.7 a leg in FP32, 17.4 against 18.4 in
+    // FP64), many from where all are busy (128^3: 34 against 25).
+    long long many, few;
+    auto t = leg_tiles(V.hb, NY - 8, cus, &many);
+    auto ts = leg_tiles(V.hb, SM - 8, cus, &few);
+    Level::Leg &g = V.legs[UP];
+    g.ny = few * 4 < many * 5 ? SM : NY;
+    t = xcd_order(g.ny == NY ? t : ts);
+    g.n = (int)t.size();
+    return upload(mg, &g.t, t);
+}
+
+template <typename T, bool VAR>
+int leg_levels(mf3d_mg *mg, bool down) {
     int cus = 0;
-    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
-    constexpr int SM = LEG_NY_SMALL, N4 = leg_ny<float>(), N8 = leg_ny<double>();
-    struct {
-        const void *fn;
-        int lds;
-    } ks[] = {{(const void *)k_leg<float, true, N4>, leg_lds<float>(true, true, N4)},
-              {(const void *)k_leg<float, false, N4>, leg_lds<float>(false, true, N4)},
-              {(const void *)k_leg<float, true, SM>, leg_lds<float>(true, true, SM)},
-              {(const void *)k_leg<float, false, SM>, leg_lds<float>(false, true, SM)},
-              {(const void *)k_leg<double, true, N8>, leg_lds<double>(true, true, N8)},
-              {(const void *)k_leg<double, false, N8>, leg_lds<double>(false, true, N8)},
-              {(const void *)k_leg<double, true, SM>, leg_lds<double>(true, true, SM)},
-              {(const void *)k_leg<double, false, SM>, leg_lds<double>(false, true, SM)}};
-    for (const auto &k : ks)
-        if (hipFuncSetAttribute(k.fn, attr, k.lds) != hipSuccess) {
-            mg->err = "hipFuncSetAttribute (leg LDS) failed";
-            return MF3D_EDEVICE;
-        }
-    for (int l = 0; l < std::min(mg->lt, L - 1); ++l) {
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, mg->cfg.device));
+    cus = std::max(1, cus);
+    for (int l = 0; l < std::min(mg->lt, mg->cfg.levels - 1); ++l) {
         Level &V = mg->lv[l];
         bool ok = V.own_ghosts;
         int yper = 0;
@@ -1806,25 +1814,24 @@ int leg_setup(mf3d_mg *mg) {
             yper |= !(g.neu & (kNeuS | kNeuN)) ? 2 : 1;
         }
         if (!ok || yper == 3) continue;  // the LDS layout is one for the launch
-        // The rows of a workgroup: a step takes 1.2 us with many rows and 0.95 with
-        // few, of which half belong to the ring.  Few on levels that leave compute
-        // units idle (64^3: 13.0 us against 14.7 a leg in FP32, 17.4 against 18.4 in
-        // FP64), many from where all are busy (128^3: 34 against 25).
-        long long many, few;
-        auto t = leg_tiles(V.hb, (mixed ? N4 : N8) - 8, std::max(1, cus), &many);
-        auto ts = leg_tiles(V.hb, SM - 8, std::max(1, cus), &few);
-        V.leg_ny = mixed ? N4 : N8;
-        if (few * 4 < many * 5) {
-            V.leg_ny = SM;
-            t = std::move(ts);
-        }
-        t = xcd_order(t);
-        V.n_leg = (int)t.size();
-        if (int rc = upload(mg, &V.t_leg, t)) return rc;
-        V.leg_down = any_down;
-        V.leg_up = any_up;
+        int rc = leg_level<T, VAR, true>(mg, V, cus);
+        if (!rc && down) rc = leg_level<T, VAR, false>(mg, V, cus);
+        if (rc) return rc;
     }
     return 0;
+}
+
+// Which levels run their legs as one launch each: red-black sweeps of lone
+// blocks with constant coefficients, two a leg, every extent even and at
+// least 8 (the ring of a tile then crosses one periodic face at most once a
+// side), above the LDS tail and the coarsest level.
+int leg_setup(mf3d_mg *mg) {
+    const mf3d_mg_cfg &c = mg->cfg;
+    const bool mixed = c.precision == MF3D_MIXED, var = c.variable_coef != 0;
+    const bool any_up = c.nu_post == 2, any_down = any_up && c.nu_pre == 2;  // the down leg writes no ghosts: the up leg needs none
+    if (!mg->legs || c.smoother != 3 || mg->refined || !any_up || (var && !mixed)) return 0;
+    return mixed ? (var ? leg_levels<float, true>(mg, any_down) : leg_levels<float, false>(mg, any_down))
+                 : leg_levels<double, false>(mg, any_down);
 }
 
 int build(mf3d_mg *mg) {

@@ -45,6 +45,13 @@
 // instruction cache, cold in every launch, so rare cases (the planes
 // beside the z faces) take a divisor from LDS instead of code of their own: 64^3
 // FP32 13.0 a leg against 16.3 in two or three launches.
+//
+// Variable coefficients (FP32): a cell's faces and 1 / ap are loaded and formed
+// once, two planes ahead, and stay in registers for its two or three uses;
+// apart, each sweep and the restriction read the three face arrays again.  On
+// 384^3 cells: down 1221 us (420 + 494 + 307) against 396, up 1096 (108 + 2 x
+// 494) against 457, of which the bytes a leg moves, 20.5 and 24.5 a cell, take
+// 235 and 281 at 4.93 TB/s.
 #pragma once
 #include "mg_common.hpp"
 #include "mg_sweep.hpp"
@@ -57,7 +64,11 @@ namespace mf3d {
 // too small to fill the card take LEG_NY_SMALL rows.
 constexpr int LEG_TX = 52, LEG_NY_SMALL = 16;
 template <typename T>
-constexpr int leg_ny() { return sizeof(T) == 4 ? 32 : 24; }
+constexpr int leg_ny(bool var) { return var ? 24 : (sizeof(T) == 4 ? 32 : 24); }
+// Variable coefficients in FP32 only: in FP64 a thread's coefficients of the
+// four planes would not fit in registers.
+template <typename T, bool VAR>
+constexpr bool leg_type() { return sizeof(T) == 4 || !VAR; }
 
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int v) {
@@ -76,7 +87,7 @@ template <typename T> __device__ __forceinline__ T from_right(T v) { return dpp<
 
 // Planes in flight: what the registers leave room for.
 template <typename T, bool UP>
-constexpr int leg_depth() { return sizeof(T) == 8 && UP ? 1 : 3; }
+constexpr int leg_depth(bool var) { return var ? 2 : (sizeof(T) == 8 && UP ? 1 : 3); }
 
 // Two neighbouring entries of a field, at a byte offset of any alignment of
 // one entry.
@@ -107,25 +118,31 @@ __device__ __forceinline__ int leg_map(int v, int n, bool per) {
     return v;
 }
 
+// The face coefficients of a variable-coefficient level (FP32).
+template <typename T> struct LegFaces {
+    const T *__restrict__ x, *__restrict__ y, *__restrict__ z;
+};
+
 // LDS: a thread's divisors on the planes beside the z faces (four), then
 // halves of 32 * (rows + 2) entries: up: the old black, red 1, black 1, red 2
 // planes (two each) and, where y is periodic, the reds they replace; down: red
 // 1, black 1 (two each), red 2 (three), black 2 (two), then the replaced reds.
 template <typename T>
-constexpr int leg_lds(bool up, bool yper, int ny) {
-    return 32 * (int)sizeof(T) * (4 * ny + (ny + 2) * (up ? 8 + (yper ? 4 : 0) : 9 + (yper ? 2 : 0)));
+constexpr int leg_lds(bool up, bool yper, int ny, bool var) {
+    return 32 * (int)sizeof(T) *
+           ((var ? 0 : 4) * ny + (ny + 2) * (up ? 8 + (yper ? 4 : 0) : 9 + (yper ? 2 : 0)));
 }
 
-template <typename T, bool UP, int NY>
+template <typename T, bool UP, int NY, bool VAR = false>
 __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *__restrict__ pout,
-                                                const T *__restrict__ rhs, uint32_t bytes,
+                                                const T *__restrict__ rhs, LegFaces<T> faces, uint32_t bytes,
                                                 const BlockLevel *__restrict__ bls, const Tile *__restrict__ tiles,
                                                 const int *__restrict__ done, const T *__restrict__ phic,
                                                 T *__restrict__ rhsc, uint32_t cbytes,
                                                 const BlockLevel *__restrict__ blc) {
     if (done && *done) return;
     extern __shared__ __align__(16) unsigned char leg_smem[];
-    T *face = reinterpret_cast<T *>(leg_smem), *sm = face + 4 * 32 * NY;
+    T *face = reinterpret_cast<T *>(leg_smem), *sm = face + (VAR ? 0 : 4) * 32 * NY;
     constexpr uint32_t W = sizeof(T);
     constexpr int LEG_NT = 32 * NY, LEG_TY = NY - 8, LEG_ROW = 32 * (NY + 2);
     constexpr int NS = 6;  // planes in the registers' rings, the unroll
@@ -172,17 +189,19 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     // divisors of planes 1 and n2 of the two columns
     auto at_face = [&](int m, bool isA) -> T & { return face[((m == 1 ? 0 : 2) + (isA ? 0 : 1)) * LEG_NT + tid]; };
     const T wallB = g.neu & kNeuB ? T(0) : c2, wallT = g.neu & kNeuT ? T(0) : c2;
-    at_face(1, true) = divisor(sA, wallB, c2);
-    at_face(1, false) = divisor(sB, wallB, c2);
-    at_face(g.n2, true) = divisor(sA, c2, wallT);
-    at_face(g.n2, false) = divisor(sB, c2, wallT);
+    if constexpr (!VAR) {
+        at_face(1, true) = divisor(sA, wallB, c2);
+        at_face(1, false) = divisor(sB, wallB, c2);
+        at_face(g.n2, true) = divisor(sA, c2, wallT);
+        at_face(g.n2, false) = divisor(sB, c2, wallT);
+    }
     // the red value of this column that goes to the lane across a periodic
     // face is the one from before the sweep
     const bool eL = px && ip == 1, eR = px && ip + 1 == g.n0;
     const bool eA = la ? eL : eR, eB = la ? eR : eL;
     // this thread's entry of an LDS half (after a pad row), its y neighbours'
     // (a pad row's zero beyond a wall), and whether one lies across a periodic face
-    const int at0 = 32 * (row + 1) + pair, atS = wS ? pair : at0 - 32, atN = wN ? pair : at0 + 32;
+    const int at0 = 32 * (row + 1) + pair, atS = !VAR && wS ? pair : at0 - 32, atN = !VAR && wN ? pair : at0 + 32;
     const bool ySo = py && jm == 1, yNo = py && jm == g.n1;
 
     auto buf = [&](int b, int slot) { return sm + (2 * b + slot) * LEG_ROW; };
@@ -204,7 +223,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     // 2m + 1 take the coarse planes m and m + 1 (rows jm/2 and jm/2 + 1 of each,
     // e0 and e1; around a periodic axis a ghost plane holds the same values as
     // the plane it wraps to); en: plane m + 2, on its way.
-    constexpr int D = leg_depth<T, UP>();
+    constexpr int D = leg_depth<T, UP>(VAR);
     struct In {
         Pair<T> f, p;
     } L[D];
@@ -212,6 +231,44 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     auto load = [&](In &q, int k) {  // plane k (mapped)
         q.f = bload2<T>(rs_f, vo, (uint32_t)k * pb);
         if constexpr (UP) q.p = bload2<T>(rs_in, vo, (uint32_t)k * pb);
+    };
+    // Variable coefficients: per plane and column the west, east, south, north and
+    // top faces and 1 / ap; the bottom face is the top one of the plane below, but
+    // for plane 1, whose own bottom face a block's edge makes one-sided (zb).
+    const auto rs_x = make_rsrc(faces.x, bytes), rs_y = make_rsrc(faces.y, bytes), rs_z = make_rsrc(faces.z, bytes);
+    constexpr int NV = VAR ? NS : 1, DV = 2;  // DV planes in flight
+    T wwA[NV], eeA[NV], ssA[NV], nnA[NV], ttA[NV], vvA[NV], wwB[NV], eeB[NV], ssB[NV], nnB[NV], ttB[NV], vvB[NV];
+    T zbA = T(0), zbB = T(0);
+    struct Faces {
+        Pair<T> x, s, n, t;
+        T xr;
+    } F[VAR ? DV : 1];
+    auto load_f = [&](Faces &q, int k) {  // plane k (mapped)
+        const uint32_t o = (uint32_t)k * pb;
+        q.x = bload2<T>(rs_x, vo, o);
+        q.xr = bload<T>(rs_x, vo + 2 * W, o);
+        q.s = bload2<T>(rs_y, vo, o);
+        q.n = bload2<T>(rs_y, vo, o + (uint32_t)g.sy * W);
+        q.t = bload2<T>(rs_z, vo, o + pb);
+    };
+    auto take_f = [&](const Faces &q, int m, auto slot, auto below) {  // into the rings; m: the plane it maps to
+        constexpr int S = VAR ? decltype(slot)::value : 0, L = VAR ? decltype(below)::value : 0;
+        wwA[S] = la ? q.x.l : q.x.r;
+        eeA[S] = la ? q.x.r : q.xr;
+        wwB[S] = la ? q.x.r : q.x.l;
+        eeB[S] = la ? q.xr : q.x.r;
+        ssA[S] = la ? q.s.l : q.s.r;
+        ssB[S] = la ? q.s.r : q.s.l;
+        nnA[S] = la ? q.n.l : q.n.r;
+        nnB[S] = la ? q.n.r : q.n.l;
+        const T bA = m == 1 ? zbA : ttA[L], bB = m == 1 ? zbB : ttB[L];
+        ttA[S] = la ? q.t.l : q.t.r;
+        ttB[S] = la ? q.t.r : q.t.l;
+        vvA[S] = T(1) / -(((((wwA[S] + eeA[S]) + ssA[S]) + nnA[S]) + bA) + ttA[S]);
+        vvB[S] = T(1) / -(((((wwB[S] + eeB[S]) + ssB[S]) + nnB[S]) + bB) + ttB[S]);
+        // here and now: moved to where they are used, the divisions would keep
+        // their operands in registers (UP 215 of them instead of 159)
+        asm volatile("" : "+v"(vvA[S]), "+v"(vvB[S]));
     };
     auto load_c = [&](T *e, int m) {  // coarse plane m of the unwrapped planes 2m - 2 .. 2m + 1
         const int nc = g.n2 >> 1, k = pz ? (m < 1 ? m + nc : (m > nc ? m - nc : m)) : (m < 0 ? 0 : (m > nc + 1 ? nc + 1 : m));
@@ -256,6 +313,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
                 a = q.p.r + own_first(before, false) / T(64);
                 b = q.p.l + outer_first(after, false) / T(64);
             }
+            asm volatile("" : "+v"(a), "+v"(b));  // here and now, as in take_f
         }
     };
     auto next = [&](int z, int before) {  // the plane that plane z maps to, after `before`'s
@@ -266,8 +324,18 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     // in FP64 the two products are rounded before they are added and the
     // order is free.  zB, zT: the neighbours below and above; qB, qT: those a
     // black update takes across a periodic face.
-    auto sum = [&](bool isA, T outer, T own, T yS, T yN, T ab, T zB, T at, T zT) -> T {
+    auto sum = [&](auto slot, bool isA, T outer, T own, T yS, T yN, T ab, T zB, T at, T zT) -> T {
         T s;
+        if constexpr (VAR) {
+            constexpr int S = decltype(slot)::value;
+            const bool left = isA ? la : !la;
+            s = (isA ? wwA : wwB)[S] * (left ? outer : own);
+            s = madd(s, (isA ? eeA : eeB)[S], left ? own : outer);
+            s = madd(s, (isA ? ssA : ssB)[S], yS);
+            s = madd(s, (isA ? nnA : nnB)[S], yN);
+            s = madd(s, ab, zB);
+            return madd(s, at, zT);
+        }
         if constexpr (RCP) {
             const bool left = isA ? la : !la;
             s = (isA ? wA : wB) * (left ? outer : own);
@@ -282,19 +350,24 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         s = madd(s, at, zT);
         return s;
     };
-    auto relax = [&](bool isA, T r, T outer, T own, T yS, T yN, int m, T zB, T zT, T qB, T qT) -> T {
+    auto relax = [&](auto slot, auto below, bool isA, T r, T outer, T own, T yS, T yN, int m, T zB, T zT, T qB, T qT) -> T {
         T d = isA ? dA : dB, ab = c2, at = c2;
+        if constexpr (VAR) {
+            d = (isA ? vvA : vvB)[decltype(slot)::value];
+            ab = (isA ? ttA : ttB)[decltype(below)::value];
+            at = (isA ? ttA : ttB)[decltype(slot)::value];
+        }
         if (m == 1 || m == g.n2) {  // uniform, rare
-            d = at_face(m, isA);
+            if constexpr (!VAR) d = at_face(m, isA);
             if (m == 1) {
-                ab = wallB;
+                ab = VAR ? (isA ? zbA : zbB) : wallB;
                 if (pz) zB = qB;
             } else {
-                at = wallT;
+                if constexpr (!VAR) at = wallT;
                 if (pz) zT = qT;
             }
         }
-        const T s = sum(isA, outer, own, yS, yN, ab, zB, at, zT);
+        const T s = sum(slot, isA, outer, own, yS, yN, ab, zB, at, zT);
         return RCP ? (r - s) * d : (r - s) / d;
     };
     const bool xw = sizeof(T) == 8 && !px, xA = xw && (la ? wL : wR), xB = xw && (la ? wR : wL);  // A, B beside a wall
@@ -311,7 +384,23 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
 #pragma unroll
     for (int d = -4; d < 2; ++d) mz[(d + NS) % NS] = leg_map(cm + d, g.n2, pz);
     int kl = mz[1];  // the last plane asked for
+    int kf = mz[0];  // the last plane whose faces were asked for
     {
+        if constexpr (VAR) {
+            const Pair<T> zb = bload2<T>(rs_z, vo, pb), t = bload2<T>(rs_z, vo, (uint32_t)(mz[NS - 1] + 1) * pb);
+            Faces f0;
+            load_f(f0, mz[0]);
+#pragma unroll
+            for (int d = 0; d < DV; ++d) {
+                kf = next(cm + 1 + d, kf);
+                load_f(F[d], kf);
+            }
+            zbA = la ? zb.l : zb.r;
+            zbB = la ? zb.r : zb.l;
+            ttA[NS - 1] = la ? t.l : t.r;
+            ttB[NS - 1] = la ? t.r : t.l;
+            take_f(f0, mz[0], Step<0>{}, Step<NS - 1>{});
+        }
         In q[3];
         if constexpr (UP) {  // planes cm - 1 (odd), cm, cm + 1
             load(q[0], mz[NS - 1]);
@@ -422,12 +511,13 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
             const T v = X[sl(0)];
             o1[sl(0)] = v;
             if (py) buf(O1, PC)[at0] = v;
-            X[sl(0)] = relax(XA, fX[sl(0)], outer_of(XA, Y[sl(0)]), Y[sl(0)], y1S, y1N, mz[sl(0)], X[sl(-1)], X[sl(1)],
+            X[sl(0)] = relax(Step<VAR ? sl(0) : 0>{}, Step<VAR ? sl(-1) : 0>{}, XA, fX[sl(0)], outer_of(XA, Y[sl(0)]), Y[sl(0)], y1S, y1N, mz[sl(0)], X[sl(-1)], X[sl(1)],
                              X[sl(-1)], X[sl(1)]);
         } else {
             const int m = mz[sl(0)];
             T d = XA ? dA : dB;
-            if (m == 1 || m == g.n2) d = at_face(m, XA);
+            if constexpr (VAR) d = (XA ? vvA : vvB)[VAR ? sl(0) : 0];
+            else if (m == 1 || m == g.n2) d = at_face(m, XA);
             X[sl(0)] = RCP ? (fX[sl(0)] - T(0)) * d : (fX[sl(0)] - T(0)) / d;
         }
         buf(R1, PC)[at0] = X[sl(0)];
@@ -435,7 +525,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         // black, sweep 1, plane c-1; across a periodic face the old reds
         {
             const T yv = edge ? o1[sl(-1)] : Y[sl(-1)];
-            X[sl(-1)] = relax(XA, fX[sl(-1)], outer_of(XA, yv), Y[sl(-1)], y2S, y2N, mz[sl(-1)], X[sl(-2)], X[sl(0)],
+            X[sl(-1)] = relax(Step<VAR ? sl(-1) : 0>{}, Step<VAR ? sl(-2) : 0>{}, XA, fX[sl(-1)], outer_of(XA, yv), Y[sl(-1)], y2S, y2N, mz[sl(-1)], X[sl(-2)], X[sl(0)],
                               o1[sl(-2)], o1[sl(0)]);
             buf(B1, 1 - PC)[at0] = X[sl(-1)];
         }
@@ -444,14 +534,14 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
             const T v = X[sl(-2)];
             o2[sl(-2)] = v;
             if (py) old2(PC)[at0] = v;
-            X[sl(-2)] = relax(XA, fX[sl(-2)], outer_of(XA, Y[sl(-2)]), Y[sl(-2)], y3S, y3N, mz[sl(-2)], X[sl(-3)],
+            X[sl(-2)] = relax(Step<VAR ? sl(-2) : 0>{}, Step<VAR ? sl(-3) : 0>{}, XA, fX[sl(-2)], outer_of(XA, Y[sl(-2)]), Y[sl(-2)], y3S, y3N, mz[sl(-2)], X[sl(-3)],
                               X[sl(-1)], X[sl(-3)], X[sl(-1)]);
             red2(PC, (J3 + 2) % 3)[at0] = X[sl(-2)];
         }
         // black, sweep 2, plane c-3
         {
             const T yv = edge ? o2[sl(-3)] : Y[sl(-3)];
-            X[sl(-3)] = relax(XA, fX[sl(-3)], outer_of(XA, yv), Y[sl(-3)], y4S, y4N, mz[sl(-3)], X[sl(-4)], X[sl(-2)],
+            X[sl(-3)] = relax(Step<VAR ? sl(-3) : 0>{}, Step<VAR ? sl(-4) : 0>{}, XA, fX[sl(-3)], outer_of(XA, yv), Y[sl(-3)], y4S, y4N, mz[sl(-3)], X[sl(-4)], X[sl(-2)],
                               o2[sl(-4)], o2[sl(-2)]);
             if constexpr (!UP) buf(B2, 1 - PC)[at0] = X[sl(-3)];
         }
@@ -463,6 +553,21 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
             const T *bb = buf(B2, PC), *br = red2(0, J3);
             auto res = [&](bool isA, T o, T f, T own, T outer, T yS, T yN, T zB, T zT, T self) {
                 // without contraction, as k_restrict: aw*W + ae*E is free of order
+                if constexpr (VAR) {
+                    constexpr int S = VAR ? sl(-4) : 0, L = VAR ? sl(-5) : 0;
+                    const bool left = isA ? la : !la;
+                    const T w = (isA ? wwA : wwB)[S], e = (isA ? eeA : eeB)[S], so = (isA ? ssA : ssB)[S],
+                            no = (isA ? nnA : nnB)[S], b = z == 1 ? (isA ? zbA : zbB) : (isA ? ttA : ttB)[L],
+                            t = (isA ? ttA : ttB)[S];
+                    T v = w * (left ? outer : own);
+                    v = v + e * (left ? own : outer);
+                    v = v + so * yS;
+                    v = v + no * yN;
+                    v = v + b * zB;
+                    v = v + t * zT;
+                    v = v + -(((((w + e) + so) + no) + b) + t) * self;
+                    return f - v;
+                }
                 T s = (RCP ? o : c0) * outer;
                 s = s + c0 * own;
                 s = s + c1 * yS;
@@ -498,6 +603,11 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         take(L[J % D], PC != 0, A[sl(2)], B[sl(2)], fA[sl(2)], fB[sl(2)]);
         kl = next(c + 2 + D, kl);
         load(L[J % D], kl);
+        if constexpr (VAR) {  // the faces of plane c+1
+            take_f(F[J % DV], mz[sl(1)], Step<sl(1)>{}, Step<sl(0)>{});
+            kf = next(c + 1 + DV, kf);
+            load_f(F[J % DV], kf);
+        }
         __syncthreads();
     };
     for (int c = cm; c <= ce; c += NS) {

@@ -1,0 +1,49 @@
+"""The one-launch legs with variable coefficients in the FP32 inner cycle
+against the same cycle with sweeps, restriction and prolongation apart
+(MF3D_LEGS=0), bitwise: extents around the tile (52 x 8 and 52 x 16 cells), the
+smallest extent (8), levels that leave compute units idle and one that does
+not, walls and periodic faces (one-sided at the block's edge) on every axis, both
+coarse operators, defect correction and GCR."""
+import warnings
+
+import numpy as np
+import pytest
+
+from multiflow3d_amd import NotConverged, PressureMultigrid
+from multiflow3d_amd import topology as T
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    ((8, 8, 8), 2, T.CHANNEL_BC),
+    ((16, 8, 24), 2, [5] * 6),
+    ((52, 16, 12), 2, T.CHANNEL_BC),
+    ((56, 24, 8), 3, [5] * 6),
+    ((104, 26, 10), 2, [5, 5, 5, 5, 4, 4]),
+    ((54, 48, 34), 2, [4] * 6),
+    ((40, 20, 96), 3, [4, 4, 5, 5, 5, 5]),
+    ((64, 64, 64), 4, [5, 5, 4, 4, 5, 5]),
+    ((160, 98, 144), 2, [5, 5, 4, 4, 5, 5]),
+]
+
+
+@pytest.mark.parametrize("n,levels,bc", SHAPES)
+@pytest.mark.parametrize("nu,coarse_op,krylov", [((2, 2), "face", True), ((1, 2), "reference", False)])
+def test_density_legs_bitwise(monkeypatch, n, levels, bc, nu, coarse_op, krylov):
+    monkeypatch.setenv("MF3D_TAIL", "0")
+    grid = T.single_block(list(n), [1.0 / 16, 1.0 / 20, 1.0 / 24], bc)
+    rng = np.random.default_rng(43)
+    dens = [np.exp(rng.uniform(0.0, 7.0, n[::-1]))]
+    f = [rng.standard_normal(n[::-1])]
+    print(f"[density legs] {n} {nu} {coarse_op}", flush=True)
+    out = []
+    for legs in "01":
+        monkeypatch.setenv("MF3D_LEGS", legs)
+        with PressureMultigrid(grid, levels, maxcy=3, eps=0.0, precision="mixed", variable_coef=True, nu_pre=nu[0],
+                               nu_post=nu[1], coarse_op=coarse_op, krylov=krylov) as mg:
+            mg.coeff(dens)
+            with warnings.catch_warnings():
+                warnings.simplefilter("ignore", NotConverged)
+                out.append(mg.newsolv_mg(f))
+    (pa, ra), (pl, rl) = out
+    assert np.isfinite(pa[0]).all() and np.array_equal(pa[0], pl[0]) and np.array_equal(ra.hist, rl.hist)
