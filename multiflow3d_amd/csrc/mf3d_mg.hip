@@ -1043,29 +1043,26 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
     relax<T, VAR>(mg, 0, post0, false, done);
 }
 
-// Outer step after the V-cycle of cycle k (from = k mod 2; k = 0: the
-// initial residual, first = true).  Defect correction: p += e, r = f - A p.
+// Outer step after the V-cycle of cycle k (from = k mod 2).  Defect correction: p += e, r = f - A p.
 // GCR(1): beta from (A z, w_prev), d = z - beta d_prev, w = A d, alpha,
 // p += alpha d, r = f - A p.
 template <typename T, int COEF>
-void outer_step_c(mf3d_mg *mg, int from, const int *done, bool first) {
+void outer_step_c(mf3d_mg *mg, int from, const int *done) {
     Level &L0 = mg->lv[0];
     const OuterCoef cf{L0.dcx, L0.dcy, L0.dcz, L0.dens};
     const bool tk = tk_on(mg, MF3D_K_OUTER, 0);
     if (mg->cfg.krylov == MF3D_OUTER_GCR) {
         const T *z = (const T *)L0.phi[L0.cur];
-        if (!first) {
-            hipLaunchKernelGGL((k_krylov_lds<2, T, T, COEF, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, z,
-                               nullptr, nullptr, nullptr, mg->kw, nullptr, nullptr, cf, mg->st, L0.db,
-                               mg->t_out, mg->partials, done);
-            hipLaunchKernelGGL(k_gcr_scalar<true>, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts,
-                               mg->st);
-            hipLaunchKernelGGL((k_krylov_lds<1, T, T, COEF, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, z,
-                               mg->kd[from], mg->kd[1 - from], nullptr, mg->kr, mg->kw, nullptr, cf, mg->st,
-                               L0.db, mg->t_out, mg->partials, done);
-            hipLaunchKernelGGL(k_gcr_scalar<false>, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts,
-                               mg->st);
-        }
+        hipLaunchKernelGGL((k_krylov_lds<2, T, T, COEF, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, z,
+                           nullptr, nullptr, nullptr, mg->kw, nullptr, nullptr, cf, mg->st, L0.db,
+                           mg->t_out, mg->partials, done);
+        hipLaunchKernelGGL(k_gcr_scalar<true>, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts,
+                           mg->st);
+        hipLaunchKernelGGL((k_krylov_lds<1, T, T, COEF, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, z,
+                           mg->kd[from], mg->kd[1 - from], nullptr, mg->kr, mg->kw, nullptr, cf, mg->st,
+                           L0.db, mg->t_out, mg->partials, done);
+        hipLaunchKernelGGL(k_gcr_scalar<false>, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts,
+                           mg->st);
         if (mg->refined) {  // p_new, its exchange (2:1 ghosts), then r = f - A p_new
             const unsigned gb = (unsigned)std::min<long long>(16384, (L0.cells_gh + 255) / 256);
             hipLaunchKernelGGL(k_paxpy, dim3(gb), dim3(256), 0, mg->stream, mg->pbuf[1 - from], mg->pbuf[from],
@@ -1111,11 +1108,11 @@ void outer_step_c(mf3d_mg *mg, int from, const int *done, bool first) {
 }
 
 template <typename T, bool VAR>
-void outer_step(mf3d_mg *mg, int from, const int *done, bool first = false) {
+void outer_step(mf3d_mg *mg, int from, const int *done) {
     if constexpr (VAR)
-        mg->dens_outer ? outer_step_c<T, kCoefDensity>(mg, from, done, first)
-                       : outer_step_c<T, kCoefArrays>(mg, from, done, first);
-    else outer_step_c<T, kCoefConst>(mg, from, done, first);
+        mg->dens_outer ? outer_step_c<T, kCoefDensity>(mg, from, done)
+                       : outer_step_c<T, kCoefArrays>(mg, from, done);
+    else outer_step_c<T, kCoefConst>(mg, from, done);
 }
 
 // Record one cycle reading pbuf[g] into a graph.
@@ -1204,17 +1201,20 @@ int solve_dev(mf3d_mg *mg, const double *f_packed, double *p_packed, double *rma
         }
     mg->last_replay = use_graph || timed;
     hipLaunchKernelGGL(k_reset_state, dim3(1), dim3(1), 0, mg->stream, mg->st, mg->cfg.eps);
-    fill<double>(mg, mg->pbuf[0], L0.cells_gh);
-    fill<T>(mg, (T *)L0.phi[L0.cur], L0.cells_gh);
-    if (mg->cfg.krylov == MF3D_OUTER_GCR) {
-        fill<double>(mg, mg->kd[0], L0.cells_gh);
-        fill<double>(mg, mg->kd[1], L0.cells_gh);
-        fill<double>(mg, mg->kw, L0.cells_gh);
+    // step 0: p_0 = 0 in pbuf[1], r_0 = f; the first cycle's direction before
+    // is multiplied by beta = 0 and must be finite, its w only enters a beta not taken
+    fill<double>(mg, mg->pbuf[1], L0.cells_gh);
+    const bool gcr = mg->cfg.krylov == MF3D_OUTER_GCR;
+    if (gcr) fill<double>(mg, mg->kd[1], L0.cells_gh);
+    {
+        const bool tk = tk_on(mg, MF3D_K_OUTER, 0);
+        if (tk) tk_mark(mg);
+        hipLaunchKernelGGL((k_outer_start<T, 8>), dim3(mg->n_out), dim3(SW_TX, 8), 0, mg->stream, f_packed, mg->f_g,
+                           (T *)L0.rhs, gcr ? mg->kr : nullptr, L0.db, mg->t_out, mg->partials);
+        if (tk) tk_mark(mg);
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, mg->stream, mg->partials, mg->nparts, mg->st,
+                           mg->d_hist, mg->d_rmax, mg->cfg.min_cycles);
     }
-    hipLaunchKernelGGL(k_unpack<double>, dim3(L0.n_in), dim3(kTileX, kTileY), 0, mg->stream, f_packed, mg->f_g,
-                       L0.db, L0.t_in);
-    // step 0: r_0 = f - A*0 from pbuf[0] into pbuf[1]
-    outer_step<T, VAR>(mg, 0, nullptr, true);
     int launched = 0;
     SolveState hs{};
     hs.done = 0;
