@@ -23,7 +23,7 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBPS = 8000.0
 W_SEED = 20261202  # the workloads' base seed
-LEGS = os.environ.get("MF3D_LEGS", "1") != "0"  # a lone block's legs as one launch each
+LEGS = os.environ.get("MF3D_LEGS", "1") != "0"  # each leg of the V-cycle as one launch
 METRIC = "MG solves/s to 1e-8 resid (mixed vs FP64), HBM GB/s % peak, p50/p99 ms"
 
 
@@ -52,7 +52,7 @@ def sweep_bytes_per_launch(w, c=0):
 
 
 def leg_bytes_per_launch(w, c=0):
-    """Finest-level launches of a lone block's V(2,2) cycle: the down leg
+    """Finest-level launches of a V(2,2) cycle run leg by leg: the down leg
     (two sweeps from zero and the restricted residual: RHS read, potential
     and coarse RHS written) and the up leg (prolongation and two sweeps: RHS,
     potential and coarse potential read, potential written), each with c
@@ -249,8 +249,8 @@ def run_uneven(steps, warmup, tol, maxcy):
                         f"periodic x/z, Neumann y, V(2,2) RBGS, {L} levels, to {tol:g} relative residual, "
                         f"ghosts by the on-device region-table exchange",
             "cells": n0, "levels": L, "blocks": [list(b.n) for b in grid.blocks],
-            "fp64": solve_leg(r64, 8, cells, roof=sweep_roofline(r64, 8, n0)),
-            "mixed": solve_leg(rmx, 4, cells, roof=sweep_roofline(rmx, 4, n0)),
+            "fp64": solve_leg(r64, 8, cells, roof=sweep_roofline(r64, 8, n0, legs=LEGS)),
+            "mixed": solve_leg(rmx, 4, cells, roof=sweep_roofline(rmx, 4, n0, legs=LEGS)),
             "mixed_rel_l2_vs_fp64": rel_l2_mean_removed(rmx["p"], r64["p"]),
             "speedup_mixed_vs_fp64": round(r64["ms"] / rmx["ms"], 3),
             "coarsest_cells": cells[-1], "direct_coarse": direct, "accuracy": acc}

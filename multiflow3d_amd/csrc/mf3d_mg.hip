@@ -227,9 +227,10 @@ struct mf3d_mg {
     // the outer passes form level 0's coefficients from the density instead of
     // reading the face arrays, bitwise the same (MF3D_OUTER_DENSITY=1 / 0: always / never)
     bool dens_outer = false;
-    // a lone block's levels run each leg of the cycle in one launch (k_leg);
+    // lone blocks' and block grids' levels run each leg of the cycle in one launch (k_leg);
     // MF3D_LEGS=0 keeps sweeps, restriction and prolongation apart, bitwise the same
     bool legs = true;
+    LegBlocks *d_around = nullptr;  // the blocks around each block (legs of block grids)
     // the velocity form's fields on the caller's ghost shell: G layers
     // (every block's `ghost`), per-block shell geometry, total length
     int G = 1;
@@ -962,26 +963,37 @@ void prolong_sweep(mf3d_mg *mg, int l, const int *done) {
 
 // The down leg of level l (two sweeps from zero, the residual into level l+1's
 // RHS) or its up leg (prolongation from level l+1, two sweeps).
-template <typename T, bool VAR, bool UP>
-void leg(mf3d_mg *mg, int l, const int *done) {
+template <typename T, bool VAR, bool UP, bool MB>
+void leg_launch(mf3d_mg *mg, int l, const int *done) {
     Level &F = mg->lv[l], &C = mg->lv[l + 1];
     const Level::Leg &g = F.legs[UP];
-    const bool tk = tk_on(mg, MF3D_K_SMOOTH, l);
-    const bool yper = !(F.hb[0].neu & (kNeuS | kNeuN));
+    const bool yper = MB || !(F.hb[0].neu & (kNeuS | kNeuN));
     const uint32_t bytes = (uint32_t)(F.cells_gh * (long long)sizeof(T));
     const uint32_t cbytes = (uint32_t)(C.cells_gh * (long long)sizeof(T));
     const LegFaces<T> faces{(const T *)F.cx, (const T *)F.cy, (const T *)F.cz};
-    if (tk) tk_mark(mg);
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(g.n), dim3(32 * g.ny), leg_lds<T>(UP, yper, g.ny, VAR), mg->stream,
                            (const T *)F.phi[F.cur], (T *)F.phi[1 - F.cur], (const T *)F.rhs, faces, bytes, F.db, g.t,
-                           done, (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db);
+                           done, (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db, mg->d_around);
     };
     constexpr int NY = leg_ny<T>(VAR);
-    if (g.ny == NY) go(k_leg<T, UP, NY, VAR>);
-    else go(k_leg<T, UP, LEG_NY_SMALL, VAR>);
+    if (g.ny == NY) go(k_leg<T, UP, NY, VAR, MB>);
+    else go(k_leg<T, UP, LEG_NY_SMALL, VAR, MB>);
+}
+
+template <typename T, bool VAR, bool UP>
+void leg(mf3d_mg *mg, int l, const int *done) {
+    Level &F = mg->lv[l];
+    const bool tk = tk_on(mg, MF3D_K_SMOOTH, l);
+    if (tk) tk_mark(mg);
+    if constexpr (VAR) {
+        leg_launch<T, VAR, UP, false>(mg, l, done);
+    } else {
+        F.own_ghosts ? leg_launch<T, VAR, UP, false>(mg, l, done) : leg_launch<T, VAR, UP, true>(mg, l, done);
+    }
     if (tk) tk_mark(mg);
     F.cur = 1 - F.cur;
+    if (UP) gather<T>(mg, l, done);  // the down leg's ghosts are not read
 }
 
 template <typename T, bool VAR>
@@ -1777,12 +1789,12 @@ std::vector<Tile> leg_tiles(const std::vector<BlockLevel> &hb, int ty, int slots
 }
 
 // One leg's kernels may use the LDS they need, and its tiles on level V.
-template <typename T, bool VAR, bool UP>
+template <typename T, bool VAR, bool UP, bool MB>
 int leg_level(mf3d_mg *mg, Level &V, int cus) {
     constexpr int SM = LEG_NY_SMALL, NY = leg_ny<T>(VAR);
     const hipFuncAttribute attr = hipFuncAttributeMaxDynamicSharedMemorySize;
-    if (hipFuncSetAttribute((const void *)k_leg<T, UP, NY, VAR>, attr, leg_lds<T>(UP, true, NY, VAR)) != hipSuccess ||
-        hipFuncSetAttribute((const void *)k_leg<T, UP, SM, VAR>, attr, leg_lds<T>(UP, true, SM, VAR)) != hipSuccess) {
+    if (hipFuncSetAttribute((const void *)k_leg<T, UP, NY, VAR, MB>, attr, leg_lds<T>(UP, true, NY, VAR)) != hipSuccess ||
+        hipFuncSetAttribute((const void *)k_leg<T, UP, SM, VAR, MB>, attr, leg_lds<T>(UP, true, SM, VAR)) != hipSuccess) {
         mg->err = "hipFuncSetAttribute (leg LDS) failed";
         return MF3D_EDEVICE;
     }
@@ -1800,36 +1812,90 @@ int leg_level(mf3d_mg *mg, Level &V, int cus) {
     return upload(mg, &g.t, t);
 }
 
+// The blocks around each block (LegBlocks), found as build_regions finds a
+// ghost's source.  Empty where the grid is not one that a leg can cross: every
+// face between two blocks whole on both sides, neighbours of neighbours the
+// same by every way, walls that do not end at a face.
+std::vector<LegBlocks> leg_blocks(const std::vector<mf3d_block_desc> &blk) {
+    auto beyond = [&](int b, int f) {  // -1: a wall
+        const mf3d_block_desc &B = blk[b];
+        if (B.nbr[f] >= 0) return B.nbr[f];
+        if (B.bc[f] != 5) return -1;
+        return B.per[f] >= 0 ? B.per[f] : b;
+    };
+    std::vector<LegBlocks> out(blk.size());
+    for (int b = 0; b < (int)blk.size(); ++b) {
+        for (int f = 0; f < 6; ++f) {
+            const int q = beyond(b, f);
+            if (q < 0) continue;
+            if (beyond(q, f ^ 1) != b) return {};
+            for (int e = 0; e < 6; ++e)
+                if (e / 2 != f / 2 && (blk[q].n[e / 2] != blk[b].n[e / 2] || (beyond(q, e) < 0) != (beyond(b, e) < 0)))
+                    return {};
+        }
+        for (int o = 0; o < 27; ++o) {
+            const int off[3] = {o % 3 - 1, o / 3 % 3 - 1, o / 9 - 1};
+            int first = -1;
+            const int ways[6][3] = {{2, 1, 0}, {2, 0, 1}, {1, 2, 0}, {1, 0, 2}, {0, 1, 2}, {0, 2, 1}};
+            for (const auto &w : ways) {
+                int cur = b;
+                for (int d : w) {
+                    const int q = off[d] ? beyond(cur, 2 * d + (off[d] > 0)) : cur;
+                    if (q >= 0) cur = q;
+                }
+                if (first >= 0 && cur != first) return {};
+                first = cur;
+            }
+            out[b].nb[o] = first;
+        }
+    }
+    return out;
+}
+
 template <typename T, bool VAR>
 int leg_levels(mf3d_mg *mg, bool down) {
     int cus = 0;
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, mg->cfg.device));
     cus = std::max(1, cus);
+    const bool grid = mg->d_around != nullptr;
     for (int l = 0; l < std::min(mg->lt, mg->cfg.levels - 1); ++l) {
         Level &V = mg->lv[l];
-        bool ok = V.own_ghosts;
+        bool ok = V.own_ghosts || (grid && !VAR);
         int yper = 0;
         for (const BlockLevel &g : V.hb) {
             ok = ok && g.n0 >= 8 && g.n1 >= 8 && g.n2 >= 8 && !((g.n0 | g.n1 | g.n2) & 1);
+            ok = ok && (V.own_ghosts || (g.c0 == V.hb[0].c0 && g.c1 == V.hb[0].c1 && g.c2 == V.hb[0].c2));
             yper |= !(g.neu & (kNeuS | kNeuN)) ? 2 : 1;
         }
-        if (!ok || yper == 3) continue;  // the LDS layout is one for the launch
-        int rc = leg_level<T, VAR, true>(mg, V, cus);
-        if (!rc && down) rc = leg_level<T, VAR, false>(mg, V, cus);
+        if (!ok || (V.own_ghosts && yper == 3)) continue;  // the LDS layout is one for the launch
+        int rc = 0;
+        if (V.own_ghosts) {
+            rc = leg_level<T, VAR, true, false>(mg, V, cus);
+            if (!rc && down) rc = leg_level<T, VAR, false, false>(mg, V, cus);
+        } else if constexpr (!VAR) {
+            rc = leg_level<T, VAR, true, true>(mg, V, cus);
+            if (!rc && down) rc = leg_level<T, VAR, false, true>(mg, V, cus);
+        }
         if (rc) return rc;
     }
     return 0;
 }
 
-// Which levels run their legs as one launch each: red-black sweeps of lone
-// blocks with constant coefficients, two a leg, every extent even and at
-// least 8 (the ring of a tile then crosses one periodic face at most once a
-// side), above the LDS tail and the coarsest level.
+// Which levels run their legs as one launch each: red-black sweeps, two a leg,
+// of lone blocks (constant coefficients, or variable ones in the FP32 cycle)
+// or of block grids that leg_blocks admits, all of one spacing (constant
+// coefficients), every extent even and at least 8 (the ring of a tile then
+// crosses one face at most a side), above the LDS tail and the coarsest level.
 int leg_setup(mf3d_mg *mg) {
     const mf3d_mg_cfg &c = mg->cfg;
     const bool mixed = c.precision == MF3D_MIXED, var = c.variable_coef != 0;
     const bool any_up = c.nu_post == 2, any_down = any_up && c.nu_pre == 2;  // the down leg writes no ghosts: the up leg needs none
     if (!mg->legs || c.smoother != 3 || mg->refined || !any_up || (var && !mixed)) return 0;
+    if (!var) {
+        const auto around = leg_blocks(mg->blk);
+        if (!around.empty())
+            if (int rc = upload(mg, &mg->d_around, around)) return rc;
+    }
     return mixed ? (var ? leg_levels<float, true>(mg, any_down) : leg_levels<float, false>(mg, any_down))
                  : leg_levels<double, false>(mg, any_down);
 }

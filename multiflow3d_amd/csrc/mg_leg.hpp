@@ -1,5 +1,5 @@
-// mg_leg.hpp -- one leg of the V-cycle on a level of a lone block in one
-// pass over memory: down (two red-black sweeps from zero, the residual and its
+// mg_leg.hpp -- one leg of the V-cycle on a level of a lone block or of a
+// conforming grid of blocks in one pass over memory: down (two red-black sweeps from zero, the residual and its
 // restriction) and up (prolongation and two red-black sweeps).
 //
 // What the sweeps, restriction and prolongation of a leg cost apart is their
@@ -27,7 +27,7 @@
 // Tiles overlap: cells in a ring around the stored ones are computed by the
 // neighbouring workgroups too, from the same inputs, one cell less on
 // every half sweep.  Beyond a periodic face the ring holds the cells it wraps
-// to.  The reference refreshes a block's ghosts only after a whole
+// to, beyond a face to another block (MB) that block's cells.  The reference refreshes a block's ghosts only after a whole
 // sweep (mgsolver.for:610-611), so across such a face a black update reads
 // the red value from before the sweep: updates keep the value they replace
 // (o1, o2), and a neighbour across the face takes that one.  Beyond a wall
@@ -35,9 +35,14 @@
 // Same operands, same order as k_rbs, k_restrict and k_prolong: bitwise
 // their results.
 //
+// A grid of blocks needs the ghosts of its potential only after the up leg, by the
+// exchange; apart, each sweep was followed by one.  Eight blocks of 96 to 192
+// cells a side (26.2 million cells), FP32: down 201 us and two exchanges of 13.5
+// against 107, up 216 and two against 116 and one.
+//
 // Measured on the level of 256^3 cells, sweeps and transfers apart against the
-// leg: FP32 down 125 us (47 + 50 + 28) against 71, up 127 (27 + 2 x 50) against 90;
-// FP64 down 264 against 140, up 310 against 190.  HBM traffic is 1.12 to 1.30
+// leg: FP32 down 125 us (47 + 50 + 28) against 69, up 127 (27 + 2 x 50) against 82;
+// FP64 down 264 against 140, up 310 against 180.  HBM traffic is 1.12 to 1.30
 // times what a leg has to move and takes half the time; the bound is a step's
 // serial chain, 2700 clocks in FP32 for about 120 vector and 80 scalar
 // instructions a wavefront between two barriers, the four updates
@@ -118,6 +123,12 @@ __device__ __forceinline__ int leg_map(int v, int n, bool per) {
     return v;
 }
 
+// The blocks that hold the cells around a block, by offset (ox, oy, oz) at
+// (oz + 1) * 9 + (oy + 1) * 3 + ox + 1; an offset beyond a wall counts as 0.
+struct LegBlocks {
+    int nb[27];
+};
+
 // The face coefficients of a variable-coefficient level (FP32).
 template <typename T> struct LegFaces {
     const T *__restrict__ x, *__restrict__ y, *__restrict__ z;
@@ -133,13 +144,14 @@ constexpr int leg_lds(bool up, bool yper, int ny, bool var) {
            ((var ? 0 : 4) * ny + (ny + 2) * (up ? 8 + (yper ? 4 : 0) : 9 + (yper ? 2 : 0)));
 }
 
-template <typename T, bool UP, int NY, bool VAR = false>
+template <typename T, bool UP, int NY, bool VAR = false, bool MB = false>
 __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *__restrict__ pout,
                                                 const T *__restrict__ rhs, LegFaces<T> faces, uint32_t bytes,
                                                 const BlockLevel *__restrict__ bls, const Tile *__restrict__ tiles,
                                                 const int *__restrict__ done, const T *__restrict__ phic,
                                                 T *__restrict__ rhsc, uint32_t cbytes,
-                                                const BlockLevel *__restrict__ blc) {
+                                                const BlockLevel *__restrict__ blc,
+                                                const LegBlocks *__restrict__ around) {
     if (done && *done) return;
     extern __shared__ __align__(16) unsigned char leg_smem[];
     T *face = reinterpret_cast<T *>(leg_smem), *sm = face + (VAR ? 0 : 4) * 32 * NY;
@@ -157,12 +169,78 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     const int row = UP ? (tid >> 7) * 4 + ((tid >> 6) & 1) + ((tid >> 5) & 1) * 2 : tid >> 5;
     const int pair = (row & 1) ? 31 - (tid & 31) : (tid & 31);
     const int i = t.x0 - 6 + 2 * pair, j = t.y0 - 4 + row;  // i odd: the pair (i, i+1)
-    const bool px = !(g.neu & (kNeuW | kNeuE)), py = !(g.neu & (kNeuS | kNeuN)), pz = !(g.neu & (kNeuB | kNeuT));
-    const int im = leg_map(i, g.n0, px) | 1, jm = leg_map(j, g.n1, py);  // | 1: beyond a wall, the last pair's left
-    const int ip = im > g.n0 ? g.n0 - 1 : im;
-    const uint32_t pb = (uint32_t)g.sz * W, cpb = (uint32_t)gc.sz * W, csy = (uint32_t)gc.sy * W;
-    const uint32_t vo = ((uint32_t)g.off + (uint32_t)(ip + (int)g.sy * jm)) * W;
-    const uint32_t vc = ((uint32_t)gc.off + (uint32_t)(((ip + 1) >> 1) + (int)gc.sy * (jm >> 1))) * W;
+    const bool wallW = g.neu & kNeuW, wallE = g.neu & kNeuE, wallS = g.neu & kNeuS, wallN = g.neu & kNeuN;
+    const bool wallBot = g.neu & kNeuB, wallTop = g.neu & kNeuT;
+    // The block, pair and row this thread's cells are in: the tile's own or,
+    // in the ring beyond a face that is no wall, those there (a lone block's
+    // own again).  Beyond a wall the nearest ones, whose values do not matter.
+    int ip, jm, n0 = g.n0, n1 = g.n1;  // extents of that block
+    uint32_t vo, vc, pb = (uint32_t)g.sz * W, cpb = (uint32_t)gc.sz * W, csy = (uint32_t)gc.sy * W;
+    uint32_t vo_b = 0, vo_t = 0, vc_b = 0, vc_t = 0;  // MB: columns of the blocks below and above
+    int n2b = g.n2;                                   // planes of the block below
+    bool inx = true, iny = true;
+    if constexpr (MB) {
+        const int *nb = around[t.b].nb;
+        const int xk = i < 1 && !wallW ? -1 : (i > g.n0 && !wallE ? 1 : 0);
+        const int yk = j < 1 && !wallS ? -1 : (j > g.n1 && !wallN ? 1 : 0);
+        const int col = 13 + 3 * yk + xk;
+        const BlockLevel &q = bls[nb[col]], &qc = blc[nb[col]];
+        n0 = q.n0;
+        n1 = q.n1;
+        inx = xk == 0;
+        iny = yk == 0;
+        ip = xk < 0 ? n0 + i : (xk > 0 ? i - g.n0 : (i < 1 ? 1 : i));
+        ip = ip > n0 - 1 ? n0 - 1 : ip;  // past what the stored cells need
+        jm = yk < 0 ? n1 + j : (yk > 0 ? j - g.n1 : (j < 1 ? 1 : j));
+        jm = jm > n1 ? n1 : jm;
+        n2b = bls[nb[4]].n2;
+        pb = (uint32_t)q.sz * W;
+        cpb = (uint32_t)qc.sz * W;
+        csy = (uint32_t)qc.sy * W;
+        const int at = ip + (int)q.sy * jm, ac = ((ip + 1) >> 1) + (int)qc.sy * (jm >> 1);
+        vo = ((uint32_t)q.off + (uint32_t)at) * W;
+        vc = ((uint32_t)qc.off + (uint32_t)ac) * W;
+        vo_b = ((uint32_t)bls[nb[col - 9]].off + (uint32_t)at) * W;
+        vo_t = ((uint32_t)bls[nb[col + 9]].off + (uint32_t)at) * W;
+        vc_b = ((uint32_t)blc[nb[col - 9]].off + (uint32_t)ac) * W;
+        vc_t = ((uint32_t)blc[nb[col + 9]].off + (uint32_t)ac) * W;
+    } else {
+        const int im = leg_map(i, g.n0, !wallW) | 1;  // | 1: beyond a wall, the last pair's left
+        ip = im > g.n0 ? g.n0 - 1 : im;
+        jm = leg_map(j, g.n1, !wallS);
+        vo = ((uint32_t)g.off + (uint32_t)(ip + (int)g.sy * jm)) * W;
+        vc = ((uint32_t)gc.off + (uint32_t)(((ip + 1) >> 1) + (int)gc.sy * (jm >> 1))) * W;
+    }
+    // where plane k (of the own block's count, up to 9 beyond it) is
+    struct At {
+        uint32_t v, s;  // byte offsets, a thread's and a scalar
+    };
+    auto plane_at = [&](int k) {
+        if (k < 1 && !wallBot) return MB ? At{vo_b + (uint32_t)(k + n2b) * pb, 0u} : At{vo, (uint32_t)(k + g.n2) * pb};
+        if (k > g.n2 && !wallTop) return MB ? At{vo_t + (uint32_t)(k - g.n2) * pb, 0u} : At{vo, (uint32_t)(k - g.n2) * pb};
+        const uint32_t m = (uint32_t)(k < 1 ? 1 : (k > g.n2 ? g.n2 : k));
+        return MB ? At{vo + m * pb, 0u} : At{vo, m * pb};
+    };
+    // the same from the plane before's, for the loads of the march of a lone
+    // block: from k alone the compiler moves them up, 40 registers in VAR
+    int kl = 0, kf = 0;
+    auto next_at = [&](int k, int &before) {
+        if constexpr (MB) {
+            return plane_at(k);
+        } else {
+            before = wallBot ? (k < 1 ? 1 : (k > g.n2 ? g.n2 : k)) : (before == g.n2 ? 1 : before + 1);
+            return At{vo, (uint32_t)before * pb};
+        }
+    };
+    auto mapped = [&](int k) { return wallBot ? (k < 1 ? 1 : (k > g.n2 ? g.n2 : k)) : (k < 1 ? k + g.n2 : (k > g.n2 ? k - g.n2 : k)); };
+    auto coarse_at = [&](int m) {  // coarse planes 0 and nc + 1 are ghosts
+        const int nc = g.n2 >> 1;
+        if (m < 0 && !wallBot) return MB ? At{vc_b + (uint32_t)(m + (n2b >> 1)) * cpb, 0u} : At{vc, (uint32_t)(m + nc) * cpb};
+        if (m > nc + 1 && !wallTop) return MB ? At{vc_t + (uint32_t)(m - nc) * cpb, 0u} : At{vc, (uint32_t)(m - nc) * cpb};
+        const uint32_t q = (uint32_t)(m < 0 ? 0 : (m > nc + 1 ? nc + 1 : m));
+        return MB ? At{vc + q * cpb, 0u} : At{vc, q * cpb};
+    };
+    const bool py = !(wallS && wallN);
     // Column A (i + j even) is the left one of an odd row's pairs and the right
     // one of an even row's.  Even rows run from right to left, so that A's outer
     // x neighbour is the lane before in both, and B's the one after.
@@ -197,12 +275,12 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     }
     // the red value of this column that goes to the lane across a periodic
     // face is the one from before the sweep
-    const bool eL = px && ip == 1, eR = px && ip + 1 == g.n0;
+    const bool eL = ip == 1 && !(inx && wallW), eR = ip + 1 == n0 && !(inx && wallE);
     const bool eA = la ? eL : eR, eB = la ? eR : eL;
     // this thread's entry of an LDS half (after a pad row), its y neighbours'
     // (a pad row's zero beyond a wall), and whether one lies across a periodic face
     const int at0 = 32 * (row + 1) + pair, atS = !VAR && wS ? pair : at0 - 32, atN = !VAR && wN ? pair : at0 + 32;
-    const bool ySo = py && jm == 1, yNo = py && jm == g.n1;
+    const bool ySo = jm == 1 && !(iny && wallS), yNo = jm == n1 && !(iny && wallN);
 
     auto buf = [&](int b, int slot) { return sm + (2 * b + slot) * LEG_ROW; };
     // buffers: up 0 old black, 1 red 1, 2 black 1, 3 red 2, 4 / 5 the reds that
@@ -228,9 +306,9 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         Pair<T> f, p;
     } L[D];
     T e0[2], e1[2], en[2];
-    auto load = [&](In &q, int k) {  // plane k (mapped)
-        q.f = bload2<T>(rs_f, vo, (uint32_t)k * pb);
-        if constexpr (UP) q.p = bload2<T>(rs_in, vo, (uint32_t)k * pb);
+    auto load = [&](In &q, const At &a) {
+        q.f = bload2<T>(rs_f, a.v, a.s);
+        if constexpr (UP) q.p = bload2<T>(rs_in, a.v, a.s);
     };
     // Variable coefficients: per plane and column the west, east, south, north and
     // top faces and 1 / ap; the bottom face is the top one of the plane below, but
@@ -243,15 +321,15 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         Pair<T> x, s, n, t;
         T xr;
     } F[VAR ? DV : 1];
-    auto load_f = [&](Faces &q, int k) {  // plane k (mapped)
-        const uint32_t o = (uint32_t)k * pb;
+    auto load_f = [&](Faces &q, const At &a) {
+        const uint32_t o = a.s;
         q.x = bload2<T>(rs_x, vo, o);
         q.xr = bload<T>(rs_x, vo + 2 * W, o);
         q.s = bload2<T>(rs_y, vo, o);
         q.n = bload2<T>(rs_y, vo, o + (uint32_t)g.sy * W);
         q.t = bload2<T>(rs_z, vo, o + pb);
     };
-    auto take_f = [&](const Faces &q, int m, auto slot, auto below) {  // into the rings; m: the plane it maps to
+    auto take_f = [&](const Faces &q, int k, auto slot, auto below) {  // plane k into the rings
         constexpr int S = VAR ? decltype(slot)::value : 0, L = VAR ? decltype(below)::value : 0;
         wwA[S] = la ? q.x.l : q.x.r;
         eeA[S] = la ? q.x.r : q.xr;
@@ -261,7 +339,8 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         ssB[S] = la ? q.s.r : q.s.l;
         nnA[S] = la ? q.n.l : q.n.r;
         nnB[S] = la ? q.n.r : q.n.l;
-        const T bA = m == 1 ? zbA : ttA[L], bB = m == 1 ? zbB : ttB[L];
+        const bool first = k == 1 || k == g.n2 + 1;
+        const T bA = first ? zbA : ttA[L], bB = first ? zbB : ttB[L];
         ttA[S] = la ? q.t.l : q.t.r;
         ttB[S] = la ? q.t.r : q.t.l;
         vvA[S] = T(1) / -(((((wwA[S] + eeA[S]) + ssA[S]) + nnA[S]) + bA) + ttA[S]);
@@ -271,9 +350,9 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         asm volatile("" : "+v"(vvA[S]), "+v"(vvB[S]));
     };
     auto load_c = [&](T *e, int m) {  // coarse plane m of the unwrapped planes 2m - 2 .. 2m + 1
-        const int nc = g.n2 >> 1, k = pz ? (m < 1 ? m + nc : (m > nc ? m - nc : m)) : (m < 0 ? 0 : (m > nc + 1 ? nc + 1 : m));
-        e[0] = bload<T>(rs_c, vc, (uint32_t)k * cpb);
-        e[1] = bload<T>(rs_c, vc + csy, (uint32_t)k * cpb);
+        const At a = coarse_at(m);
+        e[0] = bload<T>(rs_c, a.v, a.s);
+        e[1] = MB ? bload<T>(rs_c, a.v + csy, a.s) : bload<T>(rs_c, a.v, a.s + csy);
     };
     // a plane's values, the potential corrected as k_prolong does it
     auto take = [&](const In &q, bool odd, T &a, T &b, T &ra, T &rb) {
@@ -316,10 +395,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
             asm volatile("" : "+v"(a), "+v"(b));  // here and now, as in take_f
         }
     };
-    auto next = [&](int z, int before) {  // the plane that plane z maps to, after `before`'s
-        return pz ? (before == g.n2 ? 1 : before + 1) : (z < 1 ? 1 : (z > g.n2 ? g.n2 : z));
-    };
-    // One update of column A (X_A) or B on a plane mapped to m.  The outer x
+    // One update of column A (X_A) or B on plane k.  The outer x
     // neighbour and the own one are ordered W, E in FP32, whose sum contracts;
     // in FP64 the two products are rounded before they are added and the
     // order is free.  zB, zT: the neighbours below and above; qB, qT: those a
@@ -350,27 +426,37 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         s = madd(s, at, zT);
         return s;
     };
-    auto relax = [&](auto slot, auto below, bool isA, T r, T outer, T own, T yS, T yN, int m, T zB, T zT, T qB, T qT) -> T {
+    auto relax = [&](auto slot, auto below, bool isA, T r, T outer, T own, T yS, T yN, int k, T zB, T zT, T qB, T qT) -> T {
         T d = isA ? dA : dB, ab = c2, at = c2;
         if constexpr (VAR) {
             d = (isA ? vvA : vvB)[decltype(slot)::value];
             ab = (isA ? ttA : ttB)[decltype(below)::value];
             at = (isA ? ttA : ttB)[decltype(slot)::value];
         }
-        if (m == 1 || m == g.n2) {  // uniform, rare
-            if constexpr (!VAR) d = at_face(m, isA);
-            if (m == 1) {
-                ab = VAR ? (isA ? zbA : zbB) : wallB;
-                if (pz) zB = qB;
+        if ((unsigned)k <= 1u || (unsigned)(k - g.n2) <= 1u) {  // beside a z face of a block; uniform, rare
+            if (k == 1 || k == g.n2 + 1) {
+                if constexpr (VAR) ab = isA ? zbA : zbB;
+                if (k == 1 && wallBot) {
+                    if constexpr (!VAR) {
+                        ab = T(0);
+                        d = at_face(1, isA);
+                    }
+                } else {
+                    zB = qB;
+                }
+            } else if (k == g.n2 && wallTop) {
+                if constexpr (!VAR) {
+                    at = T(0);
+                    d = at_face(k, isA);
+                }
             } else {
-                if constexpr (!VAR) at = wallT;
-                if (pz) zT = qT;
+                zT = qT;
             }
         }
         const T s = sum(slot, isA, outer, own, yS, yN, ab, zB, at, zT);
         return RCP ? (r - s) * d : (r - s) / d;
     };
-    const bool xw = sizeof(T) == 8 && !px, xA = xw && (la ? wL : wR), xB = xw && (la ? wR : wL);  // A, B beside a wall
+    const bool xw = sizeof(T) == 8 && (wallW || wallE), xA = xw && (la ? wL : wR), xB = xw && (la ? wR : wL);  // A, B beside a wall
     auto outer_of = [&](bool isA, T v) {
         T o = isA ? from_left(v) : from_right(v);
         if (xw) o = (isA ? xA : xB) ? T(0) : o;  // uniform
@@ -379,42 +465,33 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
 
     const int cm = UP ? t.z0 - 3 : t.z0 - 4, ce = UP ? t.z1 + 3 : t.z1 + 4;  // first and last step
     constexpr int P0 = UP ? 0 : 1;                                           // parity of cm (z0 is odd)
-    // plane cm + d sits in slot d mod NS; mz: the plane each slot's maps to
-    int mz[NS];
-#pragma unroll
-    for (int d = -4; d < 2; ++d) mz[(d + NS) % NS] = leg_map(cm + d, g.n2, pz);
-    int kl = mz[1];  // the last plane asked for
-    int kf = mz[0];  // the last plane whose faces were asked for
+    // plane cm + d sits in slot d mod NS
+    kl = mapped(cm + 1 + D);
+    kf = mapped(cm + DV);
     {
         if constexpr (VAR) {
-            const Pair<T> zb = bload2<T>(rs_z, vo, pb), t = bload2<T>(rs_z, vo, (uint32_t)(mz[NS - 1] + 1) * pb);
+            const Pair<T> zb = bload2<T>(rs_z, vo, pb), t = bload2<T>(rs_z, vo, plane_at(cm - 1).s + pb);
             Faces f0;
-            load_f(f0, mz[0]);
+            load_f(f0, plane_at(cm));
 #pragma unroll
-            for (int d = 0; d < DV; ++d) {
-                kf = next(cm + 1 + d, kf);
-                load_f(F[d], kf);
-            }
+            for (int d = 0; d < DV; ++d) load_f(F[d], plane_at(cm + 1 + d));
             zbA = la ? zb.l : zb.r;
             zbB = la ? zb.r : zb.l;
             ttA[NS - 1] = la ? t.l : t.r;
             ttB[NS - 1] = la ? t.r : t.l;
-            take_f(f0, mz[0], Step<0>{}, Step<NS - 1>{});
+            take_f(f0, cm, Step<0>{}, Step<NS - 1>{});
         }
         In q[3];
         if constexpr (UP) {  // planes cm - 1 (odd), cm, cm + 1
-            load(q[0], mz[NS - 1]);
+            load(q[0], plane_at(cm - 1));
             load_c(e0, (cm - 2) / 2);
             load_c(e1, cm / 2);
             load_c(en, cm / 2 + 1);
         }
-        load(q[1], mz[0]);
-        load(q[2], mz[1]);
+        load(q[1], plane_at(cm));
+        load(q[2], plane_at(cm + 1));
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            kl = next(cm + 2 + d, kl);
-            load(L[d], kl);
-        }
+        for (int d = 0; d < D; ++d) load(L[d], plane_at(cm + 2 + d));
         if constexpr (UP) {
             take(q[0], true, A[NS - 1], B[NS - 1], fA[NS - 1], fB[NS - 1]);
             e0[0] = e1[0];
@@ -434,15 +511,15 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
                                       ghost_image(i + 1, g.n0, g.neu & kNeuW, g.neu & kNeuE) >= 0 ||
                                       ghost_image(j, g.n1, g.neu & kNeuS, g.neu & kNeuN) >= 0));  // in the wavefront
     const int sy = (int)g.sy;
-    const uint32_t ob = (uint32_t)g.off * W;
+    const uint32_t ob = (uint32_t)g.off * W, ob_z = (uint32_t)g.sz * W;
     auto roff = [&](int x, int y) { return ob + (uint32_t)(x + sy * y) * W; };
     const uint32_t vs = roff(i, j);
     auto store = [&](int z, T a, T b) {  // plane z of this thread's stored cells and their ghost images
         if (z < t.z0 || z > t.z1) return;  // uniform
         if (!stored) return;
         const Pair<T> v{la ? a : b, la ? b : a};
-        bstore2<T>(rs_out, v, vs, (uint32_t)z * pb);
-        if (!UP || !(img || z == 1 || z == g.n2)) return;  // uniform; the up leg reads no ghosts of its level
+        bstore2<T>(rs_out, v, vs, (uint32_t)z * ob_z);
+        if (!UP || MB || !(img || z == 1 || z == g.n2)) return;  // uniform; the up leg reads no ghosts of its level
         const int iz = ghost_image(z, g.n2, g.neu & kNeuB, g.neu & kNeuT);
         int x = i, y = j;  // opaque, or the addresses of every image stay in registers
         asm volatile("" : "+v"(x), "+v"(y));
@@ -450,7 +527,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         const int xr = ghost_image(x + 1, g.n0, g.neu & kNeuW, g.neu & kNeuE);
         const int yg = ghost_image(y, g.n1, g.neu & kNeuS, g.neu & kNeuN);
         auto plane = [&](int zz) {
-            const uint32_t s = (uint32_t)zz * pb;
+            const uint32_t s = (uint32_t)zz * ob_z;
             if (zz != z) bstore2<T>(rs_out, v, roff(x, y), s);
             if (yg >= 0) bstore2<T>(rs_out, v, roff(x, yg), s);
             if (xl >= 0) {
@@ -477,7 +554,6 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         T *X = XA ? A : B, *Y = XA ? B : A;
         const T *fX = XA ? fA : fB, *fY = XA ? fB : fA;
         const bool edge = XA ? eB : eA;  // of the sending column, Y
-        mz[sl(2)] = next(c + 2, mz[sl(1)]);
         // the y neighbours of the four updates, written in the step before
         T y1S = T(0), y1N = T(0);
         if constexpr (UP) {
@@ -511,13 +587,12 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
             const T v = X[sl(0)];
             o1[sl(0)] = v;
             if (py) buf(O1, PC)[at0] = v;
-            X[sl(0)] = relax(Step<VAR ? sl(0) : 0>{}, Step<VAR ? sl(-1) : 0>{}, XA, fX[sl(0)], outer_of(XA, Y[sl(0)]), Y[sl(0)], y1S, y1N, mz[sl(0)], X[sl(-1)], X[sl(1)],
+            X[sl(0)] = relax(Step<VAR ? sl(0) : 0>{}, Step<VAR ? sl(-1) : 0>{}, XA, fX[sl(0)], outer_of(XA, Y[sl(0)]), Y[sl(0)], y1S, y1N, c, X[sl(-1)], X[sl(1)],
                              X[sl(-1)], X[sl(1)]);
         } else {
-            const int m = mz[sl(0)];
             T d = XA ? dA : dB;
             if constexpr (VAR) d = (XA ? vvA : vvB)[VAR ? sl(0) : 0];
-            else if (m == 1 || m == g.n2) d = at_face(m, XA);
+            else if ((c == 1 && wallBot) || (c == g.n2 && wallTop)) d = at_face(c, XA);
             X[sl(0)] = RCP ? (fX[sl(0)] - T(0)) * d : (fX[sl(0)] - T(0)) / d;
         }
         buf(R1, PC)[at0] = X[sl(0)];
@@ -525,7 +600,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         // black, sweep 1, plane c-1; across a periodic face the old reds
         {
             const T yv = edge ? o1[sl(-1)] : Y[sl(-1)];
-            X[sl(-1)] = relax(Step<VAR ? sl(-1) : 0>{}, Step<VAR ? sl(-2) : 0>{}, XA, fX[sl(-1)], outer_of(XA, yv), Y[sl(-1)], y2S, y2N, mz[sl(-1)], X[sl(-2)], X[sl(0)],
+            X[sl(-1)] = relax(Step<VAR ? sl(-1) : 0>{}, Step<VAR ? sl(-2) : 0>{}, XA, fX[sl(-1)], outer_of(XA, yv), Y[sl(-1)], y2S, y2N, c - 1, X[sl(-2)], X[sl(0)],
                               o1[sl(-2)], o1[sl(0)]);
             buf(B1, 1 - PC)[at0] = X[sl(-1)];
         }
@@ -534,14 +609,14 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
             const T v = X[sl(-2)];
             o2[sl(-2)] = v;
             if (py) old2(PC)[at0] = v;
-            X[sl(-2)] = relax(Step<VAR ? sl(-2) : 0>{}, Step<VAR ? sl(-3) : 0>{}, XA, fX[sl(-2)], outer_of(XA, Y[sl(-2)]), Y[sl(-2)], y3S, y3N, mz[sl(-2)], X[sl(-3)],
+            X[sl(-2)] = relax(Step<VAR ? sl(-2) : 0>{}, Step<VAR ? sl(-3) : 0>{}, XA, fX[sl(-2)], outer_of(XA, Y[sl(-2)]), Y[sl(-2)], y3S, y3N, c - 2, X[sl(-3)],
                               X[sl(-1)], X[sl(-3)], X[sl(-1)]);
             red2(PC, (J3 + 2) % 3)[at0] = X[sl(-2)];
         }
         // black, sweep 2, plane c-3
         {
             const T yv = edge ? o2[sl(-3)] : Y[sl(-3)];
-            X[sl(-3)] = relax(Step<VAR ? sl(-3) : 0>{}, Step<VAR ? sl(-4) : 0>{}, XA, fX[sl(-3)], outer_of(XA, yv), Y[sl(-3)], y4S, y4N, mz[sl(-3)], X[sl(-4)], X[sl(-2)],
+            X[sl(-3)] = relax(Step<VAR ? sl(-3) : 0>{}, Step<VAR ? sl(-4) : 0>{}, XA, fX[sl(-3)], outer_of(XA, yv), Y[sl(-3)], y4S, y4N, c - 3, X[sl(-4)], X[sl(-2)],
                               o2[sl(-4)], o2[sl(-2)]);
             if constexpr (!UP) buf(B2, 1 - PC)[at0] = X[sl(-3)];
         }
@@ -591,7 +666,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
             acc = acc + rb;
             acc = acc + ul;
             acc = acc + ur;
-            if (!PC && z >= t.z0 && z <= t.z1 && stored && !(row & 1)) bstore<T>(rs_c, T(0.125) * acc, vcs, (uint32_t)(z >> 1) * cpb);
+            if (!PC && z >= t.z0 && z <= t.z1 && stored && !(row & 1)) bstore<T>(rs_c, T(0.125) * acc, vcs, (uint32_t)(z >> 1) * (uint32_t)(gc.sz * W));
         }
         if constexpr (UP && PC == 0) {  // plane c+2 is even: the next two coarse planes
             e0[0] = e1[0];
@@ -601,12 +676,10 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
             load_c(en, (c + 2) / 2 + 2);
         }
         take(L[J % D], PC != 0, A[sl(2)], B[sl(2)], fA[sl(2)], fB[sl(2)]);
-        kl = next(c + 2 + D, kl);
-        load(L[J % D], kl);
+        load(L[J % D], next_at(c + 2 + D, kl));
         if constexpr (VAR) {  // the faces of plane c+1
-            take_f(F[J % DV], mz[sl(1)], Step<sl(1)>{}, Step<sl(0)>{});
-            kf = next(c + 1 + DV, kf);
-            load_f(F[J % DV], kf);
+            take_f(F[J % DV], c + 1, Step<sl(1)>{}, Step<sl(0)>{});
+            load_f(F[J % DV], next_at(c + 1 + DV, kf));
         }
         __syncthreads();
     };
