@@ -19,7 +19,10 @@
 // chunk return at once.  The host synchronises once per chunk.
 #include <hip/hip_runtime.h>
 
+#include <sched.h>
+
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -28,6 +31,8 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -132,6 +137,8 @@ struct mf3d_mg {
     double *d_hist = nullptr, *d_rmax = nullptr;
     double *d_io = nullptr;  // device staging for host transfers (packed)
     double *h_io = nullptr;  // pinned host staging
+    double *h_io2 = nullptr;  // a second one, for fields copied one after another (host_fields)
+    hipEvent_t io_ev[2] = {};
     long long io_len = 0;
     long long cells = 0;
     long long bytes = 0;
@@ -1324,6 +1331,138 @@ template <typename TD, typename TS>
 void convert(mf3d_mg *mg, TD *dst, const TS *src, long long n) {
     const unsigned gb = (unsigned)std::min<long long>((n + 255) / 256, 16384);
     hipLaunchKernelGGL((k_convert<TD, TS>), dim3(gb), dim3(256), 0, mg->stream, dst, src, n);
+}
+
+// Planes k0 .. k1-1 of one block's packed box of `ring` layers, at o in the vector.
+struct HostPiece {
+    int b, k0, k1;
+    long long o;
+};
+
+// One piece between a caller's block array and the packed vector, in one copy
+// where its rows and planes follow each other in both.
+void copy_piece(const mf3d_mg *mg, const HostPiece &q, double *caller, double *packed, int ring, bool in) {
+    const mf3d_block_desc &B = mg->blk[q.b];
+    const int ld0 = B.ld[0] ? B.ld[0] : B.n[0] + 2 * B.ghost, ld1 = B.ld[1] ? B.ld[1] : B.n[1] + 2 * B.ghost;
+    const int e0 = B.n[0] + 2 * ring, e1 = B.n[1] + 2 * ring, s = B.ghost - ring;
+    double *p = packed + q.o;
+    auto copy = [&](double *c, size_t n) {
+        std::memcpy(in ? p : c, in ? c : p, sizeof(double) * n);
+        p += n;
+    };
+    for (int k = q.k0; k < q.k1; ++k) {
+        double *plane = caller + (size_t)s + (size_t)ld0 * ((size_t)s + (size_t)ld1 * (k + s));
+        if (e0 == ld0) copy(plane, (size_t)e0 * e1);
+        else
+            for (int j = 0; j < e1; ++j) copy(plane + (size_t)ld0 * j, e0);
+    }
+}
+
+// nf fields (a caller's block arrays each) to the device (in) or back, with
+// `ring` ghost layers.  The packing is memory-bound on one core (9 GB/s) where
+// the link takes 55: threads of this call pack pieces of 256 KiB in order, and
+// field f travels from one of two pinned buffers while f + 1 is packed into the
+// other.  A velocity step of two cycles on eight blocks of 32^3, 48^3 and 64^3
+// cells, 7 fields in and 4 out: 1.9, 7.0 and 15.0 ms with one thread, 1.4, 2.9
+// and 5.7 with up to eight.  A thread for every 4 MiB from 12 MiB (at 24^3, 10
+// MiB, two threads gain nothing: 1.10 against 1.13 ms); hosts that refuse
+// threads or memory take one buffer and the calling thread.
+int host_fields(mf3d_mg *mg, bool in, double *const *const *caller, double *const *dev, int nf, int ring) {
+    std::vector<HostPiece> pieces;
+    long long o = 0;
+    for (int b = 0; b < mg->cfg.nblocks; ++b) {
+        const mf3d_block_desc &B = mg->blk[b];
+        const long long plane = (long long)(B.n[0] + 2 * ring) * (B.n[1] + 2 * ring);
+        const int n2 = B.n[2] + 2 * ring, step = (int)std::max(1LL, 32768 / plane);
+        for (int k = 0; k < n2; k += step) {
+            pieces.push_back(HostPiece{b, k, std::min(n2, k + step), o});
+            o += plane * (pieces.back().k1 - k);
+        }
+    }
+    const size_t bytes = sizeof(double) * (size_t)o;
+    const int np = (int)pieces.size();
+    cpu_set_t set;
+    const int cpus = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
+    int nt = (int)std::min<size_t>({8, (size_t)std::max(0, cpus - 1), bytes * nf >> 22});
+    if (nt < 3) nt = 0;
+    if (nt >= 2 && !mg->h_io2) {
+        if (hipHostMalloc((void **)&mg->h_io2, sizeof(double) * mg->io_len, hipHostMallocDefault) != hipSuccess) {
+            mg->h_io2 = nullptr;
+            (void)hipGetLastError();
+        }
+    }
+    for (hipEvent_t &e : mg->io_ev)
+        if (nt >= 2 && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            e = nullptr;
+            (void)hipGetLastError();
+        }
+    if (!mg->h_io2 || !mg->io_ev[0] || !mg->io_ev[1]) nt = 0;
+    double *buf[2] = {mg->h_io, mg->h_io2};
+    std::atomic<int> next{0}, open{in ? 2 : 0};  // fields whose buffer the threads may use
+    std::atomic<bool> stop{false};
+    std::vector<std::atomic<int>> packed(nf);
+    for (auto &a : packed) a = 0;
+    auto work = [&] {
+        for (;;) {
+            const int c = next.fetch_add(1);
+            if (c >= nf * np) return;
+            const int f = c / np;
+            while (open.load(std::memory_order_acquire) <= f) {
+                if (stop.load()) return;
+                std::this_thread::yield();
+            }
+            const HostPiece &q = pieces[c % np];
+            copy_piece(mg, q, caller[f][q.b], buf[f & 1], ring, in);
+            packed[f].fetch_add(1, std::memory_order_release);
+        }
+    };
+    std::vector<std::thread> threads;
+    try {
+        threads.reserve(nt);
+        for (int t = 0; t < nt; ++t) threads.emplace_back(work);
+    } catch (const std::system_error &) {  // what runs already does the work
+    }
+    if (threads.empty()) {
+        for (int f = 0; f < nf; ++f) {
+            auto copy = [&] { for (const HostPiece &q : pieces) copy_piece(mg, q, caller[f][q.b], mg->h_io, ring, in); };
+            if (in) copy();
+            HIPCHK(in ? hipMemcpyAsync(dev[f], mg->h_io, bytes, hipMemcpyHostToDevice, mg->stream)
+                      : hipMemcpyAsync(mg->h_io, dev[f], bytes, hipMemcpyDeviceToHost, mg->stream));
+            HIPCHK(hipStreamSynchronize(mg->stream));
+            if (!in) copy();
+        }
+        return 0;
+    }
+    auto travel = [&](int f) {
+        hipError_t e = in ? hipMemcpyAsync(dev[f], buf[f & 1], bytes, hipMemcpyHostToDevice, mg->stream)
+                          : hipMemcpyAsync(buf[f & 1], dev[f], bytes, hipMemcpyDeviceToHost, mg->stream);
+        return e == hipSuccess ? hipEventRecord(mg->io_ev[f & 1], mg->stream) : e;
+    };
+    auto wait_packed = [&](int f) {
+        while (packed[f].load(std::memory_order_acquire) < np) std::this_thread::yield();
+    };
+    hipError_t e = hipSuccess;
+    for (int f = 0; !in && f < 2 && f < nf && e == hipSuccess; ++f) e = travel(f);
+    for (int f = 0; f < nf && e == hipSuccess; ++f) {
+        if (in) {
+            wait_packed(f);
+            e = travel(f);
+            if (f + 2 >= nf) continue;
+        }
+        if (e == hipSuccess) e = hipEventSynchronize(mg->io_ev[f & 1]);  // field f has travelled
+        if (e != hipSuccess) break;
+        open.store(in ? f + 3 : f + 1, std::memory_order_release);
+        if (!in) {
+            wait_packed(f);
+            if (f + 2 < nf) e = travel(f + 2);
+        }
+    }
+    stop = true;
+    for (std::thread &t : threads) t.join();
+    const hipError_t last = hipStreamSynchronize(mg->stream);  // the buffers are free again
+    HIPCHK(e);
+    HIPCHK(last);
+    return 0;
 }
 
 // mgkcyc: the caller's pp (one ghost layer, same shape as the level-0 arena)
@@ -3056,22 +3195,15 @@ int mf3d_mg_newsolv(mf3d_mg *mg, const double *const *ustar, const double *const
     const size_t bytes = sizeof(double) * (size_t)mg->cells_w;
     for (int i = 0; i < 8; ++i)
         if (!mg->vf[i] && (i < 7 || su) && (rc = dev_alloc(mg, (void **)&mg->vf[i], bytes))) return rc;
-    const double *const *in[7] = {ustar, vstar, wstar, u, v, w, p};
-    for (int i = 0; i < 7; ++i) {
-        host_to_packed(mg, in[i], mg->h_io, G);
-        HIPCHK(hipMemcpyAsync(mg->vf[i], mg->h_io, bytes, hipMemcpyHostToDevice, mg->stream));
-        HIPCHK(hipStreamSynchronize(mg->stream));
-    }
+    double *const *in[7] = {const_cast<double *const *>(ustar), const_cast<double *const *>(vstar),
+                            const_cast<double *const *>(wstar), u, v, w, p};
+    if ((rc = host_fields(mg, true, in, mg->vf, 7, G))) return rc;
     const VelFields F{mg->vf[0], mg->vf[1], mg->vf[2], mg->vf[3], mg->vf[4], mg->vf[5], mg->vf[6],
                       mg->cfg.variable_coef ? L0.dens : nullptr};
     rc = newsolv_any(mg, F, dt, alfapr, eps, su ? mg->vf[7] : nullptr, rmax_out, iters_out, rmax_hist);
     if (rc < 0) return rc;
     double *const *out[4] = {u, v, w, p};
-    for (int i = 0; i < 4; ++i) {
-        HIPCHK(hipMemcpyAsync(mg->h_io, mg->vf[3 + i], bytes, hipMemcpyDeviceToHost, mg->stream));
-        HIPCHK(hipStreamSynchronize(mg->stream));
-        packed_to_host(mg, mg->h_io, out[i], G);
-    }
+    if (const int e = host_fields(mg, false, out, mg->vf + 3, 4, G)) return e;
     if (su) {
         hipLaunchKernelGGL(k_pack<double>, dim3(L0.n_in), dim3(kTileX, kTileY), 0, mg->stream, mg->vf[7], mg->d_io,
                            mg->d_vw, L0.t_in);
@@ -3156,6 +3288,9 @@ void mf3d_mg_destroy(mf3d_mg *mg) {
     drop_graphs(mg);
     for (void *p : mg->allocs) (void)hipFree(p);
     if (mg->h_io) (void)hipHostFree(mg->h_io);
+    if (mg->h_io2) (void)hipHostFree(mg->h_io2);
+    for (hipEvent_t e : mg->io_ev)
+        if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : mg->ev_eager.ev) (void)hipEventDestroy(e);
     if (mg->stream) (void)hipStreamDestroy(mg->stream);
     delete mg;
