@@ -91,7 +91,7 @@ struct Level {
     // the level's legs as one launch each (k_leg): tiles, and which legs
     struct Leg {
         Tile *t = nullptr;
-        int n = 0, ny = 0;  // workgroups (0: the leg runs as separate kernels), rows of one
+        int n = 0, ny = 0;  // workgroups (0: the leg runs as separate kernels), rows of one (0: boxes, k_leg3)
     } legs[2];              // down, up
     Region *r_full = nullptr;
     int n_full = 0, max_full = 0;
@@ -984,6 +984,14 @@ void leg_launch(mf3d_mg *mg, int l, const int *done) {
                            done, (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db, mg->d_around);
     };
     constexpr int NY = leg_ny<T>(VAR);
+    if constexpr (!MB) {
+        if (!g.ny) {
+            hipLaunchKernelGGL((k_leg3<T, UP, VAR>), dim3(g.n), dim3(L3_NT), leg3_lds<T>(), mg->stream,
+                               (const T *)F.phi[F.cur], (T *)F.phi[1 - F.cur], (const T *)F.rhs, faces, bytes, F.db, g.t,
+                               done, (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db);
+            return;
+        }
+    }
     if (g.ny == NY) go(k_leg<T, UP, NY, VAR, MB>);
     else go(k_leg<T, UP, LEG_NY_SMALL, VAR, MB>);
 }
@@ -1931,24 +1939,46 @@ std::vector<Tile> leg_tiles(const std::vector<BlockLevel> &hb, int ty, int slots
 template <typename T, bool VAR, bool UP, bool MB>
 int leg_level(mf3d_mg *mg, Level &V, int cus) {
     constexpr int SM = LEG_NY_SMALL, NY = leg_ny<T>(VAR);
-    const hipFuncAttribute attr = hipFuncAttributeMaxDynamicSharedMemorySize;
-    if (hipFuncSetAttribute((const void *)k_leg<T, UP, NY, VAR, MB>, attr, leg_lds<T>(UP, true, NY, VAR)) != hipSuccess ||
-        hipFuncSetAttribute((const void *)k_leg<T, UP, SM, VAR, MB>, attr, leg_lds<T>(UP, true, SM, VAR)) != hipSuccess) {
-        mg->err = "hipFuncSetAttribute (leg LDS) failed";
-        return MF3D_EDEVICE;
-    }
+    Level::Leg &g = V.legs[UP];
+    // the kernel's LDS; tiles, or the other leg's where they are the same
+    auto take = [&](const void *kernel, int lds, int ny, std::vector<Tile> t) {
+        if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) {
+            mg->err = "hipFuncSetAttribute (leg LDS) failed";
+            return (int)MF3D_EDEVICE;
+        }
+        g.ny = ny;
+        g.n = (int)t.size();
+        const Level::Leg &other = V.legs[!UP];
+        if (other.n && other.ny == ny) {
+            g.t = other.t;
+            return 0;
+        }
+        return upload(mg, &g.t, xcd_order(std::move(t)));
+    };
     // The rows of a workgroup: a step takes 1.2 us with many rows and 0.95 with
     // few, of which half belong to the ring.  Few on levels that leave compute
     // units idle (64^3: 13.0 us against 14.7 a leg in FP32, 17.4 against 18.4 in
     // FP64), many from where all are busy (128^3: 34 against 25).
+    if constexpr (!MB) {
+        std::vector<Tile> box;
+        for (int b = 0; b < (int)V.hb.size(); ++b)
+            for (int z = 1; z <= V.hb[b].n2; z += L3_TILE)
+                for (int y = 1; y <= V.hb[b].n1; y += L3_TILE)
+                    for (int x = 1; x <= V.hb[b].n0; x += L3_TILE) box.push_back(Tile{b, x, y, z, z + L3_TILE - 1});
+        // Boxes while they do not fill the card: two a compute unit, the FP64 up leg one
+        // (us a leg, march / boxes; down, up.  FP64 32^3 13.0 / 6.7, 13.4 / 9.3; 48^3
+        // 14.2 / 7.6, 13.8 / 10.0; 64^3 17.0 / 13.6, 16.4 / 17.6; FP32 32^3 9.1 / 5.6,
+        // 10.8 / 7.3; 64^3 11.4 / 8.5, 12.2 / 10.7; 80^3 14.9 / 13.7, 16.6 / 17.6; 96^3
+        // 15.2 / 22.3, 17.3 / 29.4).
+        if ((int)box.size() <= (sizeof(T) == 8 && UP ? 1 : 2) * cus)
+            return take((const void *)k_leg3<T, UP, VAR>, leg3_lds<T>(), 0, std::move(box));
+    }
     long long many, few;
     auto t = leg_tiles(V.hb, NY - 8, cus, &many);
     auto ts = leg_tiles(V.hb, SM - 8, cus, &few);
-    Level::Leg &g = V.legs[UP];
-    g.ny = few * 4 < many * 5 ? SM : NY;
-    t = xcd_order(g.ny == NY ? t : ts);
-    g.n = (int)t.size();
-    return upload(mg, &g.t, t);
+    if (few * 4 < many * 5)
+        return take((const void *)k_leg<T, UP, SM, VAR, MB>, leg_lds<T>(UP, true, SM, VAR), SM, std::move(ts));
+    return take((const void *)k_leg<T, UP, NY, VAR, MB>, leg_lds<T>(UP, true, NY, VAR), NY, std::move(t));
 }
 
 // The blocks around each block (LegBlocks), found as build_regions finds a

@@ -152,7 +152,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
                                                 T *__restrict__ rhsc, uint32_t cbytes,
                                                 const BlockLevel *__restrict__ blc,
                                                 const LegBlocks *__restrict__ around) {
-    if (done && *done) return;
+    const int stop = done ? *done : 0;  // awaited with the tile
     extern __shared__ __align__(16) unsigned char leg_smem[];
     T *face = reinterpret_cast<T *>(leg_smem), *sm = face + (VAR ? 0 : 4) * 32 * NY;
     constexpr uint32_t W = sizeof(T);
@@ -160,6 +160,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     constexpr int NS = 6;  // planes in the registers' rings, the unroll
     const Tile t = tiles[blockIdx.x];
     const BlockLevel g = bls[t.b], gc = blc[t.b];
+    if (stop) return;
     const auto rs_in = make_rsrc(pin, bytes), rs_f = make_rsrc(rhs, bytes), rs_out = make_rsrc(pout, bytes);
     const auto rs_c = make_rsrc(UP ? phic : rhsc, cbytes);
     // A wavefront takes two rows: down, whose restriction adds them, an odd row
@@ -289,10 +290,6 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     constexpr int R1 = UP ? 1 : 0, B1 = UP ? 2 : 1, B2 = 2, O1 = 4, O2 = UP ? 5 : 4;
     auto red2 = [&](int slot2, int slot3) { return UP ? buf(3, slot2) : sm + (6 + slot3) * LEG_ROW; };
     auto old2 = [&](int slot2) { return UP ? buf(O2, slot2) : sm + (9 + slot2) * LEG_ROW; };
-    for (int e = tid; e < LEG_ROW * (UP ? 8 + (py ? 4 : 0) : 9 + (py ? 2 : 0)); e += LEG_NT)
-        sm[e] = T(0);  // the pad rows stay zero; the first steps read the rest before it is written
-    __syncthreads();
-
     T A[NS], B[NS], fA[NS], fB[NS], o1[NS], o2[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) A[s] = B[s] = fA[s] = fB[s] = o1[s] = o2[s] = T(0);
@@ -469,17 +466,14 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     kl = mapped(cm + 1 + D);
     kf = mapped(cm + DV);
     {
+        Pair<T> zb, top;
+        Faces f0;
         if constexpr (VAR) {
-            const Pair<T> zb = bload2<T>(rs_z, vo, pb), t = bload2<T>(rs_z, vo, plane_at(cm - 1).s + pb);
-            Faces f0;
+            zb = bload2<T>(rs_z, vo, pb);
+            top = bload2<T>(rs_z, vo, plane_at(cm - 1).s + pb);
             load_f(f0, plane_at(cm));
 #pragma unroll
             for (int d = 0; d < DV; ++d) load_f(F[d], plane_at(cm + 1 + d));
-            zbA = la ? zb.l : zb.r;
-            zbB = la ? zb.r : zb.l;
-            ttA[NS - 1] = la ? t.l : t.r;
-            ttB[NS - 1] = la ? t.r : t.l;
-            take_f(f0, cm, Step<0>{}, Step<NS - 1>{});
         }
         In q[3];
         if constexpr (UP) {  // planes cm - 1 (odd), cm, cm + 1
@@ -492,6 +486,16 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         load(q[2], plane_at(cm + 1));
 #pragma unroll
         for (int d = 0; d < D; ++d) load(L[d], plane_at(cm + 2 + d));
+        // while they travel; the pad rows stay zero, the first steps read the rest before it is written
+        for (int e = tid; e < LEG_ROW * (UP ? 8 + (py ? 4 : 0) : 9 + (py ? 2 : 0)); e += LEG_NT) sm[e] = T(0);
+        __syncthreads();
+        if constexpr (VAR) {
+            zbA = la ? zb.l : zb.r;
+            zbB = la ? zb.r : zb.l;
+            ttA[NS - 1] = la ? top.l : top.r;
+            ttB[NS - 1] = la ? top.r : top.l;
+            take_f(f0, cm, Step<0>{}, Step<NS - 1>{});
+        }
         if constexpr (UP) {
             take(q[0], true, A[NS - 1], B[NS - 1], fA[NS - 1], fB[NS - 1]);
             e0[0] = e1[0];
@@ -695,6 +699,267 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
         step(c + 4, Step<4>{});
         if (c + 5 > ce) break;
         step(c + 5, Step<5>{});
+    }
+}
+
+// The same leg on a small level of a lone block, a box at a time: a workgroup takes
+// 8 x 8 x 8 cells with a ring of 4 (16^3 cells) into LDS and does the four half
+// sweeps there, one barrier each, where the march above takes a step of about
+// 1 us for each of at least ten planes.  The ring makes it eight times the
+// cells of the box, so it pays only while the level does not fill the card
+// (32^3 FP64: 6.7 us down and 9.3 up where the march takes 13.0 and 13.4; both
+// sides by size stand at the rule in leg_level).  One workgroup of 1024 threads has a
+// compute unit's registers in FP64 (82 a thread) and with variable
+// coefficients; held to 64, for two, it spills and takes 11.3 and 13.0.
+//
+// A thread owns two pairs of cells (odd i and i + 1), eight planes apart: one red
+// and one black cell each, their RHS (and coefficients) in registers.  In P every
+// cell's potential; in Q the values that the red updates replace, which a
+// black update takes across a periodic face.  Each half sweep updates the
+// cells one further in from the box's surface.
+constexpr int L3_N = 16, L3_TILE = 8, L3_SY = 18, L3_SZ = L3_SY * L3_N, L3_CELLS = L3_SZ * L3_N, L3_NT = 1024;
+template <typename T>
+constexpr int leg3_lds() { return 2 * L3_CELLS * (int)sizeof(T); }
+
+template <typename T, bool UP, bool VAR>
+__global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__restrict__ pout,
+                                                const T *__restrict__ rhs, LegFaces<T> faces, uint32_t bytes,
+                                                const BlockLevel *__restrict__ bls, const Tile *__restrict__ tiles,
+                                                const int *__restrict__ done, const T *__restrict__ phic,
+                                                T *__restrict__ rhsc, uint32_t cbytes,
+                                                const BlockLevel *__restrict__ blc) {
+    const int stop = done ? *done : 0;  // awaited with the tile
+    extern __shared__ __align__(16) unsigned char leg_smem[];
+    T *P = reinterpret_cast<T *>(leg_smem), *Q = P + L3_CELLS;
+    constexpr uint32_t W = sizeof(T);
+    constexpr bool RCP = sizeof(T) == 4;  // the FP32 inner cycle multiplies by 1/ap
+    const Tile t = tiles[blockIdx.x];
+    const BlockLevel g = bls[t.b], gc = blc[t.b];
+    if (stop) return;
+    const auto rs_in = make_rsrc(pin, bytes), rs_f = make_rsrc(rhs, bytes), rs_out = make_rsrc(pout, bytes);
+    const auto rs_c = make_rsrc(UP ? phic : rhsc, cbytes);
+    const auto rs_x = make_rsrc(faces.x, bytes), rs_y = make_rsrc(faces.y, bytes), rs_z = make_rsrc(faces.z, bytes);
+    const bool px = !(g.neu & kNeuW), py = !(g.neu & kNeuS), pz = !(g.neu & kNeuB);  // a lone block's faces come in pairs
+    const T c0 = cconst<T>(g, 0), c1 = cconst<T>(g, 1), c2 = cconst<T>(g, 2);
+    const int tid = (int)threadIdx.x, i = tid & 7, y = (tid >> 3) & 15, zh = tid >> 7;
+    const uint32_t pb = (uint32_t)g.sz * W, rb = (uint32_t)g.sy * W;
+    auto wrap = [](int v, int n, bool per) { return per ? (v < 1 ? v + n : (v > n ? v - n : v)) : (v < 1 ? 1 : (v > n ? n : v)); };
+    const int X = t.x0 - 4 + 2 * i, Y = t.y0 - 4 + y;
+    const int im = wrap(X, g.n0, px) | 1, ip = im > g.n0 ? g.n0 - 1 : im, jm = wrap(Y, g.n1, py);
+
+    // this thread's cells: r red (i + j + k odd), b black
+    T fr[2], fb[2], pr[2], pbk[2];
+    int qr[2], qb[2], dr[2], db[2];
+    unsigned er[2], eb[2];  // faces of the block beside the cell: W E S N B T
+    struct Coef {
+        T w, e, s, n, b, t;
+    } kr[VAR ? 2 : 1], kb[VAR ? 2 : 1];
+    T vr[VAR ? 2 : 1], vb[VAR ? 2 : 1];
+    struct In {
+        Pair<T> f, p, xl, s, n, b, t;
+        T xr;
+    } in[2];
+    bool left[2];  // the left cell is the red one
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int z = zh + 8 * u, km = wrap(t.z0 - 4 + z, g.n2, pz);
+        const uint32_t o = ((uint32_t)g.off + (uint32_t)(ip + (int)g.sy * jm)) * W, s = (uint32_t)km * pb;
+        in[u].f = bload2<T>(rs_f, o + s, 0);
+        if constexpr (UP) in[u].p = bload2<T>(rs_in, o + s, 0);
+        if constexpr (VAR) {
+            in[u].xl = bload2<T>(rs_x, o + s, 0);
+            in[u].xr = bload<T>(rs_x, o + s + 2 * W, 0);
+            in[u].s = bload2<T>(rs_y, o + s, 0);
+            in[u].n = bload2<T>(rs_y, o + s + rb, 0);
+            in[u].b = bload2<T>(rs_z, o + s, 0);
+            in[u].t = bload2<T>(rs_z, o + s + pb, 0);
+        }
+        left[u] = !((Y + t.z0 + z) & 1);
+        const int q = 2 * i + L3_SY * y + L3_SZ * z;
+        const int d = min(min(y, 15 - y), min(z, 15 - z));
+        const int dl = min(d, min(2 * i, 15 - 2 * i)), dd = min(d, min(2 * i + 1, 14 - 2 * i));
+        const unsigned e = (jm == 1 ? 4u : 0u) | (jm == g.n1 ? 8u : 0u) | (km == 1 ? 16u : 0u) | (km == g.n2 ? 32u : 0u);
+        const unsigned el = e | (ip == 1 ? 1u : 0u), ed = e | (ip + 1 == g.n0 ? 2u : 0u);
+        qr[u] = left[u] ? q : q + 1;
+        qb[u] = left[u] ? q + 1 : q;
+        dr[u] = left[u] ? dl : dd;
+        db[u] = left[u] ? dd : dl;
+        er[u] = left[u] ? el : ed;
+        eb[u] = left[u] ? ed : el;
+    }
+    if constexpr (UP) {  // the coarse potential around the box, 10^3, waits in Q
+        if (tid < 1000) {
+            const int a = tid % 10, b = tid / 10 % 10, c = tid / 100;
+            auto coarse = [](int v, int n, bool per) {  // 0 and n + 1 are ghosts
+                return per ? (v < 0 ? v + n : (v > n + 1 ? v - n : v)) : (v < 0 ? 0 : (v > n + 1 ? n + 1 : v));
+            };
+            const int ci = coarse((t.x0 - 5) / 2 + a, gc.n0, px), cj = coarse((t.y0 - 5) / 2 + b, gc.n1, py),
+                      ck = coarse((t.z0 - 5) / 2 + c, gc.n2, pz);
+            Q[tid] = bload<T>(rs_c, ((uint32_t)gc.off + (uint32_t)(ci + (int)gc.sy * cj + (int)gc.sz * ck)) * W, 0);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int z = zh + 8 * u;
+        Pair<T> p{T(0), T(0)};
+        if constexpr (UP) {  // corrected as k_prolong does it
+            const T *e = Q + i + 10 * ((y + 1) >> 1) + 100 * ((z + 1) >> 1);
+            const T wj0 = (y & 1) ? T(3) : T(1), wj1 = (y & 1) ? T(1) : T(3);
+            const T wk0 = (z & 1) ? T(3) : T(1), wk1 = (z & 1) ? T(1) : T(3);
+            auto child = [&](int a, T wi0, T wi1) {
+                T s = (wi0 * wj0 * wk0) * e[a];
+                s = s + (wi0 * wj1 * wk0) * e[a + 10];
+                s = s + (wi0 * wj0 * wk1) * e[a + 100];
+                s = s + (wi0 * wj1 * wk1) * e[a + 110];
+                s = s + (wi1 * wj0 * wk0) * e[a + 1];
+                s = s + (wi1 * wj1 * wk0) * e[a + 11];
+                s = s + (wi1 * wj0 * wk1) * e[a + 101];
+                s = s + (wi1 * wj1 * wk1) * e[a + 111];
+                return s / T(64);
+            };
+            p.l = in[u].p.l + child(0, T(1), T(3));
+            p.r = in[u].p.r + child(1, T(3), T(1));
+        }
+        fr[u] = left[u] ? in[u].f.l : in[u].f.r;
+        fb[u] = left[u] ? in[u].f.r : in[u].f.l;
+        pr[u] = left[u] ? p.l : p.r;
+        pbk[u] = left[u] ? p.r : p.l;
+        if constexpr (VAR) {
+            const In &v = in[u];
+            const Coef l{v.xl.l, v.xl.r, v.s.l, v.n.l, v.b.l, v.t.l}, r{v.xl.r, v.xr, v.s.r, v.n.r, v.b.r, v.t.r};
+            kr[u] = left[u] ? l : r;
+            kb[u] = left[u] ? r : l;
+            auto inv = [](const Coef &k) { return T(1) / -(((((k.w + k.e) + k.s) + k.n) + k.b) + k.t); };
+            vr[u] = inv(kr[u]);
+            vb[u] = inv(kb[u]);
+        }
+    }
+    if constexpr (UP) __syncthreads();  // Q is free
+
+    auto coef = [&](int u, bool red, unsigned e) {  // walls have no coefficient
+        if constexpr (VAR) return red ? kr[u] : kb[u];
+        else
+            return Coef{(e & 1) && !px ? T(0) : c0, (e & 2) && !px ? T(0) : c0, (e & 4) && !py ? T(0) : c1,
+                        (e & 8) && !py ? T(0) : c1, (e & 16) && !pz ? T(0) : c2, (e & 32) && !pz ? T(0) : c2};
+    };
+    auto diag = [](const Coef &k) { return -(((((k.w + k.e) + k.s) + k.n) + k.b) + k.t); };
+    auto divide = [&](int u, bool red, const Coef &k, T r) {
+        if constexpr (VAR) return r * (red ? vr[u] : vb[u]);
+        else if constexpr (RCP) return r * (T(1) / diag(k));
+        else return r / diag(k);
+    };
+    auto update = [&](int u, bool red) {
+        const int q = red ? qr[u] : qb[u];
+        const unsigned e = red ? er[u] : eb[u];
+        T w = P[q - 1], ea = P[q + 1], s = P[q - L3_SY], n = P[q + L3_SY], b = P[q - L3_SZ], tp = P[q + L3_SZ];
+        if (!red && e) {  // across a periodic face, the red value from before the sweep
+            if ((e & 1) && px) w = Q[q - 1];
+            if ((e & 2) && px) ea = Q[q + 1];
+            if ((e & 4) && py) s = Q[q - L3_SY];
+            if ((e & 8) && py) n = Q[q + L3_SY];
+            if ((e & 16) && pz) b = Q[q - L3_SZ];
+            if ((e & 32) && pz) tp = Q[q + L3_SZ];
+        }
+        const Coef k = coef(u, red, e);
+        T a = k.w * w;
+        a = madd(a, k.e, ea);
+        a = madd(a, k.s, s);
+        a = madd(a, k.n, n);
+        a = madd(a, k.b, b);
+        a = madd(a, k.t, tp);
+        return divide(u, red, k, (red ? fr[u] : fb[u]) - a);
+    };
+    constexpr int D0 = UP ? 1 : 0;  // distance from the box's surface of the first half sweep
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        if constexpr (UP) {
+            P[qr[u]] = pr[u];
+        } else {
+            pr[u] = divide(u, true, coef(u, true, er[u]), fr[u] - T(0));
+            P[qr[u]] = pr[u];
+            Q[qr[u]] = T(0);
+        }
+        P[qb[u]] = pbk[u];
+    }
+    __syncthreads();
+    auto reds = [&](int dmin) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            if (dr[u] >= dmin) {
+                const T v = update(u, true);
+                Q[qr[u]] = pr[u];
+                P[qr[u]] = pr[u] = v;
+            }
+        __syncthreads();
+    };
+    auto blacks = [&](int dmin) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            if (db[u] >= dmin) P[qb[u]] = pbk[u] = update(u, false);
+        __syncthreads();
+    };
+    if constexpr (UP) reds(D0);
+    blacks(D0 + 1);
+    reds(D0 + 2);
+    blacks(D0 + 3);
+
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int z = zh + 8 * u, Z = t.z0 - 4 + z;
+        if (i < 2 || i > 5 || y < 4 || y > 11 || z < 4 || z > 11) continue;  // the ring
+        if (X > g.n0 || Y > g.n1 || Z > g.n2) continue;
+        const Pair<T> v{left[u] ? pr[u] : pbk[u], left[u] ? pbk[u] : pr[u]};
+        auto at = [&](int x, int yy, int zz) { return ((uint32_t)g.off + (uint32_t)(x + (int)g.sy * yy)) * W + (uint32_t)zz * pb; };
+        bstore2<T>(rs_out, v, at(X, Y, Z), 0);
+        if constexpr (UP) {  // the ghost images; the up leg reads no ghosts of its level, so down writes none
+            const int xl = ghost_image(X, g.n0, g.neu & kNeuW, g.neu & kNeuE);
+            const int xr = ghost_image(X + 1, g.n0, g.neu & kNeuW, g.neu & kNeuE);
+            const int yg = ghost_image(Y, g.n1, g.neu & kNeuS, g.neu & kNeuN);
+            const int zg = ghost_image(Z, g.n2, g.neu & kNeuB, g.neu & kNeuT);
+#pragma unroll 1
+            for (int m = 0; m < 4; ++m) {
+                const int yy = m & 1 ? yg : Y, zz = m & 2 ? zg : Z;
+                if (yy < 0 || zz < 0) continue;
+                if (m) bstore2<T>(rs_out, v, at(X, yy, zz), 0);
+                if (xl >= 0) bstore<T>(rs_out, v.l, at(xl, yy, zz), 0);
+                if (xr >= 0) bstore<T>(rs_out, v.r, at(xr, yy, zz), 0);
+            }
+        } else {  // the residual, its ghosts refreshed, without contraction as k_restrict
+            auto residual = [&](bool red) {
+                const int q = red ? qr[u] : qb[u];
+                const Coef k = coef(u, red, red ? er[u] : eb[u]);
+                T s = k.w * P[q - 1];
+                s = s + k.e * P[q + 1];
+                s = s + k.s * P[q - L3_SY];
+                s = s + k.n * P[q + L3_SY];
+                s = s + k.b * P[q - L3_SZ];
+                s = s + k.t * P[q + L3_SZ];
+                s = s + diag(k) * P[q];
+                return (red ? fr[u] : fb[u]) - s;
+            };
+            Q[qr[u]] = residual(true);
+            Q[qb[u]] = residual(false);
+        }
+    }
+    if constexpr (!UP) {
+        __syncthreads();
+        if (tid < 64) {
+            const int a = tid & 3, b = (tid >> 2) & 3, c = tid >> 4;
+            const int ci = (t.x0 + 1) / 2 + a, cj = (t.y0 + 1) / 2 + b, ck = (t.z0 + 1) / 2 + c;
+            if (ci <= gc.n0 && cj <= gc.n1 && ck <= gc.n2) {
+                const T *r = Q + (4 + 2 * a) + L3_SY * (4 + 2 * b) + L3_SZ * (4 + 2 * c);
+                T s = r[0];
+                s = s + r[1];
+                s = s + r[L3_SY];
+                s = s + r[L3_SY + 1];
+                s = s + r[L3_SZ];
+                s = s + r[L3_SZ + 1];
+                s = s + r[L3_SZ + L3_SY];
+                s = s + r[L3_SZ + L3_SY + 1];
+                bstore<T>(rs_c, T(0.125) * s, ((uint32_t)gc.off + (uint32_t)(ci + (int)gc.sy * cj + (int)gc.sz * ck)) * W, 0);
+            }
+        }
     }
 }
 
