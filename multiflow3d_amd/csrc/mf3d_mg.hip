@@ -983,7 +983,6 @@ void leg_launch(mf3d_mg *mg, int l, const int *done) {
                            (const T *)F.phi[F.cur], (T *)F.phi[1 - F.cur], (const T *)F.rhs, faces, bytes, F.db, g.t,
                            done, (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db, mg->d_around);
     };
-    constexpr int NY = leg_ny<T>(VAR);
     if constexpr (!MB) {
         if (!g.ny) {
             hipLaunchKernelGGL((k_leg3<T, UP, VAR>), dim3(g.n), dim3(L3_NT), leg3_lds<T>(), mg->stream,
@@ -992,8 +991,11 @@ void leg_launch(mf3d_mg *mg, int l, const int *done) {
             return;
         }
     }
-    if (g.ny == NY) go(k_leg<T, UP, NY, VAR, MB>);
-    else go(k_leg<T, UP, LEG_NY_SMALL, VAR, MB>);
+    if constexpr (leg_march<T, VAR>()) {
+        constexpr int NY = leg_ny<T>(VAR);
+        if (g.ny == NY) go(k_leg<T, UP, NY, VAR, MB>);
+        else go(k_leg<T, UP, LEG_NY_SMALL, VAR, MB>);
+    }
 }
 
 template <typename T, bool VAR, bool UP>
@@ -1020,11 +1022,9 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
     }
     // the down leg of level l; true: it restricted into level l+1 too
     auto down = [&](int l, bool zero) {
-        if constexpr (leg_type<T, VAR>()) {
-            if (zero && mg->lv[l].legs[0].n) {
-                leg<T, VAR, false>(mg, l, done);
-                return true;
-            }
+        if (zero && mg->lv[l].legs[0].n) {
+            leg<T, VAR, false>(mg, l, done);
+            return true;
         }
         relax<T, VAR>(mg, l, mg->cfg.nu_pre, zero, done);
         return false;
@@ -1050,12 +1050,8 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
         for (int l = ldown - 1; l >= 0; --l) {
             if (l == L - 1) continue;
             int post = mg->cfg.nu_post;
-            bool whole = false;
-            if constexpr (leg_type<T, VAR>()) {
-                whole = mg->lv[l].legs[1].n != 0;
-                if (whole) leg<T, VAR, true>(mg, l, done);
-            }
-            if (whole) {
+            if (mg->lv[l].legs[1].n) {
+                leg<T, VAR, true>(mg, l, done);
                 post = 0;
             } else if (fused_prolong(mg, l)) {
                 prolong_sweep<T, VAR>(mg, l, done);
@@ -1938,7 +1934,6 @@ std::vector<Tile> leg_tiles(const std::vector<BlockLevel> &hb, int ty, int slots
 // One leg's kernels may use the LDS they need, and its tiles on level V.
 template <typename T, bool VAR, bool UP, bool MB>
 int leg_level(mf3d_mg *mg, Level &V, int cus) {
-    constexpr int SM = LEG_NY_SMALL, NY = leg_ny<T>(VAR);
     Level::Leg &g = V.legs[UP];
     // the kernel's LDS; tiles, or the other leg's where they are the same
     auto take = [&](const void *kernel, int lds, int ny, std::vector<Tile> t) {
@@ -1969,16 +1964,23 @@ int leg_level(mf3d_mg *mg, Level &V, int cus) {
         // (us a leg, march / boxes; down, up.  FP64 32^3 13.0 / 6.7, 13.4 / 9.3; 48^3
         // 14.2 / 7.6, 13.8 / 10.0; 64^3 17.0 / 13.6, 16.4 / 17.6; FP32 32^3 9.1 / 5.6,
         // 10.8 / 7.3; 64^3 11.4 / 8.5, 12.2 / 10.7; 80^3 14.9 / 13.7, 16.6 / 17.6; 96^3
-        // 15.2 / 22.3, 17.3 / 29.4).
-        if ((int)box.size() <= (sizeof(T) == 8 && UP ? 1 : 2) * cus)
+        // 15.2 / 22.3, 17.3 / 29.4).  FP64 with variable coefficients has no march:
+        // boxes against separate kernels, a leg pair, 48^3 22 / 44, 64^3 36 / 39,
+        // 80^3 70 / 87, 96^3 124 / 129: four a compute unit.
+        const int per_cu = sizeof(T) == 8 ? (VAR ? 4 : (UP ? 1 : 2)) : 2;
+        if ((int)box.size() <= per_cu * cus)
             return take((const void *)k_leg3<T, UP, VAR>, leg3_lds<T>(), 0, std::move(box));
     }
-    long long many, few;
-    auto t = leg_tiles(V.hb, NY - 8, cus, &many);
-    auto ts = leg_tiles(V.hb, SM - 8, cus, &few);
-    if (few * 4 < many * 5)
-        return take((const void *)k_leg<T, UP, SM, VAR, MB>, leg_lds<T>(UP, true, SM, VAR), SM, std::move(ts));
-    return take((const void *)k_leg<T, UP, NY, VAR, MB>, leg_lds<T>(UP, true, NY, VAR), NY, std::move(t));
+    if constexpr (leg_march<T, VAR>()) {
+        constexpr int SM = LEG_NY_SMALL, NY = leg_ny<T>(VAR);
+        long long many, few;
+        auto t = leg_tiles(V.hb, NY - 8, cus, &many);
+        auto ts = leg_tiles(V.hb, SM - 8, cus, &few);
+        if (few * 4 < many * 5)
+            return take((const void *)k_leg<T, UP, SM, VAR, MB>, leg_lds<T>(UP, true, SM, VAR), SM, std::move(ts));
+        return take((const void *)k_leg<T, UP, NY, VAR, MB>, leg_lds<T>(UP, true, NY, VAR), NY, std::move(t));
+    }
+    return 0;
 }
 
 // The blocks around each block (LegBlocks), found as build_regions finds a
@@ -2040,7 +2042,8 @@ int leg_levels(mf3d_mg *mg, bool down) {
         int rc = 0;
         if (V.own_ghosts) {
             rc = leg_level<T, VAR, true, false>(mg, V, cus);
-            if (!rc && down) rc = leg_level<T, VAR, false, false>(mg, V, cus);
+            // the down leg writes no ghosts: it needs an up leg, which reads none
+            if (!rc && down && V.legs[1].n) rc = leg_level<T, VAR, false, false>(mg, V, cus);
         } else if constexpr (!VAR) {
             rc = leg_level<T, VAR, true, true>(mg, V, cus);
             if (!rc && down) rc = leg_level<T, VAR, false, true>(mg, V, cus);
@@ -2051,7 +2054,7 @@ int leg_levels(mf3d_mg *mg, bool down) {
 }
 
 // Which levels run their legs as one launch each: red-black sweeps, two a leg,
-// of lone blocks (constant coefficients, or variable ones in the FP32 cycle)
+// of lone blocks (FP64 with variable coefficients on small levels only)
 // or of block grids that leg_blocks admits, all of one spacing (constant
 // coefficients), every extent even and at least 8 (the ring of a tile then
 // crosses one face at most a side), above the LDS tail and the coarsest level.
@@ -2059,14 +2062,14 @@ int leg_setup(mf3d_mg *mg) {
     const mf3d_mg_cfg &c = mg->cfg;
     const bool mixed = c.precision == MF3D_MIXED, var = c.variable_coef != 0;
     const bool any_up = c.nu_post == 2, any_down = any_up && c.nu_pre == 2;  // the down leg writes no ghosts: the up leg needs none
-    if (!mg->legs || c.smoother != 3 || mg->refined || !any_up || (var && !mixed)) return 0;
+    if (!mg->legs || c.smoother != 3 || mg->refined || !any_up) return 0;
     if (!var) {
         const auto around = leg_blocks(mg->blk);
         if (!around.empty())
             if (int rc = upload(mg, &mg->d_around, around)) return rc;
     }
     return mixed ? (var ? leg_levels<float, true>(mg, any_down) : leg_levels<float, false>(mg, any_down))
-                 : leg_levels<double, false>(mg, any_down);
+                 : (var ? leg_levels<double, true>(mg, any_down) : leg_levels<double, false>(mg, any_down));
 }
 
 int build(mf3d_mg *mg) {

@@ -70,10 +70,10 @@ namespace mf3d {
 constexpr int LEG_TX = 52, LEG_NY_SMALL = 16;
 template <typename T>
 constexpr int leg_ny(bool var) { return var ? 24 : (sizeof(T) == 4 ? 32 : 24); }
-// Variable coefficients in FP32 only: in FP64 a thread's coefficients of the
-// four planes would not fit in registers.
+// Variable coefficients are marched in FP32 only: in FP64 a thread's
+// coefficients of the four planes would not fit in registers.
 template <typename T, bool VAR>
-constexpr bool leg_type() { return sizeof(T) == 4 || !VAR; }
+constexpr bool leg_march() { return sizeof(T) == 4 || !VAR; }
 
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int v) {
@@ -830,9 +830,12 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
             const Coef l{v.xl.l, v.xl.r, v.s.l, v.n.l, v.b.l, v.t.l}, r{v.xl.r, v.xr, v.s.r, v.n.r, v.b.r, v.t.r};
             kr[u] = left[u] ? l : r;
             kb[u] = left[u] ? r : l;
-            auto inv = [](const Coef &k) { return T(1) / -(((((k.w + k.e) + k.s) + k.n) + k.b) + k.t); };
-            vr[u] = inv(kr[u]);
-            vb[u] = inv(kb[u]);
+            auto divisor = [](const Coef &k) {
+                const T ap = -(((((k.w + k.e) + k.s) + k.n) + k.b) + k.t);
+                return RCP ? T(1) / ap : ap;
+            };
+            vr[u] = divisor(kr[u]);
+            vb[u] = divisor(kb[u]);
         }
     }
     if constexpr (UP) __syncthreads();  // Q is free
@@ -845,7 +848,7 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
     };
     auto diag = [](const Coef &k) { return -(((((k.w + k.e) + k.s) + k.n) + k.b) + k.t); };
     auto divide = [&](int u, bool red, const Coef &k, T r) {
-        if constexpr (VAR) return r * (red ? vr[u] : vb[u]);
+        if constexpr (VAR) return RCP ? r * (red ? vr[u] : vb[u]) : r / (red ? vr[u] : vb[u]);
         else if constexpr (RCP) return r * (T(1) / diag(k));
         else return r / diag(k);
     };
