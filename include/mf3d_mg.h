@@ -309,7 +309,9 @@ int mf3d_mg_ghost_table(const mf3d_mg_cfg *cfg, const mf3d_block_desc *blocks, i
  * mf3d_mg_graph_replay).  Cycles skipped after convergence are not
  * counted.  mf3d_mg_time_kernel selects the kernel (MF3D_K_*; 0 = off)
  * and resets the counters; mf3d_mg_kernel_time returns the launches seen
- * and their summed time. */
+ * and their summed time.  MF3D_K_SMOOTH counts a leg of the V-cycle (two
+ * sweeps and the transfer) where the level runs legs as one launch each;
+ * MF3D_K_RESTRICT and MF3D_K_PROLONG run them as separate kernels. */
 enum {
     MF3D_K_OFF = 0,
     MF3D_K_SMOOTH = 1,

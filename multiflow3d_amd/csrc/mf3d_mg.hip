@@ -1020,9 +1020,11 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
         tail<T, VAR>(mg, zero_start, done);
         return;
     }
+    // timing the restriction or the prolongation keeps them kernels of their own
+    const bool legs = mg->tk != MF3D_K_RESTRICT && mg->tk != MF3D_K_PROLONG;
     // the down leg of level l; true: it restricted into level l+1 too
     auto down = [&](int l, bool zero) {
-        if (zero && mg->lv[l].legs[0].n) {
+        if (zero && legs && mg->lv[l].legs[0].n) {
             leg<T, VAR, false>(mg, l, done);
             return true;
         }
@@ -1050,7 +1052,7 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
         for (int l = ldown - 1; l >= 0; --l) {
             if (l == L - 1) continue;
             int post = mg->cfg.nu_post;
-            if (mg->lv[l].legs[1].n) {
+            if (legs && mg->lv[l].legs[1].n) {
                 leg<T, VAR, true>(mg, l, done);
                 post = 0;
             } else if (fused_prolong(mg, l)) {
@@ -2063,7 +2065,7 @@ int leg_setup(mf3d_mg *mg) {
     const bool mixed = c.precision == MF3D_MIXED, var = c.variable_coef != 0;
     const bool any_up = c.nu_post == 2, any_down = any_up && c.nu_pre == 2;  // the down leg writes no ghosts: the up leg needs none
     if (!mg->legs || c.smoother != 3 || mg->refined || !any_up) return 0;
-    if (!var) {
+    if (!var && !mg->lv[0].own_ghosts) {
         const auto around = leg_blocks(mg->blk);
         if (!around.empty())
             if (int rc = upload(mg, &mg->d_around, around)) return rc;
