@@ -983,13 +983,11 @@ void leg_launch(mf3d_mg *mg, int l, const int *done) {
                            (const T *)F.phi[F.cur], (T *)F.phi[1 - F.cur], (const T *)F.rhs, faces, bytes, F.db, g.t,
                            done, (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db, mg->d_around);
     };
-    if constexpr (!MB) {
-        if (!g.ny) {
-            hipLaunchKernelGGL((k_leg3<T, UP, VAR>), dim3(g.n), dim3(L3_NT), leg3_lds<T>(), mg->stream,
-                               (const T *)F.phi[F.cur], (T *)F.phi[1 - F.cur], (const T *)F.rhs, faces, bytes, F.db, g.t,
-                               done, (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db);
-            return;
-        }
+    if (!g.ny) {
+        hipLaunchKernelGGL((k_leg3<T, UP, VAR, MB>), dim3(g.n), dim3(L3_NT), leg3_lds<T>(), mg->stream,
+                           (const T *)F.phi[F.cur], (T *)F.phi[1 - F.cur], (const T *)F.rhs, faces, bytes, F.db, g.t,
+                           done, (const T *)C.phi[C.cur], (T *)C.rhs, cbytes, C.db, mg->d_around);
+        return;
     }
     if constexpr (leg_march<T, VAR>()) {
         constexpr int NY = leg_ny<T>(VAR);
@@ -1956,23 +1954,21 @@ int leg_level(mf3d_mg *mg, Level &V, int cus) {
     // few, of which half belong to the ring.  Few on levels that leave compute
     // units idle (64^3: 13.0 us against 14.7 a leg in FP32, 17.4 against 18.4 in
     // FP64), many from where all are busy (128^3: 34 against 25).
-    if constexpr (!MB) {
-        std::vector<Tile> box;
-        for (int b = 0; b < (int)V.hb.size(); ++b)
-            for (int z = 1; z <= V.hb[b].n2; z += L3_TILE)
-                for (int y = 1; y <= V.hb[b].n1; y += L3_TILE)
-                    for (int x = 1; x <= V.hb[b].n0; x += L3_TILE) box.push_back(Tile{b, x, y, z, z + L3_TILE - 1});
-        // Boxes while they do not fill the card: two a compute unit, the FP64 up leg one
-        // (us a leg, march / boxes; down, up.  FP64 32^3 13.0 / 6.7, 13.4 / 9.3; 48^3
-        // 14.2 / 7.6, 13.8 / 10.0; 64^3 17.0 / 13.6, 16.4 / 17.6; FP32 32^3 9.1 / 5.6,
-        // 10.8 / 7.3; 64^3 11.4 / 8.5, 12.2 / 10.7; 80^3 14.9 / 13.7, 16.6 / 17.6; 96^3
-        // 15.2 / 22.3, 17.3 / 29.4).  FP64 with variable coefficients has no march:
-        // boxes against separate kernels, a leg pair, 48^3 22 / 44, 64^3 36 / 39,
-        // 80^3 70 / 87, 96^3 124 / 129: four a compute unit.
-        const int per_cu = sizeof(T) == 8 ? (VAR ? 4 : (UP ? 1 : 2)) : 2;
-        if ((int)box.size() <= per_cu * cus)
-            return take((const void *)k_leg3<T, UP, VAR>, leg3_lds<T>(), 0, std::move(box));
-    }
+    std::vector<Tile> box;
+    for (int b = 0; b < (int)V.hb.size(); ++b)
+        for (int z = 1; z <= V.hb[b].n2; z += L3_TILE)
+            for (int y = 1; y <= V.hb[b].n1; y += L3_TILE)
+                for (int x = 1; x <= V.hb[b].n0; x += L3_TILE) box.push_back(Tile{b, x, y, z, z + L3_TILE - 1});
+    // Boxes while they do not fill the card: two a compute unit, the FP64 up leg one
+    // (us a leg, march / boxes; down, up.  FP64 32^3 13.0 / 6.7, 13.4 / 9.3; 48^3
+    // 14.2 / 7.6, 13.8 / 10.0; 64^3 17.0 / 13.6, 16.4 / 17.6; FP32 32^3 9.1 / 5.6,
+    // 10.8 / 7.3; 64^3 11.4 / 8.5, 12.2 / 10.7; 80^3 14.9 / 13.7, 16.6 / 17.6; 96^3
+    // 15.2 / 22.3, 17.3 / 29.4).  FP64 with variable coefficients has no march:
+    // boxes against separate kernels, a leg pair, 48^3 22 / 44, 64^3 36 / 39,
+    // 80^3 70 / 87, 96^3 124 / 129: four a compute unit.
+    const int per_cu = sizeof(T) == 8 ? (VAR ? 4 : (UP ? 1 : 2)) : 2;
+    if ((int)box.size() <= per_cu * cus)
+        return take((const void *)k_leg3<T, UP, VAR, MB>, leg3_lds<T>(), 0, std::move(box));
     if constexpr (leg_march<T, VAR>()) {
         constexpr int SM = LEG_NY_SMALL, NY = leg_ny<T>(VAR);
         long long many, few;

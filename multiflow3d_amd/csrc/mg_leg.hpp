@@ -702,7 +702,7 @@ __global__ __launch_bounds__(32 * NY) void k_leg(const T *__restrict__ pin, T *_
     }
 }
 
-// The same leg on a small level of a lone block, a box at a time: a workgroup takes
+// The same leg on a small level, a box at a time: a workgroup takes
 // 8 x 8 x 8 cells with a ring of 4 (16^3 cells) into LDS and does the four half
 // sweeps there, one barrier each, where the march above takes a step of about
 // 1 us for each of at least ten planes.  The ring makes it eight times the
@@ -721,13 +721,14 @@ constexpr int L3_N = 16, L3_TILE = 8, L3_SY = 18, L3_SZ = L3_SY * L3_N, L3_CELLS
 template <typename T>
 constexpr int leg3_lds() { return 2 * L3_CELLS * (int)sizeof(T); }
 
-template <typename T, bool UP, bool VAR>
+template <typename T, bool UP, bool VAR, bool MB = false>
 __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__restrict__ pout,
                                                 const T *__restrict__ rhs, LegFaces<T> faces, uint32_t bytes,
                                                 const BlockLevel *__restrict__ bls, const Tile *__restrict__ tiles,
                                                 const int *__restrict__ done, const T *__restrict__ phic,
                                                 T *__restrict__ rhsc, uint32_t cbytes,
-                                                const BlockLevel *__restrict__ blc) {
+                                                const BlockLevel *__restrict__ blc,
+                                                const LegBlocks *__restrict__ around) {
     const int stop = done ? *done : 0;  // awaited with the tile
     extern __shared__ __align__(16) unsigned char leg_smem[];
     T *P = reinterpret_cast<T *>(leg_smem), *Q = P + L3_CELLS;
@@ -739,18 +740,29 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
     const auto rs_in = make_rsrc(pin, bytes), rs_f = make_rsrc(rhs, bytes), rs_out = make_rsrc(pout, bytes);
     const auto rs_c = make_rsrc(UP ? phic : rhsc, cbytes);
     const auto rs_x = make_rsrc(faces.x, bytes), rs_y = make_rsrc(faces.y, bytes), rs_z = make_rsrc(faces.z, bytes);
-    const bool px = !(g.neu & kNeuW), py = !(g.neu & kNeuS), pz = !(g.neu & kNeuB);  // a lone block's faces come in pairs
+    const bool wallW = g.neu & kNeuW, wallE = g.neu & kNeuE, wallS = g.neu & kNeuS, wallN = g.neu & kNeuN;
+    const bool wallBot = g.neu & kNeuB, wallTop = g.neu & kNeuT;
     const T c0 = cconst<T>(g, 0), c1 = cconst<T>(g, 1), c2 = cconst<T>(g, 2);
     const int tid = (int)threadIdx.x, i = tid & 7, y = (tid >> 3) & 15, zh = tid >> 7;
-    const uint32_t pb = (uint32_t)g.sz * W, rb = (uint32_t)g.sy * W;
-    auto wrap = [](int v, int n, bool per) { return per ? (v < 1 ? v + n : (v > n ? v - n : v)) : (v < 1 ? 1 : (v > n ? n : v)); };
+    const uint32_t rb = (uint32_t)g.sy * W;
     const int X = t.x0 - 4 + 2 * i, Y = t.y0 - 4 + y;
-    const int im = wrap(X, g.n0, px) | 1, ip = im > g.n0 ? g.n0 - 1 : im, jm = wrap(Y, g.n1, py);
-
+    // the side of the block that coordinate v is on (0: the block, or beyond a wall),
+    // and the cell 1..m there (n, m: extents of the block and of the one there)
+    auto side = [](int v, int n, bool lo, bool hi) { return v < 1 && !lo ? -1 : (v > n && !hi ? 1 : 0); };
+    auto cell = [](int v, int n, int m, int k) {
+        const int c = k < 0 ? v + m : (k > 0 ? v - n : v);
+        return c < 1 ? 1 : (c > m ? m : c);
+    };
+    const int xk = side(X, g.n0, wallW, wallE), yk = side(Y, g.n1, wallS, wallN);
+    const int *nb = MB ? around[t.b].nb : nullptr;
+    const BlockLevel &own = MB ? bls[nb[13 + 3 * yk + xk]] : bls[t.b];  // the column's block, beside this one
+    const int n0 = own.n0, n1 = own.n1;
+    const int im = cell(X, g.n0, n0, xk) | 1, ip = im > n0 ? n0 - 1 : im, jm = cell(Y, g.n1, n1, yk);
+    const uint32_t pb = (uint32_t)own.sz * W;
     // this thread's cells: r red (i + j + k odd), b black
     T fr[2], fb[2], pr[2], pbk[2];
     int qr[2], qb[2], dr[2], db[2];
-    unsigned er[2], eb[2];  // faces of the block beside the cell: W E S N B T
+    unsigned er[2], eb[2];  // faces of its block beside the cell, W E S N B T: to other cells, then (<< 6) walls
     struct Coef {
         T w, e, s, n, b, t;
     } kr[VAR ? 2 : 1], kb[VAR ? 2 : 1];
@@ -762,8 +774,10 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
     bool left[2];  // the left cell is the red one
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-        const int z = zh + 8 * u, km = wrap(t.z0 - 4 + z, g.n2, pz);
-        const uint32_t o = ((uint32_t)g.off + (uint32_t)(ip + (int)g.sy * jm)) * W, s = (uint32_t)km * pb;
+        const int z = zh + 8 * u, Z = t.z0 - 4 + z, zk = side(Z, g.n2, wallBot, wallTop);
+        const BlockLevel &there = MB ? bls[nb[13 + 9 * zk + 3 * yk + xk]] : bls[t.b];
+        const int n2 = there.n2, km = cell(Z, g.n2, n2, zk);
+        const uint32_t o = ((uint32_t)there.off + (uint32_t)(ip + (int)own.sy * jm)) * W, s = (uint32_t)km * pb;
         in[u].f = bload2<T>(rs_f, o + s, 0);
         if constexpr (UP) in[u].p = bload2<T>(rs_in, o + s, 0);
         if constexpr (VAR) {
@@ -778,8 +792,10 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
         const int q = 2 * i + L3_SY * y + L3_SZ * z;
         const int d = min(min(y, 15 - y), min(z, 15 - z));
         const int dl = min(d, min(2 * i, 15 - 2 * i)), dd = min(d, min(2 * i + 1, 14 - 2 * i));
-        const unsigned e = (jm == 1 ? 4u : 0u) | (jm == g.n1 ? 8u : 0u) | (km == 1 ? 16u : 0u) | (km == g.n2 ? 32u : 0u);
-        const unsigned el = e | (ip == 1 ? 1u : 0u), ed = e | (ip + 1 == g.n0 ? 2u : 0u);
+        auto face = [](bool at, bool wall, unsigned bit) { return at ? (wall ? bit << 6 : bit) : 0u; };
+        const unsigned e = face(jm == 1, yk == 0 && wallS, 4) | face(jm == n1, yk == 0 && wallN, 8) |
+                           face(km == 1, zk == 0 && wallBot, 16) | face(km == n2, zk == 0 && wallTop, 32);
+        const unsigned el = e | face(ip == 1, xk == 0 && wallW, 1), ed = e | face(ip + 1 == n0, xk == 0 && wallE, 2);
         qr[u] = left[u] ? q : q + 1;
         qb[u] = left[u] ? q + 1 : q;
         dr[u] = left[u] ? dl : dd;
@@ -790,12 +806,17 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
     if constexpr (UP) {  // the coarse potential around the box, 10^3, waits in Q
         if (tid < 1000) {
             const int a = tid % 10, b = tid / 10 % 10, c = tid / 100;
-            auto coarse = [](int v, int n, bool per) {  // 0 and n + 1 are ghosts
-                return per ? (v < 0 ? v + n : (v > n + 1 ? v - n : v)) : (v < 0 ? 0 : (v > n + 1 ? n + 1 : v));
+            auto cside = [](int v, int n, bool lo, bool hi) { return v < 0 && !lo ? -1 : (v > n + 1 && !hi ? 1 : 0); };
+            auto ccell = [](int v, int n, int m, int k) {  // 0 and m + 1 are ghosts
+                const int q = k < 0 ? v + m : (k > 0 ? v - n : v);
+                return q < 0 ? 0 : (q > m + 1 ? m + 1 : q);
             };
-            const int ci = coarse((t.x0 - 5) / 2 + a, gc.n0, px), cj = coarse((t.y0 - 5) / 2 + b, gc.n1, py),
-                      ck = coarse((t.z0 - 5) / 2 + c, gc.n2, pz);
-            Q[tid] = bload<T>(rs_c, ((uint32_t)gc.off + (uint32_t)(ci + (int)gc.sy * cj + (int)gc.sz * ck)) * W, 0);
+            const int cx = (t.x0 - 5) / 2 + a, cy = (t.y0 - 5) / 2 + b, cz = (t.z0 - 5) / 2 + c;
+            const int ka = cside(cx, gc.n0, wallW, wallE), kb2 = cside(cy, gc.n1, wallS, wallN),
+                      kc = cside(cz, gc.n2, wallBot, wallTop);
+            const BlockLevel &q = MB ? blc[nb[13 + 9 * kc + 3 * kb2 + ka]] : blc[t.b];
+            const int ci = ccell(cx, gc.n0, q.n0, ka), cj = ccell(cy, gc.n1, q.n1, kb2), ck = ccell(cz, gc.n2, q.n2, kc);
+            Q[tid] = bload<T>(rs_c, ((uint32_t)q.off + (uint32_t)(ci + (int)q.sy * cj + (int)q.sz * ck)) * W, 0);
         }
         __syncthreads();
     }
@@ -843,8 +864,8 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
     auto coef = [&](int u, bool red, unsigned e) {  // walls have no coefficient
         if constexpr (VAR) return red ? kr[u] : kb[u];
         else
-            return Coef{(e & 1) && !px ? T(0) : c0, (e & 2) && !px ? T(0) : c0, (e & 4) && !py ? T(0) : c1,
-                        (e & 8) && !py ? T(0) : c1, (e & 16) && !pz ? T(0) : c2, (e & 32) && !pz ? T(0) : c2};
+            return Coef{(e & 64) ? T(0) : c0, (e & 128) ? T(0) : c0, (e & 256) ? T(0) : c1,
+                        (e & 512) ? T(0) : c1, (e & 1024) ? T(0) : c2, (e & 2048) ? T(0) : c2};
     };
     auto diag = [](const Coef &k) { return -(((((k.w + k.e) + k.s) + k.n) + k.b) + k.t); };
     auto divide = [&](int u, bool red, const Coef &k, T r) {
@@ -856,13 +877,13 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
         const int q = red ? qr[u] : qb[u];
         const unsigned e = red ? er[u] : eb[u];
         T w = P[q - 1], ea = P[q + 1], s = P[q - L3_SY], n = P[q + L3_SY], b = P[q - L3_SZ], tp = P[q + L3_SZ];
-        if (!red && e) {  // across a periodic face, the red value from before the sweep
-            if ((e & 1) && px) w = Q[q - 1];
-            if ((e & 2) && px) ea = Q[q + 1];
-            if ((e & 4) && py) s = Q[q - L3_SY];
-            if ((e & 8) && py) n = Q[q + L3_SY];
-            if ((e & 16) && pz) b = Q[q - L3_SZ];
-            if ((e & 32) && pz) tp = Q[q + L3_SZ];
+        if (!red && (e & 63)) {  // across a face of its block, the red value from before the sweep
+            if (e & 1) w = Q[q - 1];
+            if (e & 2) ea = Q[q + 1];
+            if (e & 4) s = Q[q - L3_SY];
+            if (e & 8) n = Q[q + L3_SY];
+            if (e & 16) b = Q[q - L3_SZ];
+            if (e & 32) tp = Q[q + L3_SZ];
         }
         const Coef k = coef(u, red, e);
         T a = k.w * w;
@@ -910,12 +931,13 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const int z = zh + 8 * u, Z = t.z0 - 4 + z;
+        const uint32_t pl = (uint32_t)g.sz * W;
         if (i < 2 || i > 5 || y < 4 || y > 11 || z < 4 || z > 11) continue;  // the ring
         if (X > g.n0 || Y > g.n1 || Z > g.n2) continue;
         const Pair<T> v{left[u] ? pr[u] : pbk[u], left[u] ? pbk[u] : pr[u]};
-        auto at = [&](int x, int yy, int zz) { return ((uint32_t)g.off + (uint32_t)(x + (int)g.sy * yy)) * W + (uint32_t)zz * pb; };
+        auto at = [&](int x, int yy, int zz) { return ((uint32_t)g.off + (uint32_t)(x + (int)g.sy * yy)) * W + (uint32_t)zz * pl; };
         bstore2<T>(rs_out, v, at(X, Y, Z), 0);
-        if constexpr (UP) {  // the ghost images; the up leg reads no ghosts of its level, so down writes none
+        if constexpr (UP && !MB) {  // the ghost images; the up leg reads no ghosts of its level, so down writes none
             const int xl = ghost_image(X, g.n0, g.neu & kNeuW, g.neu & kNeuE);
             const int xr = ghost_image(X + 1, g.n0, g.neu & kNeuW, g.neu & kNeuE);
             const int yg = ghost_image(Y, g.n1, g.neu & kNeuS, g.neu & kNeuN);
@@ -928,7 +950,8 @@ __global__ __launch_bounds__(L3_NT) void k_leg3(const T *__restrict__ pin, T *__
                 if (xl >= 0) bstore<T>(rs_out, v.l, at(xl, yy, zz), 0);
                 if (xr >= 0) bstore<T>(rs_out, v.r, at(xr, yy, zz), 0);
             }
-        } else {  // the residual, its ghosts refreshed, without contraction as k_restrict
+        }
+        if constexpr (!UP) {  // the residual, its ghosts refreshed, without contraction as k_restrict
             auto residual = [&](bool red) {
                 const int q = red ? qr[u] : qb[u];
                 const Coef k = coef(u, red, red ? er[u] : eb[u]);
