@@ -91,6 +91,7 @@ struct Level {
     // the level's legs as one launch each (k_leg): tiles, and which legs
     struct Leg {
         Tile *t = nullptr;
+        int first = 0;      // of the legs' tiles, uploaded together
         int n = 0, ny = 0;  // workgroups (0: the leg runs as separate kernels), rows of one (0: boxes, k_leg3)
     } legs[2];              // down, up
     Region *r_full = nullptr;
@@ -1933,7 +1934,7 @@ std::vector<Tile> leg_tiles(const std::vector<BlockLevel> &hb, int ty, int slots
 
 // One leg's kernels may use the LDS they need, and its tiles on level V.
 template <typename T, bool VAR, bool UP, bool MB>
-int leg_level(mf3d_mg *mg, Level &V, int cus) {
+int leg_level(mf3d_mg *mg, Level &V, int cus, std::vector<Tile> &all) {
     Level::Leg &g = V.legs[UP];
     // the kernel's LDS; tiles, or the other leg's where they are the same
     auto take = [&](const void *kernel, int lds, int ny, std::vector<Tile> t) {
@@ -1945,22 +1946,21 @@ int leg_level(mf3d_mg *mg, Level &V, int cus) {
         g.n = (int)t.size();
         const Level::Leg &other = V.legs[!UP];
         if (other.n && other.ny == ny) {
-            g.t = other.t;
+            g.first = other.first;
             return 0;
         }
-        return upload(mg, &g.t, xcd_order(std::move(t)));
+        g.first = (int)all.size();
+        t = xcd_order(t);
+        all.insert(all.end(), t.begin(), t.end());
+        return 0;
     };
-    // The rows of a workgroup: a step takes 1.2 us with many rows and 0.95 with
-    // few, of which half belong to the ring.  Few on levels that leave compute
-    // units idle (64^3: 13.0 us against 14.7 a leg in FP32, 17.4 against 18.4 in
-    // FP64), many from where all are busy (128^3: 34 against 25).
     std::vector<Tile> box;
     for (int b = 0; b < (int)V.hb.size(); ++b)
         for (int z = 1; z <= V.hb[b].n2; z += L3_TILE)
             for (int y = 1; y <= V.hb[b].n1; y += L3_TILE)
                 for (int x = 1; x <= V.hb[b].n0; x += L3_TILE) box.push_back(Tile{b, x, y, z, z + L3_TILE - 1});
     // Boxes while they do not fill the card: two a compute unit, the FP64 up leg one
-    // (us a leg, march / boxes; down, up.  FP64 32^3 13.0 / 6.7, 13.4 / 9.3; 48^3
+    // (us a leg of a lone block, march / boxes; down, up.  FP64 32^3 13.0 / 6.7, 13.4 / 9.3; 48^3
     // 14.2 / 7.6, 13.8 / 10.0; 64^3 17.0 / 13.6, 16.4 / 17.6; FP32 32^3 9.1 / 5.6,
     // 10.8 / 7.3; 64^3 11.4 / 8.5, 12.2 / 10.7; 80^3 14.9 / 13.7, 16.6 / 17.6; 96^3
     // 15.2 / 22.3, 17.3 / 29.4).  FP64 with variable coefficients has no march:
@@ -1971,6 +1971,10 @@ int leg_level(mf3d_mg *mg, Level &V, int cus) {
         return take((const void *)k_leg3<T, UP, VAR, MB>, leg3_lds<T>(), 0, std::move(box));
     if constexpr (leg_march<T, VAR>()) {
         constexpr int SM = LEG_NY_SMALL, NY = leg_ny<T>(VAR);
+        // The rows of a marching workgroup: a step takes 1.2 us with many rows and 0.95
+        // with few, of which half belong to the ring.  Few on levels that leave
+        // compute units idle (64^3: 13.0 us against 14.7 a leg in FP32, 17.4 against
+        // 18.4 in FP64), many from where all are busy (128^3: 34 against 25).
         long long many, few;
         auto t = leg_tiles(V.hb, NY - 8, cus, &many);
         auto ts = leg_tiles(V.hb, SM - 8, cus, &few);
@@ -2027,6 +2031,7 @@ int leg_levels(mf3d_mg *mg, bool down) {
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, mg->cfg.device));
     cus = std::max(1, cus);
     const bool grid = mg->d_around != nullptr;
+    std::vector<Tile> all;
     for (int l = 0; l < std::min(mg->lt, mg->cfg.levels - 1); ++l) {
         Level &V = mg->lv[l];
         bool ok = V.own_ghosts || (grid && !VAR);
@@ -2039,15 +2044,20 @@ int leg_levels(mf3d_mg *mg, bool down) {
         if (!ok || (V.own_ghosts && yper == 3)) continue;  // the LDS layout is one for the launch
         int rc = 0;
         if (V.own_ghosts) {
-            rc = leg_level<T, VAR, true, false>(mg, V, cus);
+            rc = leg_level<T, VAR, true, false>(mg, V, cus, all);
             // the down leg writes no ghosts: it needs an up leg, which reads none
-            if (!rc && down && V.legs[1].n) rc = leg_level<T, VAR, false, false>(mg, V, cus);
+            if (!rc && down && V.legs[1].n) rc = leg_level<T, VAR, false, false>(mg, V, cus, all);
         } else if constexpr (!VAR) {
-            rc = leg_level<T, VAR, true, true>(mg, V, cus);
-            if (!rc && down) rc = leg_level<T, VAR, false, true>(mg, V, cus);
+            rc = leg_level<T, VAR, true, true>(mg, V, cus, all);
+            if (!rc && down) rc = leg_level<T, VAR, false, true>(mg, V, cus, all);
         }
         if (rc) return rc;
     }
+    if (all.empty()) return 0;
+    Tile *d = nullptr;
+    if (int rc = upload(mg, &d, all)) return rc;
+    for (Level &V : mg->lv)
+        for (Level::Leg &g : V.legs) g.t = d + g.first;
     return 0;
 }
 
