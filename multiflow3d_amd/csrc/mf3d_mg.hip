@@ -22,6 +22,7 @@
 #include <sched.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cmath>
 #include <cstdio>
@@ -150,9 +151,9 @@ struct mf3d_mg {
     hipGraphExec_t cyc[2] = {nullptr, nullptr};
     // coarse tail: levels lt..L-1 run in LDS, one workgroup per block
     int lt = 0;
-    BlockLevel *d_tail = nullptr;
-    TLv *d_tlv = nullptr;          // its levels (as d_tail) and their cell and ghost lists
-    unsigned *d_ttab = nullptr;
+    const BlockLevel *d_tail = nullptr;
+    const TLv *d_tlv = nullptr;    // its levels (as d_tail) and their cell and ghost lists
+    const unsigned *d_ttab = nullptr;
     size_t tail_lds = 0;
     // outer step tiles (finest level)
     Tile *t_out = nullptr;
@@ -287,6 +288,12 @@ int dev_alloc(mf3d_mg *mg, void **p, size_t bytes) {
     mg->allocs.push_back(*p);
     mg->bytes += (long long)bytes;
     return 0;
+}
+
+// Room for one more allocation: an allocation-free solve leaves out what it can
+// do without rather than refuse.
+bool room_for(const mf3d_mg *mg, size_t bytes) {
+    return !mg->arena || ((bytes + 255) & ~size_t(255)) <= mg->arena_cap - mg->arena_used;
 }
 
 template <typename X>
@@ -937,7 +944,7 @@ void tail(mf3d_mg *mg, bool from_zero, const int *done) {
         co.cz[l - lt] = (const T *)mg->lv[l].cz;
     }
     hipLaunchKernelGGL((k_tail<T, VAR>), dim3(mg->cfg.nblocks), dim3(TAIL_NT), mg->tail_lds, mg->stream, mg->d_tail,
-                       (const TLv *)mg->d_tlv, (const unsigned *)mg->d_ttab, mg->cfg.nblocks, L - lt, (const T *)V.rhs, from_zero ? nullptr : (const T *)V.phi[V.cur],
+                       mg->d_tlv, mg->d_ttab, mg->cfg.nblocks, L - lt, (const T *)V.rhs, from_zero ? nullptr : (const T *)V.phi[V.cur],
                        (T *)V.phi[1 - V.cur], co, mg->cfg.nu_pre, mg->cfg.nu_post,
                        mg->cdirect ? (const double *)mg->d_cinv : nullptr, mg->nc,
                        TailC64<T>{mg->c64 ? 1 : 0, mg->lv[L - 1].dcx, mg->lv[L - 1].dcy, mg->lv[L - 1].dcz}, done);
@@ -1532,18 +1539,32 @@ int choose_tail(mf3d_mg *mg) {
         mg->err = "hipFuncSetAttribute (tail LDS) failed";
         return MF3D_EDEVICE;
     }
+    return 0;
+}
+
+// What k_tail reads about its levels: their blocks, their LDS places (TLv) and
+// their cell and ghost lists, in one upload.  Blocks of equal extents and walls
+// share their lists: an allocation-free solve of two cycles on 64 unconnected
+// blocks of 8^3 cells, two levels, takes 0.48 ms, with lists for each block 0.68.
+// Where such a solve has no room left for them, the levels run as kernels of
+// their own, bitwise the same.
+int tail_upload(mf3d_mg *mg) {
+    const int L = mg->cfg.levels, nb = mg->cfg.nblocks;
+    if (mg->lt == L) return 0;
     std::vector<BlockLevel> tl;
     std::vector<TLv> lv;
     std::vector<unsigned> tab;
+    std::map<std::array<int, 4>, TLv> lists;
     std::vector<int> off(nb, 0);  // LDS entries: every level's potential, then every level's RHS
     for (int l = mg->lt; l < L; ++l)
         for (int b = 0; b < nb; ++b) {
             const BlockLevel &g = mg->lv[l].hb[b];
             tl.push_back(g);
-            TLv v = tlv_of(g.n0, g.n1, g.n2, g.neu);
+            const auto at = lists.try_emplace({g.n0, g.n1, g.n2, g.neu}, tlv_of(g.n0, g.n1, g.n2, g.neu));
+            if (at.second) tail_tables(at.first->second, tab);
+            TLv v = at.first->second;
             v.po = off[b];
             off[b] += v.sz * (v.n2 + 2);
-            tail_tables(v, tab);
             lv.push_back(v);
         }
     for (int l = mg->lt, q = 0; l < L; ++l)
@@ -1551,9 +1572,21 @@ int choose_tail(mf3d_mg *mg) {
             lv[q].ro = off[b];
             off[b] += lv[q].sz * (lv[q].n2 + 2);
         }
-    int rc;
-    if ((rc = upload(mg, &mg->d_tail, tl)) || (rc = upload(mg, &mg->d_tlv, lv))) return rc;
-    return upload(mg, &mg->d_ttab, tab);
+    const size_t o_lv = sizeof(BlockLevel) * tl.size(), o_tab = o_lv + sizeof(TLv) * lv.size();
+    std::vector<char> all(o_tab + sizeof(unsigned) * tab.size());
+    if (!room_for(mg, all.size())) {
+        mg->lt = L;
+        return 0;
+    }
+    std::memcpy(all.data(), tl.data(), o_lv);
+    std::memcpy(all.data() + o_lv, lv.data(), o_tab - o_lv);
+    std::memcpy(all.data() + o_tab, tab.data(), all.size() - o_tab);
+    char *d = nullptr;
+    if (int rc = upload(mg, &d, all)) return rc;
+    mg->d_tail = (const BlockLevel *)d;
+    mg->d_tlv = (const TLv *)(d + o_lv);
+    mg->d_ttab = (const unsigned *)(d + o_tab);
+    return 0;
 }
 
 template <typename T, bool VAR>
@@ -2252,7 +2285,7 @@ int build(mf3d_mg *mg) {
         mg->n_out = (int)tout.size();
         if ((rc = upload(mg, &mg->t_out, tout))) return rc;
     }
-    if ((rc = decide_coarse(mg)) || (rc = choose_tail(mg)) || (rc = leg_setup(mg))) return rc;
+    if ((rc = decide_coarse(mg)) || (rc = choose_tail(mg))) return rc;
     if (mg->cdirect && (rc = coarse_setup(mg))) return rc;
     if (mg->c64) {
         const long long ghc = mg->lv[L - 1].cells_gh;
@@ -2283,6 +2316,8 @@ int build(mf3d_mg *mg) {
         if ((rc = dev_alloc(mg, (void **)&mg->d_io, sizeof(double) * mg->io_len))) return rc;
         HIPCHK(hipHostMalloc((void **)&mg->h_io, sizeof(double) * mg->io_len, hipHostMallocDefault));
     }
+    // what a cycle can do without comes last
+    if ((rc = tail_upload(mg)) || (rc = leg_setup(mg))) return rc;
     // every field starts at zero (coeff zeroes phi, mgsolver.for:60-67)
     for (int l = 0; l < L; ++l) {
         Level &V = mg->lv[l];

@@ -1,0 +1,44 @@
+"""Problems near the end of the allocation-free solve's 32 MiB scratch: what is
+only there for speed (the LDS tail's lists) is left out where it has no room, so
+the numbers of blocks that the solver's fields leave room for are accepted, and
+the result is bitwise a handle's."""
+import numpy as np
+import pytest
+
+from multiflow3d_amd import topology as T
+from tests.test_zz_no_alloc import _handle, _noalloc
+
+pytestmark = pytest.mark.gpu
+
+H = [1.0 / 16, 1.0 / 20, 1.0 / 24]
+
+
+class _Blocks(list):
+    """Blocks that do not touch."""
+
+    def __init__(self, n, count):
+        super().__init__(T.Block(n=list(n), h=list(H)) for _ in range(count))
+        self.blocks = self
+
+
+def _same(grid, levels, **kw):
+    f = np.random.default_rng(83).standard_normal(sum(b.cells for b in grid.blocks))
+    print(f"[scratch] {len(grid.blocks)} blocks of {grid.blocks[0].n}, {levels} levels, {kw}", flush=True)
+    kw = dict(maxcy=2, eps=0.0, **kw)
+    _, p, hist, rmax, k = _noalloc(grid, levels, f, **kw)
+    _, ph, hh, rh, kh = _handle(grid, levels, f, **kw)
+    assert np.isfinite(p).all() and k == kh == 2 and rmax == rh
+    assert np.array_equal(hist, hh[:k + 1]) and np.array_equal(p, ph)
+
+
+@pytest.mark.parametrize("n,levels,count,precision", [
+    ((2, 2, 2), 1, 7013, "fp64"),
+    ((2, 2, 2), 1, 8354, "mixed"),
+    ((4, 4, 4), 2, 2157, "fp64"),
+    ((8, 8, 8), 2, 687, "mixed"),
+    ((16, 16, 16), 1, 116, "fp64"),
+    ((16, 16, 16), 3, 138, "mixed"),
+    ((16, 16, 16), 3, 20, "fp64"),   # room for everything
+])
+def test_unconnected_blocks_accepted(n, levels, count, precision):
+    _same(_Blocks(n, count), levels, precision=precision)
