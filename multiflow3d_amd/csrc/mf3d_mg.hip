@@ -2059,11 +2059,11 @@ std::vector<LegBlocks> leg_blocks(const std::vector<mf3d_block_desc> &blk) {
 }
 
 template <typename T, bool VAR>
-int leg_levels(mf3d_mg *mg, bool down) {
+int leg_levels(mf3d_mg *mg, bool down, const std::vector<LegBlocks> &around) {
     int cus = 0;
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, mg->cfg.device));
     cus = std::max(1, cus);
-    const bool grid = mg->d_around != nullptr;
+    const bool grid = !around.empty();
     std::vector<Tile> all;
     for (int l = 0; l < std::min(mg->lt, mg->cfg.levels - 1); ++l) {
         Level &V = mg->lv[l];
@@ -2087,30 +2087,33 @@ int leg_levels(mf3d_mg *mg, bool down) {
         if (rc) return rc;
     }
     if (all.empty()) return 0;
+    if (!room_for(mg, sizeof(Tile) * all.size() + 256 + sizeof(LegBlocks) * around.size())) {
+        for (Level &V : mg->lv) V.legs[0] = V.legs[1] = Level::Leg{};
+        return 0;
+    }
     Tile *d = nullptr;
     if (int rc = upload(mg, &d, all)) return rc;
     for (Level &V : mg->lv)
         for (Level::Leg &g : V.legs) g.t = d + g.first;
-    return 0;
+    return grid ? upload(mg, &mg->d_around, around) : 0;
 }
 
 // Which levels run their legs as one launch each: red-black sweeps, two a leg,
 // of lone blocks (FP64 with variable coefficients on small levels only)
 // or of block grids that leg_blocks admits, all of one spacing (constant
 // coefficients), every extent even and at least 8 (the ring of a tile then
-// crosses one face at most a side), above the LDS tail and the coarsest level.
+// crosses one face at most a side), above the LDS tail and the coarsest level;
+// none where an allocation-free solve has no room for their tables.
 int leg_setup(mf3d_mg *mg) {
     const mf3d_mg_cfg &c = mg->cfg;
     const bool mixed = c.precision == MF3D_MIXED, var = c.variable_coef != 0;
     const bool any_up = c.nu_post == 2, any_down = any_up && c.nu_pre == 2;  // the down leg writes no ghosts: the up leg needs none
     if (!mg->legs || c.smoother != 3 || mg->refined || !any_up) return 0;
-    if (!var && !mg->lv[0].own_ghosts) {
-        const auto around = leg_blocks(mg->blk);
-        if (!around.empty())
-            if (int rc = upload(mg, &mg->d_around, around)) return rc;
-    }
-    return mixed ? (var ? leg_levels<float, true>(mg, any_down) : leg_levels<float, false>(mg, any_down))
-                 : (var ? leg_levels<double, true>(mg, any_down) : leg_levels<double, false>(mg, any_down));
+    std::vector<LegBlocks> around;
+    if (!var && !mg->lv[0].own_ghosts) around = leg_blocks(mg->blk);
+    if (mixed)
+        return var ? leg_levels<float, true>(mg, any_down, around) : leg_levels<float, false>(mg, any_down, around);
+    return var ? leg_levels<double, true>(mg, any_down, around) : leg_levels<double, false>(mg, any_down, around);
 }
 
 int build(mf3d_mg *mg) {

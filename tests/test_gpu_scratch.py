@@ -1,5 +1,5 @@
 """Problems near the end of the allocation-free solve's 32 MiB scratch: what is
-only there for speed (the LDS tail's lists) is left out where it has no room, so
+only there for speed (the LDS tail's lists, the legs' tables) is left out where it has no room, so
 the numbers of blocks that the solver's fields leave room for are accepted, and
 the result is bitwise a handle's."""
 import numpy as np
@@ -42,3 +42,13 @@ def _same(grid, levels, **kw):
 ])
 def test_unconnected_blocks_accepted(n, levels, count, precision):
     _same(_Blocks(n, count), levels, precision=precision)
+
+
+@pytest.mark.parametrize("make,levels,kw", [
+    (lambda: T.single_block([8, 8, 6132], H, T.CHANNEL_BC), 2, dict(precision="fp64")),
+    (lambda: T.single_block([8, 8, 7478], H, T.CHANNEL_BC), 2, dict(precision="mixed")),
+    (lambda: T.block_grid([8] * 93, [8] * 2, [8] * 2, T.CHANNEL_BC, H), 2, dict(precision="fp64", krylov=True)),
+    (lambda: T.block_grid([2] * 1252, [2] * 2, [2] * 2, T.CHANNEL_BC, H), 1, dict(precision="fp64", krylov=True)),
+], ids=["rod_fp64", "rod_mixed", "grid_gcr", "one_level_gcr"])
+def test_legs_without_room(make, levels, kw):
+    _same(make(), levels, **kw)
