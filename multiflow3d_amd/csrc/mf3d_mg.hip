@@ -599,6 +599,8 @@ std::vector<Tile> xcd_order(const std::vector<Tile> &t) {
 
 inline int inner_bytes(const mf3d_mg_cfg &c) { return c.precision == MF3D_MIXED ? 4 : 8; }
 
+constexpr size_t kAdiTable = 3 * 2 * ADC_CLS * ADC_LINE;  // a block's classes: axes, apr and a, classes, places
+
 long long estimate(const mf3d_mg_cfg &c, const mf3d_block_desc *b) {
     const std::vector<int> own = own_levels(c.nblocks, b, c.levels);
     long long tot = 0;
@@ -1848,9 +1850,10 @@ int coarse_factor(mf3d_mg *mg) {
 // largest block's ghosted potential and the tables fit in kAdiLdsMax bytes;
 // else the whole-sweep LDS kernel where the level's largest block (its ghosted potential and the per-diagonal
 // scratch, with the RHS if that fits too) fits in kAdiLdsMax bytes.
+// classes: whether the class-table kernel may be taken.
 constexpr size_t kAdiLdsMax = 150 * 1024;
 
-int adi_setup(mf3d_mg *mg) {
+int adi_setup(mf3d_mg *mg, bool classes) {
     const size_t w = inner_bytes(mg->cfg);
     const char *env = std::getenv("MF3D_ADI_LDS");
     const bool allow = !(env && env[0] == '0');
@@ -1874,7 +1877,7 @@ int adi_setup(mf3d_mg *mg) {
         const size_t cls_lds = (cells + 2 * (size_t)tt + 2 * ADC_CLS * ADC_LINE) * w;
         const bool fits = allow && diag <= 1024;  // the next diagonal's prefetch: 4 entries per thread
         V.adi_k = 0;
-        if (allow && !mg->cfg.variable_coef && line <= ADC_LINE && cls_lds <= kAdiLdsMax) {
+        if (classes && allow && !mg->cfg.variable_coef && line <= ADC_LINE && cls_lds <= kAdiLdsMax) {
             V.adi_k = plane <= ADC_NT ? 1 : (plane <= 2 * ADC_NT ? 2 : 5);  // ADC_LINE^2 <= 5 * ADC_NT
             V.adi_lds = cls_lds;
             V.adi_sstride = tt;
@@ -1903,6 +1906,42 @@ int adi_setup(mf3d_mg *mg) {
             }
     }
     return 0;
+}
+
+// Whether an allocation-free solve has room for the tables that adi_setup chose.
+bool adi_fits(const mf3d_mg *mg) {
+    const size_t w = inner_bytes(mg->cfg);
+    size_t need = 0;
+    bool global = false;
+    auto add = [&](size_t bytes) { need += (bytes + 255) & ~size_t(255); };
+    for (const Level &V : mg->lv) {
+        global = global || !V.adi_lds;
+        if (V.adi_k) {
+            add(V.hb.size() * kAdiTable * w);
+        } else if (V.adi_lds) {
+            for (int a = 0; a < 6; ++a) add(V.cells_gh * w);
+        }
+    }
+    if (global) add(mg->lv[0].cells_gh * w);
+    return room_for(mg, need);
+}
+
+int adi_alloc(mf3d_mg *mg) {
+    const size_t w = inner_bytes(mg->cfg);
+    int rc;
+    bool global = false;  // a level runs the per-pass kernels: their a(m) scratch
+    for (Level &V : mg->lv) {
+        global = global || !V.adi_lds;
+        if (V.adi_k) {
+            if ((rc = dev_alloc(mg, &V.adi_tab, V.hb.size() * kAdiTable * w))) return rc;
+        } else if (V.adi_lds) {
+            for (int a = 0; a < 3; ++a)
+                if ((rc = dev_alloc(mg, &V.adi_apr[a], V.cells_gh * w)) ||
+                    (rc = dev_alloc(mg, &V.adi_a[a], V.cells_gh * w)))
+                    return rc;
+        }
+    }
+    return global ? dev_alloc(mg, &mg->d_adi, mg->lv[0].cells_gh * w) : 0;
 }
 
 // The ADI Thomas coefficients of the levels whose sweeps run in LDS, from
@@ -2344,19 +2383,8 @@ int build(mf3d_mg *mg) {
     // constant coefficients are final now; variable ones at each coeff
     if (!c.variable_coef && (rc = coarse_factor<false>(mg))) return rc;
     if (c.smoother == 2) {
-        if ((rc = adi_setup(mg))) return rc;
-        bool global = false;  // a level runs the per-pass kernels: their a(m) scratch
-        for (Level &V : mg->lv) {
-            global = global || !V.adi_lds;
-            if (V.adi_k) {
-                if ((rc = dev_alloc(mg, &V.adi_tab, (size_t)nb * 6 * ADC_CLS * ADC_LINE * w))) return rc;
-            } else if (V.adi_lds)
-                for (int a = 0; a < 3; ++a)
-                    if ((rc = dev_alloc(mg, &V.adi_apr[a], V.cells_gh * w)) ||
-                        (rc = dev_alloc(mg, &V.adi_a[a], V.cells_gh * w)))
-                        return rc;
-        }
-        if (global && (rc = dev_alloc(mg, &mg->d_adi, L0.cells_gh * w))) return rc;
+        if ((rc = adi_setup(mg, true)) || (!adi_fits(mg) && (rc = adi_setup(mg, false))) || (rc = adi_alloc(mg)))
+            return rc;
         // constant coefficients are final now; variable ones at each coeff
         if (!c.variable_coef && (rc = mixed ? adi_coef_build<float, false>(mg) : adi_coef_build<double, false>(mg)))
             return rc;

@@ -1,6 +1,7 @@
 """Problems near the end of the allocation-free solve's 32 MiB scratch: what is
-only there for speed (the LDS tail's lists, the legs' tables) is left out where it has no room, so
-the numbers of blocks that the solver's fields leave room for are accepted, and
+only there for speed (the LDS tail's lists, the legs' tables, the
+line smoother's class tables) is left out where it has no room, so the
+numbers of blocks that the solver's fields leave room for are accepted, and
 the result is bitwise a handle's."""
 import numpy as np
 import pytest
@@ -52,3 +53,14 @@ def test_unconnected_blocks_accepted(n, levels, count, precision):
 ], ids=["rod_fp64", "rod_mixed", "grid_gcr", "one_level_gcr"])
 def test_legs_without_room(make, levels, kw):
     _same(make(), levels, **kw)
+
+
+@pytest.mark.parametrize("n,levels,count,precision", [
+    ((2, 2, 2), 1, 6195, "mixed"),
+    ((4, 4, 4), 2, 1168, "fp64"),
+    ((8, 8, 8), 3, 261, "fp64"),
+    ((5, 5, 6), 1, 1295, "mixed"),
+])
+def test_line_smoother_blocks_accepted(n, levels, count, precision):
+    _same(T.block_grid([n[0]] * count, [n[1]], [n[2]], [5, 5, 4, 4, 4, 3], H), levels, precision=precision, smoother=2,
+          nu_post=1)
