@@ -601,7 +601,9 @@ inline int inner_bytes(const mf3d_mg_cfg &c) { return c.precision == MF3D_MIXED 
 
 constexpr size_t kAdiTable = 3 * 2 * ADC_CLS * ADC_LINE;  // a block's classes: axes, apr and a, classes, places
 
-long long estimate(const mf3d_mg_cfg &c, const mf3d_block_desc *b) {
+// The bytes of a handle; classes: with the line smoother's class tables, which
+// an allocation-free solve takes only where it has room for them.
+long long estimate(const mf3d_mg_cfg &c, const mf3d_block_desc *b, bool classes) {
     const std::vector<int> own = own_levels(c.nblocks, b, c.levels);
     long long tot = 0;
     const long long w = inner_bytes(c);
@@ -611,7 +613,10 @@ long long estimate(const mf3d_mg_cfg &c, const mf3d_block_desc *b) {
             gh += (long long)(dim_at(b[i], 0, l, own[i]) + 2) * (dim_at(b[i], 1, l, own[i]) + 2) * (dim_at(b[i], 2, l, own[i]) + 2);
         tot += gh * w * 3;                                     // phi (two) and rhs
         if (c.variable_coef) tot += gh * (w * 3 + 8 * 4);      // coefficients, FP64 copies, density
-        if (c.smoother == 2) tot += gh * w * 6;                // ADI Thomas coefficients (LDS levels)
+        if (c.smoother == 2) {  // ADI Thomas coefficients (LDS levels)
+            const long long tables = classes && !c.variable_coef ? c.nblocks * (long long)kAdiTable : 0;
+            tot += w * std::max(gh * 6, tables);
+        }
     }
     long long gh0 = 0, in0 = 0;
     for (int i = 0; i < c.nblocks; ++i) {
@@ -3008,7 +3013,7 @@ int mf3d_mg_abi_version(void) { return MF3D_MG_ABI_VERSION; }
 int64_t mf3d_mg_estimate_bytes(const mf3d_mg_cfg *cfg, const mf3d_block_desc *blocks) {
     if (!cfg || !blocks) return MF3D_EINVAL;
     if (!validate(*cfg, blocks).empty()) return MF3D_EINVAL;
-    return estimate(*cfg, blocks);
+    return estimate(*cfg, blocks, true);
 }
 
 int mf3d_mg_create(const mf3d_mg_cfg *cfg, const mf3d_block_desc *blocks, mf3d_mg **out) {
@@ -3246,7 +3251,7 @@ int mf3d_mg_solve_device_noalloc(const mf3d_mg_cfg *cfg, const mf3d_block_desc *
         gh0 += (long long)(blocks[i].n[0] + 2) * (blocks[i].n[1] + 2) * (blocks[i].n[2] + 2);
         in0 += (long long)blocks[i].n[0] * blocks[i].n[1] * blocks[i].n[2];
     }
-    const long long need = estimate(*cfg, blocks) - std::max(gh0, in0) * 8 + (1LL << 20);
+    const long long need = estimate(*cfg, blocks, false) - std::max(gh0, in0) * 8 + (1LL << 20);
     if (need > (long long)MF3D_NOALLOC_SCRATCH_BYTES) {
         tmp.err = "the solve needs about " + std::to_string(need >> 20) + " MiB of device memory, more than the " +
                   std::to_string((long long)MF3D_NOALLOC_SCRATCH_BYTES >> 20) +
