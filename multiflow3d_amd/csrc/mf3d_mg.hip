@@ -23,7 +23,6 @@
 
 #include <algorithm>
 #include <array>
-#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -31,9 +30,8 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -41,6 +39,7 @@
 #include "mg_coarse.hpp"
 #include "mg_common.hpp"
 #include "mg_ghostmap.hpp"
+#include "mg_hostpack.hpp"
 #include "mg_leg.hpp"
 #include "mg_refine.hpp"
 #include "mg_outer.hpp"
@@ -1387,97 +1386,86 @@ void copy_piece(const mf3d_mg *mg, const HostPiece &q, double *caller, double *p
 // MiB, two threads gain nothing: 1.10 against 1.13 ms); hosts that refuse
 // threads or memory take one buffer and the calling thread.
 int host_fields(mf3d_mg *mg, bool in, double *const *const *caller, double *const *dev, int nf, int ring) {
-    std::vector<HostPiece> pieces;
-    long long o = 0;
-    for (int b = 0; b < mg->cfg.nblocks; ++b) {
-        const mf3d_block_desc &B = mg->blk[b];
-        const long long plane = (long long)(B.n[0] + 2 * ring) * (B.n[1] + 2 * ring);
-        const int n2 = B.n[2] + 2 * ring, step = (int)std::max(1LL, 32768 / plane);
-        for (int k = 0; k < n2; k += step) {
-            pieces.push_back(HostPiece{b, k, std::min(n2, k + step), o});
-            o += plane * (pieces.back().k1 - k);
-        }
-    }
-    const size_t bytes = sizeof(double) * (size_t)o;
-    const int np = (int)pieces.size();
+    const int nb = mg->cfg.nblocks;
+    auto plane_of = [&](int b) { return (long long)(mg->blk[b].n[0] + 2 * ring) * (mg->blk[b].n[1] + 2 * ring); };
+    long long len = 0;
+    for (int b = 0; b < nb; ++b) len += plane_of(b) * (mg->blk[b].n[2] + 2 * ring);
+    const size_t bytes = sizeof(double) * (size_t)len;
     cpu_set_t set;
     const int cpus = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
     int nt = (int)std::min<size_t>({8, (size_t)std::max(0, cpus - 1), bytes * nf >> 22});
     if (nt < 3) nt = 0;
-    if (nt >= 2 && !mg->h_io2) {
+    std::vector<HostPiece> pieces;
+    try {
+        long long o = 0;
+        for (int b = 0; nt && b < nb; ++b) {
+            const long long plane = plane_of(b);
+            const int n2 = mg->blk[b].n[2] + 2 * ring, step = (int)std::max(1LL, 32768 / plane);
+            for (int k = 0; k < n2; k += step) {
+                pieces.push_back(HostPiece{b, k, std::min(n2, k + step), o});
+                o += plane * (pieces.back().k1 - k);
+            }
+        }
+    } catch (const std::bad_alloc &) {
+        nt = 0;
+    }
+    if (nt && !mg->h_io2) {
         if (hipHostMalloc((void **)&mg->h_io2, sizeof(double) * mg->io_len, hipHostMallocDefault) != hipSuccess) {
             mg->h_io2 = nullptr;
             (void)hipGetLastError();
         }
     }
     for (hipEvent_t &e : mg->io_ev)
-        if (nt >= 2 && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        if (nt && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
             e = nullptr;
             (void)hipGetLastError();
         }
     if (!mg->h_io2 || !mg->io_ev[0] || !mg->io_ev[1]) nt = 0;
     double *buf[2] = {mg->h_io, mg->h_io2};
-    std::atomic<int> next{0}, open{in ? 2 : 0};  // fields whose buffer the threads may use
-    std::atomic<bool> stop{false};
-    std::vector<std::atomic<int>> packed(nf);
-    for (auto &a : packed) a = 0;
-    auto work = [&] {
-        for (;;) {
-            const int c = next.fetch_add(1);
-            if (c >= nf * np) return;
-            const int f = c / np;
-            while (open.load(std::memory_order_acquire) <= f) {
-                if (stop.load()) return;
-                std::this_thread::yield();
-            }
-            const HostPiece &q = pieces[c % np];
-            copy_piece(mg, q, caller[f][q.b], buf[f & 1], ring, in);
-            packed[f].fetch_add(1, std::memory_order_release);
-        }
-    };
-    std::vector<std::thread> threads;
-    try {
-        threads.reserve(nt);
-        for (int t = 0; t < nt; ++t) threads.emplace_back(work);
-    } catch (const std::system_error &) {  // what runs already does the work
-    }
-    if (threads.empty()) {
-        for (int f = 0; f < nf; ++f) {
-            auto copy = [&] { for (const HostPiece &q : pieces) copy_piece(mg, q, caller[f][q.b], mg->h_io, ring, in); };
-            if (in) copy();
-            HIPCHK(in ? hipMemcpyAsync(dev[f], mg->h_io, bytes, hipMemcpyHostToDevice, mg->stream)
-                      : hipMemcpyAsync(mg->h_io, dev[f], bytes, hipMemcpyDeviceToHost, mg->stream));
-            HIPCHK(hipStreamSynchronize(mg->stream));
-            if (!in) copy();
-        }
-        return 0;
-    }
-    auto travel = [&](int f) {
-        hipError_t e = in ? hipMemcpyAsync(dev[f], buf[f & 1], bytes, hipMemcpyHostToDevice, mg->stream)
-                          : hipMemcpyAsync(buf[f & 1], dev[f], bytes, hipMemcpyDeviceToHost, mg->stream);
-        return e == hipSuccess ? hipEventRecord(mg->io_ev[f & 1], mg->stream) : e;
-    };
-    auto wait_packed = [&](int f) {
-        while (packed[f].load(std::memory_order_acquire) < np) std::this_thread::yield();
-    };
+    auto copy = [&](int f, int q) { copy_piece(mg, pieces[q], caller[f][pieces[q].b], buf[f & 1], ring, in); };
     hipError_t e = hipSuccess;
-    for (int f = 0; !in && f < 2 && f < nf && e == hipSuccess; ++f) e = travel(f);
-    for (int f = 0; f < nf && e == hipSuccess; ++f) {
-        if (in) {
-            wait_packed(f);
-            e = travel(f);
-            if (f + 2 >= nf) continue;
+    {
+        PackTeam team(nf, (int)pieces.size(), copy);
+        if (!team.start(nt)) {
+            for (int f = 0; f < nf; ++f) {
+                auto whole = [&] {
+                    long long o = 0;
+                    for (int b = 0; b < nb; ++b) {
+                        const int n2 = mg->blk[b].n[2] + 2 * ring;
+                        copy_piece(mg, HostPiece{b, 0, n2, o}, caller[f][b], mg->h_io, ring, in);
+                        o += plane_of(b) * n2;
+                    }
+                };
+                if (in) whole();
+                HIPCHK(in ? hipMemcpyAsync(dev[f], mg->h_io, bytes, hipMemcpyHostToDevice, mg->stream)
+                          : hipMemcpyAsync(mg->h_io, dev[f], bytes, hipMemcpyDeviceToHost, mg->stream));
+                HIPCHK(hipStreamSynchronize(mg->stream));
+                if (!in) whole();
+            }
+            return 0;
         }
-        if (e == hipSuccess) e = hipEventSynchronize(mg->io_ev[f & 1]);  // field f has travelled
-        if (e != hipSuccess) break;
-        open.store(in ? f + 3 : f + 1, std::memory_order_release);
-        if (!in) {
-            wait_packed(f);
-            if (f + 2 < nf) e = travel(f + 2);
+        auto travel = [&](int f) {
+            hipError_t r = in ? hipMemcpyAsync(dev[f], buf[f & 1], bytes, hipMemcpyHostToDevice, mg->stream)
+                              : hipMemcpyAsync(buf[f & 1], dev[f], bytes, hipMemcpyDeviceToHost, mg->stream);
+            return r == hipSuccess ? hipEventRecord(mg->io_ev[f & 1], mg->stream) : r;
+        };
+        if (in) team.open(2);
+        for (int f = 0; !in && f < 2 && f < nf && e == hipSuccess; ++f) e = travel(f);
+        for (int f = 0; f < nf && e == hipSuccess; ++f) {
+            if (in) {
+                team.wait(f);
+                e = travel(f);
+                if (f + 2 >= nf) continue;
+            }
+            if (e == hipSuccess) e = hipEventSynchronize(mg->io_ev[f & 1]);  // field f has travelled
+            if (e != hipSuccess) break;
+            team.open(in ? f + 3 : f + 1);
+            if (!in) {
+                team.wait(f);
+                if (f + 2 < nf) e = travel(f + 2);
+            }
         }
     }
-    stop = true;
-    for (std::thread &t : threads) t.join();
     const hipError_t last = hipStreamSynchronize(mg->stream);  // the buffers are free again
     HIPCHK(e);
     HIPCHK(last);
