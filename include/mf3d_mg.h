@@ -207,7 +207,8 @@ int mf3d_mg_solve_device(mf3d_mg *mg, const double *f_dev, double *p_dev, void *
  * allocating routine, and it needs no handle.  f_dev, p_dev, rmax_out,
  * iters_out and hist are as in mf3d_mg_solve_device (results are bitwise
  * those of a handle created with the same cfg and blocks, with the default
- * sweep tiling, MF3D_AUTOTUNE=0).  Constant coefficients only
+ * sweep tiling, MF3D_AUTOTUNE=0); tables that only make a cycle faster are
+ * left out where the array has no room for them.  Constant coefficients only
  * (variable_coef = 0, else MF3D_ENOTSUP).  A problem whose hierarchy does
  * not fit the array returns MF3D_ENOMEM before any device work.  The array
  * is shared by every call on a GPU and keeps the last call's contents

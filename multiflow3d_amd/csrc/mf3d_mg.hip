@@ -2028,9 +2028,16 @@ int leg_level(mf3d_mg *mg, Level &V, int cus, std::vector<Tile> &all) {
     // (us a leg of a lone block, march / boxes; down, up.  FP64 32^3 13.0 / 6.7, 13.4 / 9.3; 48^3
     // 14.2 / 7.6, 13.8 / 10.0; 64^3 17.0 / 13.6, 16.4 / 17.6; FP32 32^3 9.1 / 5.6,
     // 10.8 / 7.3; 64^3 11.4 / 8.5, 12.2 / 10.7; 80^3 14.9 / 13.7, 16.6 / 17.6; 96^3
-    // 15.2 / 22.3, 17.3 / 29.4).  FP64 with variable coefficients has no march:
+    // 15.2 / 22.3, 17.3 / 29.4.  FP32 with variable coefficients, boxes against march,
+    // a leg pair: 48^3 -10.6, 64^3 -3.3, 72^3 +3.1, 80^3 +11.4, 96^3 +40).  FP64 with variable
+    // coefficients has no march:
     // boxes against separate kernels, a leg pair, 48^3 22 / 44, 64^3 36 / 39,
     // 80^3 70 / 87, 96^3 124 / 129: four a compute unit.
+    // Block grids by the same count.  Their boxes against march, a leg pair, FP64 / FP32: 8 x 8 x 8
+    // blocks of 8^3 -42 / -18, 5 x 5 x 5 of 16^3 +10 / -6, 3 x 3 x 3 of 32^3 +54 / +13,
+    // 80 of 40 x 10 x 24 +84 / +28; but 16 x 10 x 10 of 8^3, marched, -125 / -58: blocks of 8 cells
+    // along x leave most of a marching tile idle, though it still takes less
+    // than separate kernels (by 47 / 109).
     const int per_cu = sizeof(T) == 8 ? (VAR ? 4 : (UP ? 1 : 2)) : 2;
     if ((int)box.size() <= per_cu * cus)
         return take((const void *)k_leg3<T, UP, VAR, MB>, leg3_lds<T>(), 0, std::move(box));

@@ -42,7 +42,7 @@
 //
 // Measured on the level of 256^3 cells, sweeps and transfers apart against the
 // leg: FP32 down 125 us (47 + 50 + 28) against 69, up 127 (27 + 2 x 50) against 82;
-// FP64 down 264 against 140, up 310 against 180.  HBM traffic is 1.12 to 1.30
+// FP64 down 264 against 140, up 310 against 180.  HBM traffic is 1.12 to 1.32
 // times what a leg has to move and takes half the time; the bound is a step's
 // serial chain, 2700 clocks in FP32 for about 120 vector and 80 scalar
 // instructions a wavefront between two barriers, the four updates
