@@ -1064,7 +1064,10 @@ void vcycle_dev(mf3d_mg *mg, bool zero_start, const int *done) {
         for (int l = ldown - 1; l >= 0; --l) {
             if (l == L - 1) continue;
             int post = mg->cfg.nu_post;
-            if (legs && mg->lv[l].legs[1].n) {
+            // the up leg takes a ghost's value from the cell it stands for: not where a
+            // caller's potential came this far without a sweep's exchange
+            const bool ghosts = l > 0 || zero_start || mg->cfg.nu_pre > 0;
+            if (legs && ghosts && mg->lv[l].legs[1].n) {
                 leg<T, VAR, true>(mg, l, done);
                 post = 0;
             } else if (fused_prolong(mg, l)) {
