@@ -2324,7 +2324,9 @@ int build(mf3d_mg *mg) {
         // From 2^22 cells the coefficients come from the density: below, the face
         // arrays fit in the caches and the divisions cost more than their bytes
         // (us for the three passes of a GCR step, arrays / density: 96^3 43 / 52,
-        // 160^3 164 / 159, 192^3 261 / 237, 256^3 580 / 496, 384^3 2127 / 1599).
+        // 160^3 164 / 159, 192^3 261 / 237, 256^3 580 / 496, 384^3 2127 / 1599; mixed.
+        // A cycle with defect correction or GCR in FP64: 160^3 5 and 9 us longer by it,
+        // 192^3 the same and 3 shorter, 256^3 19 and 50 shorter).
         mg->dens_outer = c.variable_coef && (dens == 2 ? L0.cells_gh > (1LL << 22) : dens == 1);
         auto tout = xcd_order(sweep_tiles(L0.hb, 8));
         mg->n_out = (int)tout.size();
